@@ -309,15 +309,35 @@ __global__ __launch_bounds__(256) void k_direct_rt(Geom g, PlaneMap m, DirectCfg
     // 16-byte stores where every row starts 16-byte aligned (then a column
     // group is either wholly inside the row or wholly past it).
     const bool vec = (g.OW & 3) == 0 && (reinterpret_cast<uintptr_t>(O) & 15) == 0;
+    if (e.n) {
+        // One row of four at a time in a runtime loop (the accumulators keep
+        // compile-time indexes): all 4 RPT at once took 120 registers.
+#pragma unroll 1
+        for (int r = 0; r < RPT; r++) {
+            float v[4];
+            int pl[4], pt[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                v[q] = acc[0][q];
+#pragma unroll
+                for (int a = 1; a < RPT; a++) v[q] = r == a ? acc[a][q] : v[q];
+                pl[q] = o;
+                pt[q] = min(orow0 + RPT * rg + r, g.OH - 1) * g.OW + min(col + q, g.OW - 1);
+            }
+            epi_eval_n<4>(e, v, pl, pt);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int a = 0; a < RPT; a++) acc[a][q] = r == a ? v[q] : acc[a][q];
+        }
+    }
     if (vec) {
 #pragma unroll
         for (int a = 0; a < RPT; a++) {
             const int row = orow0 + RPT * rg + a;
-            const int pt = row * g.OW + col;
             if (row < g.OH && col < g.OW)
                 *reinterpret_cast<float4*>(out + (size_t)row * g.OW + col) =
-                    make_float4(epi(e, acc[a][0], o, pt), epi(e, acc[a][1], o, pt + 1), epi(e, acc[a][2], o, pt + 2),
-                                epi(e, acc[a][3], o, pt + 3));
+                    make_float4(acc[a][0], acc[a][1], acc[a][2], acc[a][3]);
         }
     } else {
 #pragma unroll
@@ -326,7 +346,7 @@ __global__ __launch_bounds__(256) void k_direct_rt(Geom g, PlaneMap m, DirectCfg
             if (row >= g.OH) continue;
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                if (col + q < g.OW) out[(size_t)row * g.OW + col + q] = epi(e, acc[a][q], o, row * g.OW + col + q);
+                if (col + q < g.OW) out[(size_t)row * g.OW + col + q] = acc[a][q];
         }
     }
 }

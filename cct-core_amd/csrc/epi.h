@@ -71,22 +71,92 @@ __device__ __forceinline__ float epi(const Epi& e, float v, int plane, int point
     return e.n == 0 ? v : epi_eval(e, v, plane, point);
 }
 
-// Re-applies the epilogue to elements this thread has just stored (kernels
-// whose accumulator arrays must stay in registers store them plainly first).
-// The fence orders the thread's earlier stores before these loads.
-__device__ __forceinline__ void epi_rewrite4(const Epi& e, float* p, int plane, int point) {
-    __threadfence();
-    float4 v = *reinterpret_cast<const float4*>(p);
-    v.x = epi_eval(e, v.x, plane, point);
-    v.y = epi_eval(e, v.y, plane, point + 1);
-    v.z = epi_eval(e, v.z, plane, point + 2);
-    v.w = epi_eval(e, v.w, plane, point + 3);
-    *reinterpret_cast<float4*>(p) = v;
+// The epilogue over N output elements of a thread, op by op: the descriptor's
+// fields (scalar loads of a runtime op index) are fetched once per op instead of
+// once per op and element, and the N operand loads of a field op are in flight
+// together.  Element by element these dependent loads were most of a small
+// launch: bias and rectifier on 16 images 64x64x16 -> 32 planes, 3x3, took
+// 22.7 us, and 13.8 us this way (12.4 us without an epilogue).  Every (plane, point) must be a valid output element, also where
+// the caller does not store the result.
+template <int N>
+__device__ __forceinline__ void epi_eval_n(const Epi& e, float (&v)[N], const int (&plane)[N], const int (&point)[N]) {
+#pragma clang fp contract(off)
+    for (int i = 0; i < e.n; i++) {
+        const int op = e.op[i];
+        float a[N];
+        if (op >= COGCONV_EPI_ADD_FIELD) {
+            const int slot = e.slot[i];
+            const float* src = e.src[slot];
+            const size_t points = (size_t)e.srcPoints[slot];
+            const bool perPlane = e.srcPlanes[slot] != 1, perPoint = e.srcPoints[slot] != 1;
+#pragma unroll
+            for (int k = 0; k < N; k++) a[k] = src[(perPlane ? plane[k] : 0) * points + (perPoint ? point[k] : 0)];
+        } else {
+            const float c = e.val[i];
+#pragma unroll
+            for (int k = 0; k < N; k++) a[k] = c;
+        }
+#define COGCONV_EPI_EACH(expr)        \
+    {                                 \
+        _Pragma("unroll")             \
+        for (int k = 0; k < N; k++) { \
+            const float x = v[k];     \
+            const float y = a[k];     \
+            (void)y;                  \
+            v[k] = (expr);            \
+        }                             \
+        break;                        \
+    }
+        switch (op) {
+        case COGCONV_EPI_ADD_CONST:
+        case COGCONV_EPI_ADD_FIELD: COGCONV_EPI_EACH(x + y)
+        case COGCONV_EPI_SUB_CONST:
+        case COGCONV_EPI_SUB_FIELD: COGCONV_EPI_EACH(x - y)
+        case COGCONV_EPI_RSUB_CONST:
+        case COGCONV_EPI_RSUB_FIELD: COGCONV_EPI_EACH(y - x)
+        case COGCONV_EPI_MUL_CONST:
+        case COGCONV_EPI_MUL_FIELD: COGCONV_EPI_EACH(x * y)
+        case COGCONV_EPI_DIV_CONST:
+        case COGCONV_EPI_DIV_FIELD: COGCONV_EPI_EACH(x / y)
+        case COGCONV_EPI_RDIV_CONST:
+        case COGCONV_EPI_RDIV_FIELD: COGCONV_EPI_EACH(y / x)
+        case COGCONV_EPI_MAX_CONST:
+        case COGCONV_EPI_MAX_FIELD: COGCONV_EPI_EACH(fmaxf(x, y))
+        case COGCONV_EPI_MIN_CONST:
+        case COGCONV_EPI_MIN_FIELD: COGCONV_EPI_EACH(fminf(x, y))
+        case COGCONV_EPI_NEG: COGCONV_EPI_EACH(-x)
+        case COGCONV_EPI_ABS: COGCONV_EPI_EACH(fabsf(x))
+        case COGCONV_EPI_SQ: COGCONV_EPI_EACH(x * x)
+        case COGCONV_EPI_SQRT: COGCONV_EPI_EACH(sqrtf(x))
+        case COGCONV_EPI_EXP: COGCONV_EPI_EACH(expf(x))
+        case COGCONV_EPI_LOG: COGCONV_EPI_EACH(logf(x))
+        case COGCONV_EPI_TANH: COGCONV_EPI_EACH(tanhf(x))
+        case COGCONV_EPI_SIGNUM: COGCONV_EPI_EACH(x > 0.f ? 1.f : (x < 0.f ? -1.f : 0.f))
+        default: break;
+        }
+#undef COGCONV_EPI_EACH
+    }
 }
 
-__device__ __forceinline__ void epi_rewrite1(const Epi& e, float* p, int plane, int point) {
-    __threadfence();
-    *p = epi_eval(e, *p, plane, point);
+// Re-applies the epilogue to the N adjacent elements from p, of which this
+// thread has just stored the first `n` (kernels whose accumulator arrays must
+// stay in registers store them plainly first).  A thread reads its own earlier
+// stores in program order, so no fence is needed.
+template <int N>
+__device__ __forceinline__ void epi_rewrite(const Epi& e, float* p, int n, int plane, int point) {
+    float v[N];
+    int pl[N], pt[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int q = min(k, n - 1);
+        v[k] = p[q];
+        pl[k] = plane;
+        pt[k] = point + q;
+    }
+    epi_eval_n<N>(e, v, pl, pt);
+#pragma unroll
+    for (int k = 0; k < N; k++)
+        if (k < n) p[k] = v[k];
 }
 
 }  // namespace cogconv

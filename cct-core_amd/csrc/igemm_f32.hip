@@ -219,7 +219,11 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
     // cols] (plane pitch 260 words, 16-byte writes), written row by row with
     // 8-byte or single-float stores.
     __syncthreads();
-    const bool vec = ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 3) == 0 && (reinterpret_cast<uintptr_t>(O) & 15) == 0;
+    // With an epilogue every output takes the tile path, whose stores apply it
+    // to values read back from LDS (16 images 64x64x16 -> 32, 3x3, bias and
+    // rectifier: 23.6 us when the threads re-read their own global stores).
+    const bool vec = e.n == 0 && ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 3) == 0 &&
+                     (reinterpret_cast<uintptr_t>(O) & 15) == 0;
     if (vec) {  // block-uniform
         floatx4* red4 = reinterpret_cast<floatx4*>(smem);  // [rw][MB][4][64]
         if (pg == 1) {
@@ -241,20 +245,6 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
                     if (mm < Mout && orow < g.OH && ocol < g.OW)
                         store_out4(O + ((size_t)(b * Mout + mm) * ph.OHf + ph.oRow0 + orow) * ph.OWf + ph.oCol0 + ocol,
                                    sum[0], sum[1], sum[2], sum[3], e);
-                }
-            }
-            // The epilogue rewrites the thread's own stores (still in L2), so the
-            // accumulators above stay in registers whatever its code size.
-            if (e.n) {
-                for (int t = 0; t < MB * 4; t++) {
-                    const int mb = t >> 2, pb = t & 3;
-                    const int mm = m0 + mb * 16 + l16;
-                    const int orow = tr * 8 + 2 * rw + (pb >> 1);
-                    const int ocol = tc * 32 + (pb & 1) * 16 + 4 * g4;
-                    if (mm < Mout && orow < g.OH && ocol < g.OW)
-                        epi_rewrite4(e, O + ((size_t)(b * Mout + mm) * ph.OHf + ph.oRow0 + orow) * ph.OWf + ph.oCol0 +
-                                            ocol,
-                                     b * Mout + mm, (ph.oRow0 + orow) * ph.OWf + ph.oCol0 + ocol);
                 }
             }
         }
@@ -279,7 +269,31 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
             for (int pb = 0; pb < 4; pb++) *tile(mb, pb) = acc[mb][pb] + *tile(mb, pb);
     }
     __syncthreads();
-    if (ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 1) == 0 && (reinterpret_cast<uintptr_t>(O) & 7) == 0) {
+    if (e.n) {
+        // Whole 32-column rows, eight elements of a thread per epilogue pass; four
+        // where eight would take more registers than the rest of the kernel.
+        const int col = tid & 31, ocol = tc * 32 + col;
+        constexpr int N = PH || FR == 1 ? 4 : 8;
+        for (int item0 = tid >> 5; item0 < MT * 8; item0 += 16 * N) {
+            float v[N];
+            int pl[N], pt[N];
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const int item = item0 + 16 * k, mm = item >> 3, row = item & 7;
+                v[k] = sO[mm * OP + row * 32 + col];
+                pl[k] = b * Mout + min(m0 + mm, Mout - 1);
+                pt[k] = (ph.oRow0 + ph.oStride * min(tr * 8 + row, g.OH - 1)) * ph.OWf + ph.oCol0 +
+                        ph.oStride * min(ocol, g.OW - 1);
+            }
+            epi_eval_n<N>(e, v, pl, pt);
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const int item = item0 + 16 * k, mm = item >> 3, row = item & 7;
+                if (m0 + mm < Mout && tr * 8 + row < g.OH && ocol < g.OW)
+                    O[(size_t)pl[k] * ph.OHf * ph.OWf + pt[k]] = v[k];
+            }
+        }
+    } else if (ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 1) == 0 && (reinterpret_cast<uintptr_t>(O) & 7) == 0) {
         const int c2 = 2 * (tid & 15);  // 8-byte stores, 16 lanes per row
         const int ocol = tc * 32 + c2;
 #pragma unroll 4
@@ -288,9 +302,8 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
             const int orow = tr * 8 + row;
             if (m0 + mm < Mout && orow < g.OH && ocol < g.OW) {
                 const float2 v = *reinterpret_cast<const float2*>(sO + mm * OP + row * 32 + c2);
-                const int pt = (ph.oRow0 + orow) * ph.OWf + ph.oCol0 + ocol, pl = b * Mout + m0 + mm;
                 *reinterpret_cast<float2*>(O + ((size_t)(b * Mout + m0 + mm) * ph.OHf + ph.oRow0 + orow) * ph.OWf +
-                                           ph.oCol0 + ocol) = make_float2(epi(e, v.x, pl, pt), epi(e, v.y, pl, pt + 1));
+                                           ph.oCol0 + ocol) = v;
             }
         }
     } else {
@@ -301,8 +314,7 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
             const int orow = tr * 8 + row;
             if (m0 + mm < Mout && orow < g.OH && ocol < g.OW)
                 O[((size_t)(b * Mout + m0 + mm) * ph.OHf + ph.oRow0 + ph.oStride * orow) * ph.OWf + ph.oCol0 +
-                  ph.oStride * ocol] = epi(e, sO[mm * OP + row * 32 + col], b * Mout + m0 + mm,
-                                           (ph.oRow0 + ph.oStride * orow) * ph.OWf + ph.oCol0 + ph.oStride * ocol);
+                  ph.oStride * ocol] = sO[mm * OP + row * 32 + col];
         }
     }
 }
@@ -582,12 +594,7 @@ __device__ __forceinline__ void up2q_body(const Geom& g, const PlaneMap& m, cons
             const int orow = 2 * R + pr, ocol = 2 * C;
             float* dst = O + ((size_t)(b * Mout + mm) * g.OH + orow) * g.OW + ocol;
             const int pt = orow * g.OW + ocol;
-            if (vec && ocol + 8 <= g.OW) {
-                epi_rewrite4(e, dst, b * Mout + mm, pt);
-                epi_rewrite4(e, dst + 4, b * Mout + mm, pt + 4);
-            } else {
-                for (int v = 0; v < 8 && ocol + v < g.OW; v++) epi_rewrite1(e, dst + v, b * Mout + mm, pt + v);
-            }
+            epi_rewrite<8>(e, dst, min(8, g.OW - ocol), b * Mout + mm, pt);
         }
     }
 }

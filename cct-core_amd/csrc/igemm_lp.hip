@@ -530,6 +530,46 @@ __device__ __forceinline__ void igemm_lp_body(const Geom& g, const PlaneMap& m, 
     // m0 + 16 mb + l16 at the four adjacent pixels 4 g4 .. 4 g4 + 3 of its
     // 16-pixel run: one 16-byte store each where output rows are 16-byte
     // aligned (a 4-column group is then wholly inside or past the row).
+    if (e.n) {
+        // With an epilogue each wave passes its outputs, one 16-plane block at a
+        // time, through its own LDS region [16 planes][2 rows x 32 columns]
+        // (pitch EP; the tile is no longer needed), so that a runtime loop can
+        // apply the ops and the accumulators stay in registers; a wave then
+        // stores whole 32-column rows.
+        constexpr int EP = 68;
+        __syncthreads();
+        float* sE = reinterpret_cast<float*>(lp_smem) + wave * (16 * EP);
+        const int orow = tr * 8 + 2 * wave + (lane >> 5), ocol = tc * 32 + (lane & 31);
+        const bool inside = orow < g.OH && ocol < g.OW;
+        const int pt = min(orow, g.OH - 1) * g.OW + min(ocol, g.OW - 1);
+#pragma unroll 1
+        for (int mb = 0; mb < MB; mb++) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < MB; i++) {
+                if (i != mb) continue;  // wave-uniform: the accumulators keep compile-time indexes
+#pragma unroll
+                for (int pb = 0; pb < 4; pb++)
+                    *reinterpret_cast<floatx4*>(sE + l16 * EP + pb * 16 + 4 * g4) = acc[i][pb];
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int p0 = 0; p0 < 16; p0 += 4) {
+                float v[4];
+                int pl[4], pp[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    v[k] = sE[(p0 + k) * EP + lane];
+                    pl[k] = b * Mout + min(m0 + mb * 16 + p0 + k, Mout - 1);
+                    pp[k] = pt;
+                }
+                epi_eval_n<4>(e, v, pl, pp);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (inside && m0 + mb * 16 + p0 + k < Mout) O[(size_t)pl[k] * g.OH * g.OW + pt] = v[k];
+            }
+        }
+        return;
+    }
     const bool vec = (g.OW & 3) == 0 && (reinterpret_cast<uintptr_t>(O) & 15) == 0;
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
@@ -546,24 +586,6 @@ __device__ __forceinline__ void igemm_lp_body(const Geom& g, const PlaneMap& m, 
 #pragma unroll
                 for (int v = 0; v < 4; v++)
                     if (ocol + v < g.OW) dst[v] = acc[mb][pb][v];
-            }
-        }
-    }
-    // The epilogue rewrites the thread's own stores (still in L2), so the
-    // accumulators above stay in registers whatever its code size.
-    if (e.n) {
-        for (int t = 0; t < MB * 4; t++) {
-            const int mb = t >> 2, pb = t & 3;
-            const int mm = m0 + mb * 16 + l16;
-            const int orow = tr * 8 + 2 * wave + (pb >> 1);
-            const int ocol = tc * 32 + (pb & 1) * 16 + 4 * g4;
-            if (mm >= Mout || orow >= g.OH || ocol >= g.OW) continue;
-            float* dst = O + ((size_t)(b * Mout + mm) * g.OH + orow) * g.OW + ocol;
-            const int pl = b * Mout + mm, pt = orow * g.OW + ocol;
-            if (vec) {
-                epi_rewrite4(e, dst, pl, pt);
-            } else {
-                for (int v = 0; v < 4 && ocol + v < g.OW; v++) epi_rewrite1(e, dst + v, pl, pt + v);
             }
         }
     }

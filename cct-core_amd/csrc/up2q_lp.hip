@@ -232,12 +232,7 @@ __global__ __launch_bounds__(512) void k_up2q_lp(Geom g, PlaneMap m, UpFused u, 
             const int orow = 2 * R + pr, ocol = 2 * C;
             float* dst = O + ((size_t)(b * Mout + mm) * g.OH + orow) * g.OW + ocol;
             const int pt = orow * g.OW + ocol;
-            if (vec && ocol + 8 <= g.OW) {
-                epi_rewrite4(e, dst, b * Mout + mm, pt);
-                epi_rewrite4(e, dst + 4, b * Mout + mm, pt + 4);
-            } else {
-                for (int v = 0; v < 8 && ocol + v < g.OW; v++) epi_rewrite1(e, dst + v, b * Mout + mm, pt + v);
-            }
+            epi_rewrite<8>(e, dst, min(8, g.OW - ocol), b * Mout + mm, pt);
         }
     }
 }
