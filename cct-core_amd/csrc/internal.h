@@ -139,6 +139,7 @@ enum KernelKind {
     KK_IGEMM_UP = 7,
     KK_DIRECT_RT = 8,
     KK_FFT = 9,
+    KK_FRAME_ROWS = 10,
 };
 
 // LDS-tiled direct kernel configuration.
@@ -312,6 +313,14 @@ hipError_t launch_up2q_lp(int precision, const Geom& g, const PlaneMap& m, const
 hipError_t launch_igemm_lp(int precision, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
                            const float* w, float* out, void* ws, hipStream_t s, int stage = LP_PACK_AND_RUN,
                            const Epi& e = kNoEpi, const cogconv_image_io* tab = nullptr, bool x16 = false);
+// FP32 frame modes as split-BF16 products (frame_rows.hip): c.MB holds the
+// output rows of a wave, c.RC the planes padded to whole 16-plane chunks.
+bool frame_rows_supported(int F);
+size_t frame_rows_lds_bytes(int F, int RW);
+size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F);
+hipError_t launch_frame_rows(const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x, const float* w,
+                             float* out, void* ws, hipStream_t s, const Epi& e = kNoEpi,
+                             const cogconv_image_io* tab = nullptr);
 hipError_t launch_block_reduce_sum(const float* in, float* out, int64_t points, int out_planes, int factor,
                                    hipStream_t s, const Epi& e = kNoEpi);
 // out = epilogue(in) over `planes` planes of `points` (the unmerged elementwise pass).
@@ -340,6 +349,10 @@ int noalloc_setup(int device);
 // (tune.cpp): the tuned variant index for `desc` on the current device and the
 // description it had when it was timed.
 int plan_variant_count(const cogconv_desc* desc, int* count);
+// cogconv_plan_create for the serving loop: FP32 plans keep to the kernels
+// without a workspace, which its admission budget has no room set aside for,
+// and whose choice does not depend on how many requests are stacked.
+int plan_create_serving(const cogconv_desc* desc, cogconv_plan* plan);
 bool tune_cache_lookup(const cogconv_desc* desc, int* variant, std::string* name);
 
 }  // namespace cogconv

@@ -565,6 +565,57 @@ bool choose_igemm_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, Ig
     return false;
 }
 
+// FP32 frame block-reduce modes as split-BF16 products (k_frame_rows): unit
+// steps, square filters; `rw` output rows a wave.
+bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw) {
+    if (d->mode != COGCONV_PROJECT_FRAME_BLOCK_REDUCE_SUM && d->mode != COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM)
+        return false;
+    if (d->precision != COGCONV_FP32 || d->in0.dims != 2 || g.FH != g.FW || !frame_rows_supported(g.FH) ||
+        g.upAr != 1 || g.upAc != 1 || g.dnR != 1 || g.dnC != 1)
+        return false;
+    IgemmCfg c;
+    std::memset(&c, 0, sizeof c);
+    c.lds_bytes = frame_rows_lds_bytes(g.FH, rw);
+    if (c.lds_bytes == 0 || c.lds_bytes > 160 * 1024) return false;
+    c.MB = rw;
+    c.Mout = m.T / m.N;
+    c.mTiles = (c.Mout + 31) / 32;
+    c.tilesR = (g.OH + 4 * rw - 1) / (4 * rw);
+    c.tilesC = (g.OW + 31) / 32;
+    c.RC = (m.R + 15) / 16 * 16;
+    // 32-bit buffer offsets: an image with its planes padded to whole chunks,
+    // and 32 output planes.
+    if ((long)c.RC * g.H * g.W * 4 >= (1L << 31) || (long)32 * g.OH * g.OW * 4 >= (1L << 31)) return false;
+    // A packed bank within the no-allocation launch's scratch array, so that the
+    // plans it took keep running there.
+    if (frame_rows_workspace_bytes(c, g.FH) > (64UL << 20)) return false;
+    *out = c;
+    return true;
+}
+
+// Estimated time (us, two launches) of the split-BF16 frame kernel, and of the
+// FP32 MFMA frame kernel (one launch) on the same op: a launch floor, plus the
+// longer of one block's serial time and the whole grid's time at full load.  A
+// chunk costs its staging and its MFMA cycles at 2.4 GHz.  The constants fit 557
+// measured calls (sides 24 to 256, 3 to 64 planes, 1 to 64 outputs, batches 1 to
+// 32, filters 3x3 to 9x9); choosing the faster estimate loses 2% against always
+// knowing the faster kernel, and gains 1.34x over the FP32 MFMA kernel alone.
+double frame_rows_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
+    const double blocks = (double)c.tilesR * c.tilesC * c.mTiles * m.B, chunks = c.RC / 16;
+    const double mfma = c.MB * g.FH * g.FW * 6 * 32 / 2400.0;  // one wave's, six products of 32 cycles a tap and row
+    const double serial = chunks * (2.0 + mfma);
+    const double load = blocks / 256 * chunks * (1.7 * mfma + 0.002 * (4 * c.MB + g.FH - 1) * (31 + g.FW));
+    return 7.9 + std::max(serial, load);
+}
+
+double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
+    const double blocks = (double)c.tilesR * c.tilesC * c.mTiles * m.B, chunks = (m.R + c.RC - 1) / c.RC;
+    const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
+    const double serial = chunks * (4.7 + mfma);
+    const double load = blocks / 256 * chunks * (2.7 * mfma + 0.0072 * c.RC / 16 * (7 + g.FH) * (31 + g.FW));
+    return 4.9 + std::max(serial, load);
+}
+
 SmallCfg choose_small(const Geom& g, const PlaneMap& m, long blocks = 4096) {
     SmallCfg c;
     c.qchunks = (g.OH * g.OW + 15) / 16;
@@ -795,6 +846,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         if (fc) v.f = *fc;
         switch (kind) {
         case KK_IGEMM_LP: v.workspace = igemm_lp_workspace_bytes(v.i, g.FH, desc->precision); break;
+        case KK_FRAME_ROWS: v.workspace = frame_rows_workspace_bytes(v.i, g.FH); break;
         case KK_FA_IGEMM:
         case KK_FA_IGEMM_LP: v.workspace = (size_t)v.f.splits * v.f.K * m.N * outPts * sizeof(float); break;
         case KK_SMALL_OUTPUT: v.workspace = (size_t)v.s.splits * m.nOut * outPts * sizeof(float); break;
@@ -915,6 +967,19 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         // The largest tile that still gives two blocks per CU.
         while (rt_first < 2 && (long)drt[rt_first].tilesR * drt[rt_first].tilesC * m.nOut < 512) rt_first++;
     }
+    // The split-BF16 frame kernel where it is estimated faster than the FP32 MFMA
+    // one by more than the estimates' own error at the crossing (5%).
+    IgemmCfg rows[3];
+    bool rows_ok[3];
+    int rows_first = -1;
+    for (int i = 0; i < 3; i++) {
+        rows_ok[i] = choose_frame_rows(desc, g, m, &rows[i], i == 0 ? 1 : (i == 1 ? 2 : 8));
+        if (!rows_ok[i]) continue;
+        if (rows_first < 0 || frame_rows_us(g, m, rows[i]) < frame_rows_us(g, m, rows[rows_first])) rows_first = i;
+    }
+    if (rows_first >= 0 && igemm_ok &&
+        frame_rows_us(g, m, rows[rows_first]) > 0.95 * igemm_frame_us(g, m, ig))
+        rows_first = -1;
     PhaseSet up;
     const bool up_ok = choose_igemm_up(desc, g, m, &up);
     FftCfg fc;
@@ -934,13 +999,17 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     if (fft_first) add_fft(fc);
     else if (upq_ok) add_up(upq);
     else if (up_ok) add_up(up);
+    else if (rows_first >= 0) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[rows_first], nullptr);
     else if (igemm_ok) add(KK_IGEMM, nullptr, nullptr, &ig, nullptr);
     else if (fa_ok) add(KK_FA_IGEMM, nullptr, nullptr, nullptr, &fa);
     else if (small_out) add(KK_SMALL_OUTPUT, nullptr, &sm, nullptr, nullptr);
     else if (rt_ok) add(KK_DIRECT_RT, &drt[rt_first], nullptr, nullptr, nullptr);
     else add(KK_DIRECT, &dr, nullptr, nullptr, nullptr);
     // Alternatives.
+    for (int i = 0; i < 3; i++)
+        if (rows_ok[i]) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[i], nullptr);
     if (igemm_ok) {
+        add(KK_IGEMM, nullptr, nullptr, &ig, nullptr);
         for (int mb : {4, 2, 1})
             for (int rc : {32, 16, 8}) {
                 const IgemmCfg c = choose_igemm_frame(g, m, mb, rc);
@@ -993,14 +1062,14 @@ bool kind_matches_algo(int kind, int algo) {
     case COGCONV_ALGO_SMALL_OUTPUT: return kind == KK_SMALL_OUTPUT;
     case COGCONV_ALGO_IMPLICIT_GEMM:
         return kind == KK_IGEMM || kind == KK_FA_IGEMM || kind == KK_IGEMM_LP || kind == KK_FA_IGEMM_LP ||
-               kind == KK_IGEMM_UP;
+               kind == KK_IGEMM_UP || kind == KK_FRAME_ROWS;
     default: return true;
     }
 }
 
 // Builds the plan for variant `vi` of `desc` (vi < 0: by algorithm hint,
 // then by the autotuning cache, then the heuristic default).
-int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan) {
+int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving = false) {
     if (!plan) return fail(COGCONV_ERR_INVALID_ARG, "null plan pointer");
     *plan = nullptr;
     cogconv_field_type out;
@@ -1010,6 +1079,7 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan) {
     if (e) return e;
     std::vector<Variant> vars;
     enumerate_variants(desc, g, m, vars);
+    const auto offered = [&](int i) { return !(serving && vars[i].kind == KK_FRAME_ROWS); };
     if (vars.empty())
         return fail(COGCONV_ERR_UNSUPPORTED,
                     "precision %d is offered for ProjectFrame/BackProjectFrame with block reduction on 2-D fields with "
@@ -1027,7 +1097,7 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan) {
         if (desc->algo == COGCONV_ALGO_SMALL_OUTPUT && outPts > 4096)
             return fail(COGCONV_ERR_UNSUPPORTED, "small-output kernel needs an output plane of at most 4096 points");
         for (int i = 0; i < (int)vars.size() && pick < 0; i++)
-            if (kind_matches_algo(vars[i].kind, desc->algo)) pick = i;
+            if (kind_matches_algo(vars[i].kind, desc->algo) && offered(i)) pick = i;
         if (pick < 0)
             return fail(COGCONV_ERR_UNSUPPORTED,
                         "implicit GEMM needs a block-reduce frame mode with a square 1/3/5/7/9 filter on 2-D fields "
@@ -1035,9 +1105,10 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan) {
                         "planes per image in dy");
     } else {
         pick = 0;
+        while (!offered(pick) && pick + 1 < (int)vars.size()) pick++;
         int tuned;
         std::string tunedName;
-        if (tune_cache_lookup(desc, &tuned, &tunedName) && tuned < (int)vars.size()) {
+        if (tune_cache_lookup(desc, &tuned, &tunedName) && tuned < (int)vars.size() && offered(tuned)) {
             // Accept the cached index only if it still names the same configuration.
             cogconv_plan_s tmp;
             std::memset(&tmp, 0, sizeof tmp);
@@ -1111,6 +1182,11 @@ extern "C" int cogconv_output_type(const cogconv_desc* desc, cogconv_field_type*
 extern "C" int cogconv_plan_create(const cogconv_desc* desc, cogconv_plan* plan) {
     clear_error();
     return make_plan(desc, -1, plan);
+}
+
+int cogconv::plan_create_serving(const cogconv_desc* desc, cogconv_plan* plan) {
+    clear_error();
+    return make_plan(desc, -1, plan, true);
 }
 
 extern "C" int cogconv_plan_variant_count(const cogconv_desc* desc, int32_t* count) {
@@ -1195,6 +1271,11 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
                  plan->icfg.vec4 ? " ld16" : "", plan->icfg.trg, plan->icfg.ring ? " ring" : "", plan->icfg.lds_bytes);
         break;
     }
+    case KK_FRAME_ROWS:
+        snprintf(buf, len, "igemm_f32x3 %s out=%dx%dx%d tile=%dx32 rows=%d threads=256 lds=%zu",
+                 mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB, plan->icfg.MB,
+                 plan->icfg.lds_bytes);
+        break;
     case KK_IGEMM_UP: {
         if (plan->ps.f.on) {
             static const char* pn[] = {"f32", "bf16", "fp16", "split_bf16"};
@@ -1309,6 +1390,9 @@ int launch_all(cogconv_plan plan, const float* in0, const float* in1, float* out
         e = launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, in0, in1, out, workspace, s,
                             LP_PACK_AND_RUN, ep);
         break;
+    case KK_FRAME_ROWS:
+        e = launch_frame_rows(plan->g, plan->m, plan->icfg, in0, in1, out, workspace, s, ep);
+        break;
     case KK_IGEMM_UP:
         if (plan->ps.f.on && plan->desc.precision != COGCONV_FP32) {
             e = launch_up2q_lp(plan->desc.precision, plan->g, plan->m, plan->ps.f, in0, in1, out, workspace, s, ep);
@@ -1358,7 +1442,8 @@ extern "C" int cogconv_launch(cogconv_plan plan, const float* in0, const float* 
 }
 
 bool cogconv::plan_table_capable(const cogconv_plan_s* plan) {
-    return plan->kind == KK_IGEMM_LP || (plan->kind == KK_IGEMM && plan->m.mode != COGCONV_PLANE_BY_PLANE);
+    return plan->kind == KK_IGEMM_LP || plan->kind == KK_FRAME_ROWS ||
+           (plan->kind == KK_IGEMM && plan->m.mode != COGCONV_PLANE_BY_PLANE);
 }
 
 int cogconv::launch_table(cogconv_plan plan, const cogconv_image_io* device_table, bool x16, const float* in1,
@@ -1367,6 +1452,9 @@ int cogconv::launch_table(cogconv_plan plan, const cogconv_image_io* device_tabl
     if (plan->kind == KK_IGEMM_LP)
         e = launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, workspace, s,
                             packed ? LP_RUN_ONLY : LP_PACK_AND_RUN, plan->epi, device_table, x16);
+    else if (plan->kind == KK_FRAME_ROWS)
+        e = launch_frame_rows(plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, workspace, s, plan->epi,
+                              device_table);
     else
         e = launch_igemm_f32(plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, s, plan->epi, device_table);
     return check_hip(e, "table launch");

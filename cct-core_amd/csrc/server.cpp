@@ -270,7 +270,7 @@ struct cogconv_server_s {
         auto it = plans.find(k);
         if (it != plans.end()) return it->second;
         cogconv_plan p = nullptr;
-        *err = cogconv_plan_create(&d, &p);
+        *err = plan_create_serving(&d, &p);
         if (*err) return nullptr;
         plans[k] = p;
         return p;
@@ -772,7 +772,7 @@ extern "C" int cogconv_server_submit(cogconv_server s, const cogconv_request* re
     if (it == s->plans.end()) {
         lk.unlock();
         cogconv_plan p = nullptr;
-        const int pe = cogconv_plan_create(&d, &p);  // also rejects an illegal descriptor
+        const int pe = plan_create_serving(&d, &p);  // also rejects an illegal descriptor
         if (pe) {
             delete q;
             return pe;

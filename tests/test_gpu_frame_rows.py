@@ -1,0 +1,131 @@
+"""The split-BF16 form of the FP32 frame modes (igemm_f32x3 plans): parity with
+the FP64 oracle at the edges of its tiles, every candidate bit for bit alike,
+operands outside the split's range, unaligned buffers and request tables."""
+import numpy as np
+import pytest
+
+import cogconv._lib as L
+import oracle as O
+from gpuhelp import assert_parity, desc_pair, oracle_ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    L.init(0)
+    yield
+    L.synchronize()
+
+
+def candidates(cd):
+    """(igemm_f32x3 plans, the FP32 MFMA plan) of a descriptor."""
+    plans = [L.Plan(cd, v) for v in range(L.variant_count(cd))]
+    rows = [p for p in plans if p.description.startswith("igemm_f32x3")]
+    mfma = [p for p in plans if p.description.startswith("igemm_f32 ")]
+    return rows, mfma[0]
+
+
+def launch(plan, a, k, off=0):
+    """The plan's result, with operands and output `off` floats past an aligned address."""
+    n = int(np.prod(plan.out_shape))
+    ba, bk, bo = L.DeviceBuffer(4 * (a.size + off)), L.DeviceBuffer.from_array(k), L.DeviceBuffer(4 * (n + off))
+    ba.upload(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+    bo.upload(np.full(n + off, 7.0, np.float32))
+    ws = L.DeviceBuffer(plan.workspace_bytes) if plan.workspace_bytes else None
+    plan.launch(ba.ptr + 4 * off, bk, bo.ptr + 4 * off, ws)
+    L.synchronize()
+    out = bo.download((n + off,))
+    assert np.all(out[:off] == 7.0)
+    for b in (ba, bk, bo, ws):
+        if b is not None:
+            b.close()
+    return out[off:].reshape(plan.out_shape)
+
+
+@pytest.mark.parametrize("mode", (O.PF_BRS, O.BPF_BRS))
+@pytest.mark.parametrize("border,B,N,K,H,W,F", [
+    (O.ZERO, 1, 1, 1, 5, 7, 3),       # smaller than one tile in every dimension
+    (O.CLAMP, 2, 15, 31, 8, 32, 3),   # whole tile, partial chunk and output block
+    (O.CYCLIC, 1, 16, 32, 9, 33, 5),  # one row and column past the tile
+    (O.VALID, 1, 17, 33, 37, 45, 5),  # one plane past the chunk and the output block
+    (O.FULL, 2, 33, 5, 11, 30, 7),
+    (O.CLAMP, 1, 40, 9, 31, 64, 7),
+    (O.ZERO, 1, 20, 65, 33, 35, 9),
+    (O.CYCLIC, 1, 5, 3, 4, 5, 9),     # the filter larger than the field
+])
+def test_every_candidate(mode, border, B, N, K, H, W, F):
+    rng = np.random.default_rng(F * 100 + H)
+    a = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    k = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    orient = O.CONV if mode == O.BPF_BRS else O.XCORR
+    od, cd = desc_pair(mode, border, orient, O.NONE, 1, B, a.shape, k.shape)
+    rows, _ = candidates(cd)
+    assert rows
+    ref, mag = oracle_ref(od, a, k)
+    first = None
+    for i, p in enumerate(rows):
+        print("CASE rows", mode, border, p.description, flush=True)
+        got = launch(p, a, k, off=i)
+        assert_parity(got, ref, mag, what=p.description)
+        first = got if first is None else first
+        assert np.array_equal(got, first), p.description
+        p.close()
+
+
+@pytest.mark.parametrize("scale", (1e-36, 1e-30, 1e30))
+def test_magnitudes_beyond_the_split(scale):
+    """Operands whose low BF16 terms underflow, and large ones: as exact as near 1."""
+    rng = np.random.default_rng(5)
+    a = (rng.uniform(0.5, 1, (18, 20, 40)) * np.float64(scale)).astype(np.float32)
+    k = rng.uniform(0.5, 1, (34 * 18, 5, 5)).astype(np.float32)
+    od, cd = desc_pair(O.PF_BRS, O.CLAMP, O.XCORR, O.NONE, 1, 1, a.shape, k.shape)
+    rows, _ = candidates(cd)
+    ref, mag = oracle_ref(od, a, k)
+    for p in rows:
+        print("CASE magnitude", scale, p.description, flush=True)
+        # all terms positive: the oracle's magnitude sum is the result itself
+        assert np.abs(launch(p, a, k) - ref).max() <= 1e-5 * ref.max()
+        assert np.all(np.abs(launch(p, a, k) - ref) <= 1e-5 * mag)
+
+
+def test_non_finite_operands():
+    """Infinities, NaNs and the largest floats reach exactly the outputs they reach in
+    the FP32 MFMA kernel, and leave the others as they are."""
+    rng = np.random.default_rng(6)
+    a = rng.integers(-3, 4, (17, 24, 70)).astype(np.float32)
+    k = rng.integers(1, 4, (33 * 17, 3, 3)).astype(np.float32)
+    a[0, 0, 0], a[3, 10, 40], a[16, 23, 69], a[5, 20, 20] = np.inf, np.nan, -np.inf, 3.4028235e38
+    k[2 * 17 + 4, 1, 1], k[30 * 17, 0, 2] = np.inf, np.nan
+    for border in (O.ZERO, O.CLAMP):
+        _, cd = desc_pair(O.PF_BRS, border, O.XCORR, O.NONE, 1, 1, a.shape, k.shape)
+        rows, mfma = candidates(cd)
+        want = launch(mfma, a, k)
+        for p in rows:
+            print("CASE non-finite", border, p.description, flush=True)
+            got = launch(p, a, k)
+            assert np.array_equal(np.isnan(got), np.isnan(want)), p.description
+            assert np.array_equal(got, want, equal_nan=True), p.description  # small integers: every sum is exact
+
+
+def test_table_launch_equals_plain():
+    rng = np.random.default_rng(7)
+    B, N, K, H, W, F = 3, 18, 20, 26, 50, 5
+    a = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    k = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    _, cd = desc_pair(O.PF_BRS, O.ZERO, O.XCORR, O.NONE, 1, B, a.shape, k.shape)
+    rows, _ = candidates(cd)
+    for p in rows:
+        print("CASE table", p.description, flush=True)
+        want = launch(p, a, k)
+        assert p.table_supported()
+        order = [2, 0, 1]  # images at unrelated addresses, in another order
+        ins = [L.DeviceBuffer.from_array(a[b * N:(b + 1) * N]) for b in range(B)]
+        outs = [L.DeviceBuffer(4 * K * H * W) for _ in range(B)]
+        bk, tab, ws = L.DeviceBuffer.from_array(k), L.DeviceBuffer(16 * B), L.DeviceBuffer(p.workspace_bytes)
+        p.launch_table([(ins[b], outs[b]) for b in order], tab, in1=bk, workspace=ws)
+        L.synchronize()
+        for b in range(B):
+            assert np.array_equal(outs[b].download((K, H, W)), want[b * K:(b + 1) * K])
+        for x in ins + outs + [bk, tab, ws]:
+            x.close()
