@@ -1,33 +1,46 @@
-// FP32 frame block-reduce modes on the BF16 matrix cores, every FP32 operand
-// split exactly into three BF16 terms:
+// Frame block-reduce modes on the BF16 / FP16 matrix cores, walking down the rows:
 //
 //   out[b*Mout + m](y, x) = sum_{r < R} sum_{t < F*F} A[m][r][t] * X_{b*N + r}(y - h + ti, x - h + tj)
 //
 // (the contraction of igemm_f32.hip; ConvolveHyperKernel.scala:153-167, 327-332,
-// borders 235-317).  x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),
-// x2 = x - x0 - x1: round to nearest leaves remainders of 16 and 8 bits, so the
-// three terms hold all 24 bits of x.  Of the nine products of two split operands
-// the six with term indexes summing to at most 2 are computed, each exact on the
-// MFMA with FP32 accumulation; the other three are below 2^-25 of the product,
-// under the rounding of one FP32 multiply.  Six BF16 MFMAs do the work of one
-// FP32 MFMA in 6/16 of its cycles.
+// borders 235-317), for operands of T terms:
 //
-// gfx950 mapping: v_mfma_f32_32x32x16_bf16, A = filters (32 output planes x 16
-// input planes at one tap), B = pixels (16 planes x 32 pixels of a row).  A block
-// of four waves owns 4*RW x 32 pixels and 32 output planes; a wave owns RW rows.
+//   BF16, FP16    T = 1: operands rounded once, one product.
+//   split-BF16    T = 2: x = x0 + x1, the products x0 w0 + x0 w1 + x1 w0.
+//   FP32          T = 3, exact: x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),
+//     x2 = x - x0 - x1.  Round to nearest leaves remainders of 16 and 8 bits, so the
+//     terms hold all 24 bits of x.  Of the nine products of two operands the six
+//     with term indexes summing to at most 2 are computed, each exact on the
+//     MFMA with FP32 accumulation; the other three are below 2^-25 of the product,
+//     under the rounding of one FP32 multiply.  Six BF16 MFMAs do the work of one
+//     FP32 MFMA in 6/16 of its cycles.
+//
+// gfx950 mapping: v_mfma_f32_32x32x16, A = filters (32 output planes x 16 input
+// planes at one tap), B = pixels (16 planes x 32 pixels of a row).  A block of
+// four waves owns 4*RW x 32 pixels and 32 output planes; a wave owns RW rows.
 // Input planes are staged 16 at a time, split, 8 planes (16 bytes) of a pixel to
-// an LDS slot.  For tap column j a wave holds the F tap rows of its filters in
+// an LDS slot; with 16-byte loads of 4 columns where rows are 16-byte aligned
+// (BF16, 24 -> 24 planes and the like: 1.02-1.07x the 4-byte loads at up to two
+// rows a wave, 0.95x at four, which keeps the 4-byte ones).  For tap column j a
+// wave holds the F tap rows of its filters in
 // registers and walks down the tile: the pixels of tile row y, read from LDS once
 // per tap column, meet tap row i for every output row y - i the wave owns.  So an
 // LDS read of a pixel fragment feeds up to F tap rows and a filter fragment RW
 // rows: RW = 4, 9x9: 63 16-byte reads for 216 MFMAs of 32 cycles a tap column.
 // Filter fragments come straight from the packed bank in L2 (1 KiB contiguous
-// each), loaded into the registers of the fragment they replace right after its
-// last use, a tap column ahead.
+// each) and pass through a ring of registers: each is loaded into the registers of
+// the fragment it replaces right after that one's last use, a tap column ahead.
 //
 // A lane's accumulators hold one pixel of 16 output planes, so a store
 // instruction writes whole 32-pixel rows of two planes at any alignment.
+//
+// Measured against the kernels it replaced (us a call): FP32 9x9, 32 -> 32 planes,
+// 8 images 256x256: 730 -> 331; split-BF16 3x3, 64 -> 64 planes, 32 images 128x128:
+// 170 -> 122; BF16 and FP16 3x3 to 9x9 over 400 random calls (3 to 64 planes, 24 to
+// 256 a side): 1.5x.  What bounds it: the matrix cores at FP32 (70% of their peak
+// at 9x9); for one term the latency of staging and of the filter stream.
 #include <algorithm>
+#include <type_traits>
 
 #include "epi.h"
 #include "lp.h"
@@ -38,29 +51,84 @@ namespace cogconv {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int FR_RC = 16;  // planes of a staged chunk (one MFMA k slice)
-// Outputs below this are computed again in plain FP32: operands near its square
-// root or above keep every term a normal BF16 number.
-constexpr float FR_TINY = 0x1p-100f;
+// Operands below this may lose bits of their last BF16 term (under 2^-126).
+constexpr float FR_SMALL = 0x1p-102f;
 
-// Splits w into T terms of type V's element: term t rounds what the earlier ones left.
-template <int T>
-__device__ __forceinline__ void split_terms(float x, __bf16 (&t)[T]) {
+// BF16 terms of an operand.
+constexpr int fr_terms(int prec) { return prec == COGCONV_FP32 ? 3 : (prec == COGCONV_SPLIT_BF16 ? 2 : 1); }
+
+// How taps meet the staged samples.
+//   FR_UNIT  unit steps: output row r sees tap row i at staged row r + i.
+//   FR_UP0 / FR_UP1  input up-sampled by 2, filter halo h even / odd: output row
+//     2r + p sees the tap rows i = h + p (mod 2), at stored row
+//     r + ceil((i - h) / 2); staged row 0 is stored row r0 - floor(h / 2); the
+//     same for columns.  Wave s of a pair (s = 0, 1) sums the even tap rows of
+//     the tap columns j = s (mod 2), then the odd ones of the others: two of the
+//     four output phases of its rows, (F*F + 1) / 2 taps for s = 0 and one less
+//     for s = 1, half a tap column held at a time.
+//   FR_DOWN  every second output.
+template <int F, int RW, int S, int T>
+struct FrameRows {
+    static constexpr bool UP = S == FR_UP0 || S == FR_UP1;
+    static constexpr int P = S == FR_UP1;                       // parity of h
+    static constexpr int STEP = S == FR_DOWN ? 2 : 1;
+    static constexpr int NP = UP ? 2 : 1;                       // phases of a dimension
+    static constexpr int off(int i) { return UP ? (i + 1 - P) / 2 : i; }
+    static constexpr int taps(int set) { return UP ? (F - set + 1) / 2 : F; }  // even / odd tap rows
+    static constexpr int TH = 4 * RW / NP;                      // output rows (of a phase) of a block
+    static constexpr int TR = STEP * (TH - 1) + off(F - 1) + 1; // staged rows
+    static constexpr int TC = STEP * 31 + off(F - 1) + 1;       // staged columns
+    static constexpr int HC = (TC + 1) / 2;                     // FR_DOWN: even columns first, then odd ones
+    static constexpr int NPIX = TR * TC;
+    // Aligned groups of 4 columns over a tile: it starts up to S4 columns into one
+    // (at -h mod 4, for h = 0, (F - 1) / 2 and F - 1).
+    static constexpr int S4 = F == 3 ? 3 : (F == 9 ? 0 : 2);
+    static constexpr int NG = (TC + S4 + 3) / 4;
+    static constexpr int LDS = 2 * T * NPIX * 16 + 16;          // and the tile's extreme magnitudes
+};
+
+// Splits x into T terms: term t rounds what the earlier ones left.
+template <int T, class E>
+__device__ __forceinline__ void split_terms(float x, E (&t)[T]) {
 #pragma unroll
     for (int k = 0; k < T; k++) {
-        t[k] = (__bf16)x;
+        t[k] = (E)x;
         if (k + 1 < T) x -= (float)t[k];
     }
 }
 
+template <int PREC>
+__device__ __forceinline__ floatx16 fr_mfma(typename LpType<PREC>::V a, typename LpType<PREC>::V b, floatx16 c) {
+    if constexpr (PREC == COGCONV_FP16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, d));
+    return v;
+}
+
+__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// Whether any lane's operands go under FR_SMALL; `least`: the smallest magnitude(x) - 1, which puts zeros last.
+__device__ __forceinline__ bool any_small(unsigned least) { return __any(least < __float_as_uint(FR_SMALL) - 1u); }
+
 // Packed bank: [32-plane output block][16-plane chunk][tap column j][tap row i][term][lane][8], where lane l
 // holds output plane l % 32 and input planes 8 (l / 32) .. + 7 (zeros past the planes), taps flipped for the
-// convolution orientation.
-template <int T>
+// convolution orientation.  After it, for the FP32 plans, one uint2 a [block][chunk][j][i]: the fragment's largest
+// magnitude (bits), and whether it holds operands under FR_SMALL.
+template <int PREC, int T>
 __global__ void k_pack_rows(Geom g, PlaneMap m, int Mout, int chunks, long total, const float* __restrict__ Wt,
-                            __bf16* __restrict__ Wp) {
+                            typename LpType<PREC>::T* __restrict__ Wp) {
+    typedef typename LpType<PREC>::T E;
+    typedef typename LpType<PREC>::V V;
     const int F = g.FH, taps = F * F;
     const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
     const int L = m.T / m.N;
+    uint2* range = reinterpret_cast<uint2*>(Wp + total * T * 8);
     for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
         const int lane = (int)(idx & 63);
         long rest = idx >> 6;
@@ -71,34 +139,48 @@ __global__ void k_pack_rows(Geom g, PlaneMap m, int Mout, int chunks, long total
         const int ch = (int)(rest % chunks);
         const int mm = (int)(rest / chunks) * 32 + (lane & 31);
         const int t = g.flip ? taps - 1 - (i * F + j) : i * F + j;
-        bf16x8 v[T];
+        V v[T];
+        unsigned most = 0u, least = ~0u;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const int r = ch * FR_RC + 8 * (lane >> 5) + e;
             float w = 0.f;
             if (r < m.R && mm < Mout) w = Wt[(size_t)(bpf ? r * L + mm : mm * m.N + r) * taps + t];
-            __bf16 q[T];
+            most = max(most, magnitude(w));
+            least = min(least, magnitude(w) - 1u);
+            E q[T];
             split_terms<T>(w, q);
 #pragma unroll
             for (int k = 0; k < T; k++) v[k][e] = q[k];
         }
 #pragma unroll
-        for (int k = 0; k < T; k++)
-            *reinterpret_cast<bf16x8*>(Wp + (((idx >> 6) * T + k) * 64 + lane) * 8) = v[k];
+        for (int k = 0; k < T; k++) *reinterpret_cast<V*>(Wp + (((idx >> 6) * T + k) * 64 + lane) * 8) = v[k];
+        if (T == 3) {  // `total` is whole waves
+            most = wave_max(most);
+            const bool small = any_small(least);
+            if (lane == 0) range[idx >> 6] = make_uint2(most, small);
+        }
     }
 }
 
 // One output element by plain FP32 multiply-adds, four planes a tap as in the FP32
-// MFMA kernel (taps off the field multiply 0, as everywhere else).
+// MFMA kernel (taps off the field multiply 0, as everywhere else; no inserted zero
+// of an up-sampled field multiplies).
 __device__ __forceinline__ float frame_point(const Geom& g, const PlaneMap& m, const float* Xb, const float* Wt, int mm,
-                                          int orow, int ocol) {
+                                             int orow, int ocol) {
     const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
     const int L = m.T / m.N, taps = g.FH * g.FW;
+    const bool up = g.upAr == 2;
     float s = 0.f;
     for (int r0 = 0; r0 < m.R; r0 += 4)
         for (int i = 0; i < g.FH; i++)
             for (int j = 0; j < g.FW; j++) {
-                int y = orow - g.hR + i, c = ocol - g.hC + j;
+                int y = orow * g.dnR - g.hR + i, c = ocol * g.dnC - g.hC + j;
+                if (up) {
+                    if ((y | c) & 1) continue;
+                    y >>= 1;
+                    c >>= 1;
+                }
                 bool in = (unsigned)y < (unsigned)g.H && (unsigned)c < (unsigned)g.W;
                 if (g.border == COGCONV_BORDER_CYCLIC) {
                     y %= g.H;
@@ -119,24 +201,20 @@ __device__ __forceinline__ float frame_point(const Geom& g, const PlaneMap& m, c
     return s;
 }
 
-template <int F, int RW>
-struct FrameRows {
-    static constexpr int T = 3;
-    static constexpr int TH = 4 * RW;               // output rows of a block
-    static constexpr int TR = TH + F - 1;           // staged rows
-    static constexpr int TC = 31 + F;               // staged columns
-    static constexpr int NPIX = TR * TC;
-    static constexpr int LDS = 2 * T * NPIX * 16;
-};
-
-template <int F, int RW, int OCC>
+template <int F, int RW, int OCC, int S, int PREC, bool VEC>
 __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, IgemmCfg c, const float* __restrict__ X,
-                                                         const float* __restrict__ Wt, const __bf16* __restrict__ Wp,
+                                                         const float* __restrict__ Wt,
+                                                         const typename LpType<PREC>::T* __restrict__ Wp,
                                                          float* __restrict__ O,
                                                          const cogconv_image_io* __restrict__ tab, Epi e) {
-    typedef FrameRows<F, RW> S;
-    constexpr int T = S::T, TC = S::TC, NPIX = S::NPIX;
+    constexpr int T = fr_terms(PREC);
+    typedef FrameRows<F, RW, S, T> Z;
+    typedef typename LpType<PREC>::T E;
+    typedef typename LpType<PREC>::V V;
+    constexpr int TC = Z::TC, NPIX = Z::NPIX, NP = Z::NP, NA = NP * RW, NT = Z::taps(0);
+    constexpr bool EXACT = T == 3;  // FP32 results
     extern __shared__ __attribute__((aligned(16))) unsigned char fr_smem[];
+    unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem + 2 * T * NPIX * 16);
 
     // Output-plane blocks of one tile are adjacent block indices (same XCD).
     int bid = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -150,22 +228,47 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, l32 = lane & 31;
+    const int pair = wave & 1;  // FR_UP
+    const int row0 = (Z::UP ? wave >> 1 : wave) * RW;
     const int Mout = c.Mout, m0 = mt * 32;
     const int HW = g.H * g.W, OHW = g.OH * g.OW;
     const float* Xb = tab ? tab[b].in0 : X + (size_t)b * m.N * HW;
     float* Ob = tab ? tab[b].out : O + (size_t)b * Mout * OHW;
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(Xb, (uint32_t)m.N * HW * 4u);  // the plan bounds this by 2^31
 
-    // Staged pixels of this thread: tid, tid + 256, ...; byte offsets within a
-    // plane with the border applied, or out of range (reads 0).
-    constexpr int NS = (NPIX + 255) / 256;
+    // Staging units of this thread, numbers tid, tid + 256, ...: a pixel (all 16
+    // planes of a chunk), or (VEC) 8 planes of an aligned group of 4 columns, which
+    // a row of W % 4 == 0 columns holds or leaves out as a whole.  Byte offsets
+    // within a plane with the border applied, or out of range (reads 0).
+    constexpr int NS = VEC ? (2 * Z::NG * Z::TR + 255) / 256 : (NPIX + 255) / 256;
+    // The next chunk's loads run under this one's MFMAs where registers allow.
+    constexpr bool AHEAD = NS <= (VEC ? 1 : S == FR_DOWN ? 3 : 2);
+    const int y0 = tr * Z::TH * Z::STEP - (Z::UP ? g.hR >> 1 : g.hR);
+    const int x0 = tc * 32 * Z::STEP - (Z::UP ? g.hC >> 1 : g.hC);
     int pOff[NS];
+    int pix[VEC ? NS : 1];          // VEC: 4 * (half * T * NPIX + pixel of the group's first column) + clamp
 #pragma unroll
     for (int k = 0; k < NS; k++) {
-        const int p = tid + 256 * k;
-        const int ty = p / TC, tx = p - ty * TC;
-        int y = tr * S::TH - g.hR + ty;
-        const int xo = stage_col_offset(g, tc * 32 - g.hC + tx);
+        const int u = tid + 256 * k;
+        int ty, x;
+        bool live;
+        if constexpr (VEC) {
+            const int h = u / (Z::NG * Z::TR), q = u - h * (Z::NG * Z::TR);
+            ty = q / Z::NG;
+            x = (x0 & ~3) + 4 * (q - ty * Z::NG);
+            live = h < 2;
+            const int side = g.border == COGCONV_BORDER_CLAMP ? (x < 0 ? 1 : (x >= g.W ? 2 : 0)) : 0;
+            pix[k] = 4 * (h * T * NPIX + ty * TC + x - x0) + side;
+            // The clamped column is in the first or the last group.
+            if (side) x = side == 1 ? 0 : g.W - 4;
+        } else {
+            ty = u / TC;
+            const int slot = u - ty * TC;
+            x = x0 + (S == FR_DOWN ? (slot < Z::HC ? 2 * slot : 2 * (slot - Z::HC) + 1) : slot);
+            live = u < NPIX;
+        }
+        int y = y0 + ty;
+        const int xo = stage_col_offset(g, x);
         bool in = (unsigned)y < (unsigned)g.H;
         if (g.border == COGCONV_BORDER_CYCLIC) {
             y %= g.H;
@@ -175,136 +278,264 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
             in = in || g.border == COGCONV_BORDER_CLAMP;
             y = min(max(y, 0), g.H - 1);
         }
-        pOff[k] = in && xo >= 0 && p < NPIX ? 4 * y * g.W + xo : STAGE_OOB;
+        pOff[k] = in && xo >= 0 && live ? 4 * y * g.W + xo : STAGE_OOB;
     }
 
-    // The five products with a low term sum apart from the leading one: in one
-    // accumulator each would round at the running sum's magnitude, six roundings
-    // a slice (9x9, 32 planes: relative error 7.9e-7, 3.0e-7 apart, and
+    // EXACT: the five products with a low term sum apart from the leading one: in
+    // one accumulator each would round at the running sum's magnitude, six
+    // roundings a slice (9x9, 32 planes: relative error 7.9e-7, 3.0e-7 apart, and
     // 6.4e-7 for the FP32 MFMA kernel, which rounds every 4 planes).
-    floatx16 acc[RW], low[RW];
+    // Accumulator set * RW + r: row r of the wave (FR_UP: even, odd tap rows).
+    floatx16 acc[NA], low[EXACT ? NA : 1];
 #pragma unroll
-    for (int r = 0; r < RW; r++)
+    for (int r = 0; r < NA; r++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[r][v] = low[r][v] = 0.f;
+        for (int v = 0; v < 16; v++) {
+            acc[r][v] = 0.f;
+            if (EXACT) low[EXACT ? r : 0][v] = 0.f;
+        }
 
     // The block's filter stream: per (chunk, tap column) F * T fragments of 1 KiB.
     const int chunks = c.RC / FR_RC;
     constexpr int FRAG = 1024, COLB = F * T * FRAG;
     const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(reinterpret_cast<const char*>(Wp) + (size_t)mt * chunks * F * COLB,
                                                   (uint32_t)(chunks * F * COLB));
-    int wOff = lane * 16;  // of the tap column whose fragments are loaded next (past the end: reads 0)
-    bf16x8 a[F][T];
+    // FR_UP: the wave's k-th tap column of a chunk, even tap rows for k < kOdd.
+    const int kOdd = (F - pair + 1) / 2;
+    auto tap_column = [&](int k) __attribute__((always_inline)) {
+        return !Z::UP ? k : (k < kOdd ? pair + 2 * k : 1 - pair + 2 * (k - kOdd));
+    };
+    // Byte offset of the fragments after column k of chunk ch (past the end: reads 0).
+    auto next_column = [&](int ch, int k) __attribute__((always_inline)) {
+        ch += k + 1 == F;
+        k = k + 1 == F ? 0 : k + 1;
+        return lane * 16 + (ch * F + tap_column(k)) * COLB + (Z::UP && k >= kOdd ? T * FRAG : 0);
+    };
+    // Filters held: a tap column, loaded one ahead, or all F of a chunk (DEEP, where
+    // they fit registers), loaded a chunk ahead.
+    constexpr bool DEEP = S == FR_UNIT && F == 3 && T == 1;
+    V a[DEEP ? F : 1][NT][T];
+    auto fragment = [&](int at, int i, int t) __attribute__((always_inline)) {
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(wr, at, (NP * i * T + t) * FRAG, 0));
+    };
 #pragma unroll
-    for (int i = 0; i < F; i++)
+    for (int k = 0; k < (DEEP ? F : 1); k++)
 #pragma unroll
-        for (int t = 0; t < T; t++)
-            a[i][t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, wOff, (i * T + t) * FRAG, 0));
-    wOff += COLB;
-
-    const int rdBase = ((half * T) * NPIX + wave * RW * TC + l32) * 16;
-    for (int ch = 0; ch < chunks; ch++) {
-        if (ch) __syncthreads();
+        for (int i = 0; i < NT; i++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            // Batches of at most 8 pixels (64 loads in flight a thread).
-            constexpr int NB = NS <= 8 ? NS : 4;
-#pragma unroll
-            for (int k0 = 0; k0 < NS; k0 += NB) {
-                float v[NB][8];
-#pragma unroll
-                for (int k = 0; k < NB; k++) {
-                    if (k0 + k >= NS) continue;
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        const int r = ch * FR_RC + 8 * h + q;
-                        v[k][q] = buffer_load_f32(xr, r < m.R ? pOff[k0 + k] : STAGE_OOB, 4 * r * HW);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the first store
-#pragma unroll
-                for (int k = 0; k < NB; k++) {
-                    const int p = tid + 256 * (k0 + k);
-                    if (k0 + k >= NS || p >= NPIX) continue;
-                    bf16x8 s[T];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        __bf16 t3[T];
-                        split_terms<T>(v[k][q], t3);
-#pragma unroll
-                        for (int t = 0; t < T; t++) s[t][q] = t3[t];
-                    }
-#pragma unroll
-                    for (int t = 0; t < T; t++)
-                        *reinterpret_cast<bf16x8*>(fr_smem + ((h * T + t) * NPIX + p) * 16) = s[t];
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll 1
-        for (int j = 0; j < F; j++) {
-            const unsigned char* bp = fr_smem + rdBase + j * 16;
-#pragma unroll
-            for (int y = 0; y < RW + F - 1; y++) {
-                bf16x8 bv[T];
-#pragma unroll
-                for (int t = 0; t < T; t++) bv[t] = *reinterpret_cast<const bf16x8*>(bp + (t * NPIX + y * TC) * 16);
-                // Products in order of the pixel term, so the first MFMAs wait for one read only.
-#pragma unroll
-                for (int tb = 0; tb < T; tb++)
-#pragma unroll
-                    for (int ta = 0; ta + tb < T; ta++)
-#pragma unroll
-                        for (int i = 0; i < F; i++) {
-                            const int r = y - i;
-                            if (r < 0 || r >= RW) continue;
-                            if (ta + tb == 0)
-                                acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], bv[0], acc[r], 0, 0, 0);
-                            else
-                                low[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][ta], bv[tb], low[r], 0, 0, 0);
-                        }
-                // Tap row y - (RW - 1) has met its last row: its registers take the next tap column's.
-                if (y >= RW - 1) {
-                    const int i = y - (RW - 1);
-#pragma unroll
-                    for (int t = 0; t < T; t++)
-                        a[i][t] = __builtin_bit_cast(
-                            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, wOff, (i * T + t) * FRAG, 0));
-                }
-            }
-            wOff += COLB;
-        }
+            for (int t = 0; t < T; t++) a[k][i][t] = fragment(DEEP ? lane * 16 + k * COLB : next_column(-1, F - 1), i, t);
+    // EXACT: whether the bank (smallW) and the tile (sRange[0]) hold operands under FR_SMALL.
+    const uint2* range = reinterpret_cast<const uint2*>(Wp + (size_t)c.mTiles * chunks * F * F * T * 512) +
+                         (size_t)mt * chunks * F * F;
+    bool smallW = false;
+    if (EXACT) {
+        for (int i = lane; i < chunks * F * F; i += 64) smallW |= range[i].y != 0;
+        if (tid < 2) sRange[tid] = 0u;
+        __syncthreads();  // before the first chunk's stores
     }
 
-    // Lane (half, l32), register v of acc[r]: output plane m0 + 8 (v / 4) + 4 half + v % 4, pixel l32 of the
-    // wave's row r.
-    const int orow0 = tr * S::TH + wave * RW, ocol = tc * 32 + l32;
+    const int rdBase = ((half * T) * NPIX + row0 * Z::STEP * TC + l32) * 16;
+    // The wave's k-th tap column of chunk ch, tap rows of set SET.
+    auto column = [&](int ch, int k, auto SET) __attribute__((always_inline)) {
+        constexpr int N = Z::taps(SET);
+        const int j = tap_column(k), next = DEEP ? lane * 16 + ((ch + 1) * F + k) * COLB : next_column(ch, k);
+        const int d = DEEP ? k : 0;
+        const int off = S == FR_DOWN ? (j & 1) * Z::HC + (j >> 1) : Z::off(j);
+        const unsigned char* bp = fr_smem + rdBase + (Z::off(SET) * TC + off) * 16;
+#pragma unroll
+        for (int y = 0; y < Z::STEP * (RW - 1) + N; y++) {
+            V bv[T];
+#pragma unroll
+            for (int t = 0; t < T; t++) bv[t] = *reinterpret_cast<const V*>(bp + (t * NPIX + y * TC) * 16);
+            // Products in order of the pixel term, so the first MFMAs wait for one read only.
+#pragma unroll
+            for (int tb = 0; tb < T; tb++)
+#pragma unroll
+                for (int ta = 0; ta + tb < T; ta++)
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        const int r = y - i;
+                        if (r < 0 || r % Z::STEP || r / Z::STEP >= RW) continue;
+                        const int at = SET * RW + r / Z::STEP;
+                        if (!EXACT || ta + tb == 0) acc[at] = fr_mfma<PREC>(a[d][i][ta], bv[tb], acc[at]);
+                        else low[EXACT ? at : 0] = fr_mfma<PREC>(a[d][i][ta], bv[tb], low[EXACT ? at : 0]);
+                    }
+            // A tap row that has met its last row gives its registers to the next tap column's.
+            if (y >= Z::STEP * (RW - 1)) {
+                const int i = y - Z::STEP * (RW - 1);
+#pragma unroll
+                for (int t = 0; t < T; t++) a[d][i][t] = fragment(next, i, t);
+            }
+        }
+        // The odd tap rows are one fewer: the last register set is only needed by
+        // the even ones of the next chunk.
+        if (N < NT)
+#pragma unroll
+            for (int t = 0; t < T; t++) a[0][NT - 1][t] = fragment(k + 1 == F ? next : STAGE_OOB, NT - 1, t);
+    };
+    // A chunk is staged in batches of loads: every plane of the thread's units (one
+    // memory round trip) where they are loaded ahead, otherwise (VEC) a unit at a
+    // time, or a half of the planes of at most 8 pixels.
+    constexpr int NB = AHEAD ? NS : VEC ? 1 : NS <= 8 ? NS : 4, HB = AHEAD && !VEC ? 2 : 1;
+    float v[NB][VEC ? 1 : 8 * HB];
+    floatx4 v4[NB][VEC ? 8 : 1];
+    auto load = [&](int ch, int h0, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            if (k0 + k >= NS) continue;
+            if constexpr (VEC) {
+                const int r8 = ch * FR_RC + 8 * (tid + 256 * (k0 + k) >= Z::NG * Z::TR);
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    // The plane is per lane (the two halves meet in a wave): plane, then a scalar one.
+                    const int at = r8 + q < m.R ? pOff[k0 + k] + 4 * (r8 - ch * FR_RC) * HW : STAGE_OOB;
+                    v4[k][q] = __builtin_bit_cast(
+                        floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, pOff[k0 + k] < 0 ? STAGE_OOB : at,
+                                                                       4 * (ch * FR_RC + q) * HW, 0));
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 8 * HB; q++) {
+                    const int r = ch * FR_RC + 8 * h0 + q;
+                    v[k][q] = buffer_load_f32(xr, r < m.R ? pOff[k0 + k] : STAGE_OOB, 4 * r * HW);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the first store
+    };
+    unsigned most = 0u;
+    auto store = [&](int h0, int k0) __attribute__((always_inline)) {
+        unsigned least = ~0u;
+        // One slot: 8 planes of a pixel, every term.
+        auto slot = [&](const float (&x)[8], int at) __attribute__((always_inline)) {
+            V s[T];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                if (EXACT) {
+                    most = max(most, magnitude(x[q]));
+                    least = min(least, magnitude(x[q]) - 1u);
+                }
+                E t3[T];
+                split_terms<T>(x[q], t3);
+#pragma unroll
+                for (int t = 0; t < T; t++) s[t][q] = t3[t];
+            }
+#pragma unroll
+            for (int t = 0; t < T; t++) *reinterpret_cast<V*>(fr_smem + (at + t * NPIX) * 16) = s[t];
+        };
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const int u = tid + 256 * (k0 + k);
+            if (k0 + k >= NS) continue;
+            if constexpr (VEC) {
+                if (u >= 2 * Z::NG * Z::TR) continue;
+                const int h = u >= Z::NG * Z::TR, q = u - h * (Z::NG * Z::TR);
+                const int tx = (x0 & ~3) - x0 + 4 * (q % Z::NG), side = pix[k0 + k] & 3;
+#pragma unroll
+                for (int c4 = 0; c4 < 4; c4++) {
+                    if (tx + c4 < 0 || tx + c4 >= TC) continue;
+                    float x[8];
+#pragma unroll
+                    for (int p = 0; p < 8; p++) {
+                        const floatx4 w = v4[k][p];
+                        x[p] = w[c4];
+                        x[p] = side == 1 ? w[0] : x[p];
+                        x[p] = side == 2 ? w[3] : x[p];
+                    }
+                    slot(x, (pix[k0 + k] >> 2) + c4);
+                }
+            } else {
+                if (u >= NPIX) continue;
+#pragma unroll
+                for (int h = 0; h < HB; h++) {
+                    float x[8];
+#pragma unroll
+                    for (int p = 0; p < 8; p++) x[p] = v[k][8 * h + p];
+                    slot(x, (h0 + h) * T * NPIX + u);
+                }
+            }
+        }
+        if (EXACT && any_small(least) && lane == 0) sRange[0] = 1u;
+    };
+    if (AHEAD) load(0, 0, 0);
+    for (int ch = 0; ch < chunks; ch++) {
+        if (ch) __syncthreads();
+        if (AHEAD) {
+            store(0, 0);
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; h += VEC ? 2 : HB)
+#pragma unroll
+                for (int k0 = 0; k0 < NS; k0 += NB) {
+                    load(ch, h, k0);
+                    store(h, k0);
+                }
+        }
+        __syncthreads();
+        if (AHEAD && ch + 1 < chunks) load(ch + 1, 0, 0);
+        constexpr int UNROLL = DEEP ? F : 1;
+#pragma unroll UNROLL
+        for (int k = 0; k < (Z::UP ? kOdd : F); k++) column(ch, k, std::integral_constant<int, 0>());
+        if constexpr (Z::UP)
+#pragma unroll 1
+            for (int k = kOdd; k < F; k++) column(ch, k, std::integral_constant<int, 1>());
+    }
+
+    // Lane (half, l32), register v of an accumulator: output plane m0 + 8 (v / 4) + 4 half + v % 4, pixel l32
+    // of the row.
+    const int orow0 = tr * Z::TH + row0, ocol0 = tc * 32 + l32;
+    auto out_row = [&](int q) __attribute__((always_inline)) { return NP * (orow0 + q % RW) + (Z::UP ? q / RW ^ Z::P : 0); };
+    auto out_col = [&](int q) __attribute__((always_inline)) {
+        return NP * ocol0 + (Z::UP ? q / RW ^ pair ^ Z::P : 0);
+    };
     // Two kinds of outputs are computed again below, by plain FP32 multiply-adds:
     // non-finite ones (an infinite or NaN operand, or one that rounds to infinity,
-    // reaches them as inf * 0 or inf - inf of its terms), and those below
-    // FR_TINY, where the low terms of operands run out of BF16's exponents.
+    // reaches them as inf * 0 or inf - inf of its terms), and those so small that
+    // products or terms under BF16's and FP32's normal range may matter to
+    // them: each of the n products of a pair of operands loses at most 2^-123,
+    // and where the tile (the bank) holds operands under FR_SMALL, whose
+    // last term may be lost, 2^-125 of the bank's (the tile's) largest.
+    float tiny = 0x1p-100f * (float)(chunks * FR_RC * F * F);
+    if (EXACT) {
+        constexpr unsigned FINITE = 0x7f7fffffu;
+        float bound = 1.f;
+        if (sRange[0]) {
+            unsigned wMost = 0u;
+            for (int i = lane; i < chunks * F * F; i += 64) wMost = max(wMost, range[i].x);
+            bound += __uint_as_float(min(wave_max(wMost), FINITE));
+        }
+        if (__any(smallW)) {  // the same in every wave
+            most = wave_max(most);
+            if (lane == 0) atomicMax(&sRange[1], most);
+            __syncthreads();
+            bound += __uint_as_float(min(sRange[1], FINITE));
+        }
+        tiny *= bound;
+    }
     float z = 0.f;
     bool redo = false;
+    if (EXACT) {
 #pragma unroll
-    for (int r = 0; r < RW; r++)
+        for (int r = 0; r < NA; r++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            acc[r][v] += low[r][v];
-            z = fmaf(acc[r][v], 0.f, z);
-            redo |= fabsf(acc[r][v]) < FR_TINY && acc[r][v] != 0.f;
-        }
-    const int pc = min(ocol, g.OW - 1);
+            for (int v = 0; v < 16; v++) {
+                acc[r][v] += low[EXACT ? r : 0][v];
+                z = fmaf(acc[r][v], 0.f, z);
+                redo |= fabsf(acc[r][v]) < tiny && acc[r][v] != 0.f;
+            }
+    }
     if (e.n || __any(redo || z != z)) {  // wave-uniform
         // Eight planes of a row at a time in a runtime loop (16 spill registers at
         // three waves a SIMD).
 #pragma unroll 1
-        for (int t = 0; t < 2 * RW; t++) {
+        for (int t = 0; t < 2 * NA; t++) {
             float v[8];
             int pl[8], pt[8];
-            const int r = t >> 1, mo0 = 16 * (t & 1) + 4 * half;  // plane of v[k]: mo0 + 8 (k / 4) + k % 4
-            const int prow = min(orow0 + r, g.OH - 1);
+            const int mo0 = 16 * (t & 1) + 4 * half;  // plane of v[k]: mo0 + 8 (k / 4) + k % 4
+            const int orow = out_row(t >> 1), ocol = out_col(t >> 1);
+            const int prow = min(orow, g.OH - 1), pc = min(ocol, g.OW - 1);
 #pragma unroll
-            for (int q = 0; q < 2 * RW; q++) {
+            for (int q = 0; q < 2 * NA; q++) {
                 if (q != t) continue;  // wave-uniform: the accumulators keep compile-time indexes
 #pragma unroll
                 for (int k = 0; k < 8; k++) v[k] = acc[q >> 1][8 * (q & 1) + k];
@@ -314,11 +545,11 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
             for (int k = 0; k < 8; k++) {
                 const int mm = m0 + mo0 + 8 * (k >> 2) + (k & 3);
                 const float a = fabsf(v[k]);
-                if (mm < Mout && (!(a < __builtin_inff()) || (a < FR_TINY && v[k] != 0.f))) again |= 1u << k;
+                if (EXACT && mm < Mout && (!(a < __builtin_inff()) || (a < tiny && v[k] != 0.f))) again |= 1u << k;
                 pl[k] = b * Mout + min(mm, Mout - 1);
                 pt[k] = prow * g.OW + pc;
             }
-            if (orow0 + r >= g.OH || ocol >= g.OW) again = 0;
+            if (orow >= g.OH || ocol >= g.OW) again = 0;
             while (again) {
                 const int k = __builtin_ctz(again);
                 again &= again - 1;
@@ -328,7 +559,7 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
             }
             if (e.n) epi_eval_n<8>(e, v, pl, pt);
 #pragma unroll
-            for (int q = 0; q < 2 * RW; q++) {
+            for (int q = 0; q < 2 * NA; q++) {
                 if (q != t) continue;
 #pragma unroll
                 for (int k = 0; k < 8; k++) acc[q >> 1][8 * (q & 1) + k] = v[k];
@@ -336,68 +567,98 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
         }
     }
     const __amdgpu_buffer_rsrc_t orr = buffer_rsrc(Ob + (size_t)m0 * OHW, (uint32_t)min(32, Mout - m0) * OHW * 4u);
+    // Streamed, but for an up-sampled output: the waves of a pair write every other column.
+    constexpr int CACHE = Z::UP ? 0 : LOAD_NT;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
         const int mo = 8 * (v >> 2) + (v & 3);
-        const bool ok = m0 + mo + 4 * half < Mout && ocol < g.OW;
+        const bool ok = m0 + mo + 4 * half < Mout;
 #pragma unroll
-        for (int r = 0; r < RW; r++) {
-            const int vo = ok && orow0 + r < g.OH ? (4 * half * OHW + (orow0 + r) * g.OW + ocol) * 4 : STAGE_OOB;
-            const float sum = acc[r][v];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), orr, vo, mo * OHW * 4, LOAD_NT);
+        for (int q = 0; q < NA; q++) {
+            const int orow = out_row(q), ocol = out_col(q);
+            const int vo = ok && orow < g.OH && ocol < g.OW ? (4 * half * OHW + orow * g.OW + ocol) * 4 : STAGE_OOB;
+            const float sum = acc[q][v];
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), orr, vo, mo * OHW * 4, CACHE);
         }
     }
 }
 
-bool frame_rows_supported(int F) { return F == 3 || F == 5 || F == 7 || F == 9; }
+// The configurations built: (filter, rows a wave, waves a SIMD, sampling, precision).
+#define FR_LP(X, P)                                                                                                 \
+    X(3, 1, 4, FR_UNIT, P) X(3, 2, 4, FR_UNIT, P) X(3, 4, 3, FR_UNIT, P) X(5, 1, 4, FR_UNIT, P) X(5, 2, 4, FR_UNIT, P) \
+    X(5, 4, 3, FR_UNIT, P) X(7, 1, 4, FR_UNIT, P) X(7, 2, 3, FR_UNIT, P) X(7, 4, 3, FR_UNIT, P)                      \
+    X(9, 1, 4, FR_UNIT, P) X(9, 2, 3, FR_UNIT, P) X(9, 4, 3, FR_UNIT, P)
+#define FR_UP(X, F, S) X(F, 1, F < 9 ? 3 : 2, S, COGCONV_FP32) X(F, 2, 2, S, COGCONV_FP32)
+#define FR_CASES(X)                                                                                                 \
+    X(3, 1, 3, FR_UNIT, COGCONV_FP32) X(5, 1, 3, FR_UNIT, COGCONV_FP32) X(7, 1, 2, FR_UNIT, COGCONV_FP32)           \
+    X(9, 1, 2, FR_UNIT, COGCONV_FP32) X(3, 2, 3, FR_UNIT, COGCONV_FP32) X(5, 2, 2, FR_UNIT, COGCONV_FP32)           \
+    X(7, 2, 2, FR_UNIT, COGCONV_FP32) X(9, 2, 2, FR_UNIT, COGCONV_FP32) X(9, 8, 1, FR_UNIT, COGCONV_FP32)           \
+    FR_UP(X, 3, FR_UP0) FR_UP(X, 3, FR_UP1) FR_UP(X, 5, FR_UP0) FR_UP(X, 7, FR_UP0) FR_UP(X, 7, FR_UP1)              \
+    FR_UP(X, 9, FR_UP0)                                                                                             \
+    X(3, 1, 2, FR_DOWN, COGCONV_FP32) X(5, 1, 2, FR_DOWN, COGCONV_FP32) X(7, 1, 2, FR_DOWN, COGCONV_FP32)           \
+    X(9, 1, 2, FR_DOWN, COGCONV_FP32)                                                                               \
+    X(3, 1, 3, FR_UNIT, COGCONV_SPLIT_BF16) X(3, 2, 3, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
+    X(3, 4, 2, FR_UNIT, COGCONV_SPLIT_BF16) X(5, 1, 3, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
+    X(5, 2, 3, FR_UNIT, COGCONV_SPLIT_BF16) X(5, 4, 2, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
+    FR_LP(X, COGCONV_BF16) FR_LP(X, COGCONV_FP16)
 
-size_t frame_rows_lds_bytes(int F, int RW) {
-    switch (F * 10 + RW) {
-    case 31: return FrameRows<3, 1>::LDS;
-    case 51: return FrameRows<5, 1>::LDS;
-    case 71: return FrameRows<7, 1>::LDS;
-    case 91: return FrameRows<9, 1>::LDS;
-    case 32: return FrameRows<3, 2>::LDS;
-    case 52: return FrameRows<5, 2>::LDS;
-    case 72: return FrameRows<7, 2>::LDS;
-    case 92: return FrameRows<9, 2>::LDS;
-    case 98: return FrameRows<9, 8>::LDS;
+// Where 16-byte staging loads pay (at four rows a wave their registers cost a block a CU).
+static constexpr bool fr_vec(int RW, int S, int prec) { return S == FR_UNIT && prec != COGCONV_FP32 && RW <= 2; }
+
+static constexpr int fr_key(int F, int RW, int S, int prec) { return ((prec * 4 + S) * 16 + F) * 16 + RW; }
+
+size_t frame_rows_lds_bytes(int F, int RW, int S, int prec) {
+    switch (fr_key(F, RW, S, prec)) {
+#define FR_LDS(F, RW, OCC, S, PREC) \
+    case fr_key(F, RW, S, PREC): return FrameRows<F, RW, S, fr_terms(PREC)>::LDS;
+        FR_CASES(FR_LDS)
+#undef FR_LDS
     default: return 0;
     }
 }
 
-size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F) {
-    return (size_t)c.mTiles * (c.RC / FR_RC) * F * F * 3 * 1024;
+size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F, int prec) {
+    return (size_t)c.mTiles * (c.RC / FR_RC) * F * F * (fr_terms(prec) * 1024 + sizeof(uint2));
 }
 
-hipError_t launch_frame_rows(const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x, const float* w,
-                             float* out, void* ws, hipStream_t s, const Epi& ep, const cogconv_image_io* tab) {
+hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
+                             const float* w, float* out, void* ws, hipStream_t s, int stage, const Epi& ep,
+                             const cogconv_image_io* tab, bool x16) {
     const long blocks = (long)c.tilesC * c.tilesR * c.mTiles * m.B;
     if (blocks <= 0 || blocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
-    __bf16* wp = static_cast<__bf16*>(ws);
-    const long total = (long)c.mTiles * (c.RC / FR_RC) * g.FH * g.FW * 64;
-    hipLaunchKernelGGL((k_pack_rows<3>), dim3((unsigned)std::min((total + 255) / 256, 4096L)), dim3(256), 0, s, g, m,
-                       c.Mout, c.RC / FR_RC, total, w, wp);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const dim3 grid((unsigned)blocks), block(256);
-#define FR_CASE(F, RW, OCC)                                                                                         \
-    case F * 10 + RW:                                                                                               \
-        hipLaunchKernelGGL((k_frame_rows<F, RW, OCC>), grid, block, c.lds_bytes, s, g, m, c, x, w, wp, out, tab, ep); \
+    if (prec == COGCONV_FP32 && stage != LP_PACK_AND_RUN) return hipErrorInvalidValue;  // the redo reads w itself
+    if (stage != LP_RUN_ONLY) {
+        const long total = (long)c.mTiles * (c.RC / FR_RC) * g.FH * g.FW * 64;
+        const dim3 grid((unsigned)std::min((total + 255) / 256, 4096L)), block(256);
+        switch (prec) {
+#define FR_PACK(PREC)                                                                                              \
+    case PREC:                                                                                                     \
+        hipLaunchKernelGGL((k_pack_rows<PREC, fr_terms(PREC)>), grid, block, 0, s, g, m, c.Mout, c.RC / FR_RC, total, w, \
+                           static_cast<LpType<PREC>::T*>(ws));                                                     \
         break;
-    switch (g.FH * 10 + c.MB) {
-        FR_CASE(3, 1, 3)
-        FR_CASE(5, 1, 3)
-        FR_CASE(7, 1, 2)
-        FR_CASE(9, 1, 2)
-        FR_CASE(3, 2, 3)
-        FR_CASE(5, 2, 2)
-        FR_CASE(7, 2, 2)
-        FR_CASE(9, 2, 2)
-        FR_CASE(9, 8, 1)
+            FR_PACK(COGCONV_FP32)
+            FR_PACK(COGCONV_BF16)
+            FR_PACK(COGCONV_FP16)
+            FR_PACK(COGCONV_SPLIT_BF16)
+#undef FR_PACK
+        default: return hipErrorInvalidValue;
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || stage == LP_PACK_ONLY) return e;
+    }
+    const dim3 grid((unsigned)blocks), block(256);
+    const bool vec = c.vec4 && (tab ? x16 : (reinterpret_cast<uintptr_t>(x) & 15) == 0);
+    switch (fr_key(g.FH, c.MB, c.variant, prec)) {
+#define FR_LAUNCH(F, RW, OCC, S, PREC)                                                                             \
+    case fr_key(F, RW, S, PREC):                                                                                   \
+        hipLaunchKernelGGL((vec ? k_frame_rows<F, RW, OCC, S, PREC, fr_vec(RW, S, PREC)>                           \
+                                : k_frame_rows<F, RW, OCC, S, PREC, false>),                                       \
+                           grid, block, c.lds_bytes, s, g, m, c, x, w, static_cast<const LpType<PREC>::T*>(ws), out, tab, ep); \
+        break;
+        FR_CASES(FR_LAUNCH)
+#undef FR_LAUNCH
     default: return hipErrorInvalidValue;
     }
-#undef FR_CASE
     return hipGetLastError();
 }
 

@@ -313,14 +313,16 @@ hipError_t launch_up2q_lp(int precision, const Geom& g, const PlaneMap& m, const
 hipError_t launch_igemm_lp(int precision, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
                            const float* w, float* out, void* ws, hipStream_t s, int stage = LP_PACK_AND_RUN,
                            const Epi& e = kNoEpi, const cogconv_image_io* tab = nullptr, bool x16 = false);
-// FP32 frame modes as split-BF16 products (frame_rows.hip): c.MB holds the
-// output rows of a wave, c.RC the planes padded to whole 16-plane chunks.
-bool frame_rows_supported(int F);
-size_t frame_rows_lds_bytes(int F, int RW);
-size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F);
-hipError_t launch_frame_rows(const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x, const float* w,
-                             float* out, void* ws, hipStream_t s, const Epi& e = kNoEpi,
-                             const cogconv_image_io* tab = nullptr);
+// FP32 frame modes as split-BF16 products, and the split-BF16 ones (frame_rows.hip):
+// c.variant is the sampling, c.MB holds the output rows of a wave, c.RC the
+// planes padded to whole 16-plane chunks.  `stage` as in launch_igemm_lp
+// (the FP32 form packs on every launch).
+enum FrameRowsSampling { FR_UNIT = 0, FR_UP0 = 1, FR_UP1 = 2, FR_DOWN = 3 };
+size_t frame_rows_lds_bytes(int F, int RW, int sampling, int precision);  // 0: not built
+size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F, int precision);
+hipError_t launch_frame_rows(int precision, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
+                             const float* w, float* out, void* ws, hipStream_t s, int stage = LP_PACK_AND_RUN,
+                             const Epi& e = kNoEpi, const cogconv_image_io* tab = nullptr, bool x16 = false);
 hipError_t launch_block_reduce_sum(const float* in, float* out, int64_t points, int out_planes, int factor,
                                    hipStream_t s, const Epi& e = kNoEpi);
 // out = epilogue(in) over `planes` planes of `points` (the unmerged elementwise pass).

@@ -18,6 +18,11 @@ struct LpType<COGCONV_BF16> {
     typedef bf16x8 V;
 };
 template <>
+struct LpType<COGCONV_FP32> {  // as three BF16 terms
+    typedef __bf16 T;
+    typedef bf16x8 V;
+};
+template <>
 struct LpType<COGCONV_SPLIT_BF16> {
     typedef __bf16 T;
     typedef bf16x8 V;

@@ -565,55 +565,78 @@ bool choose_igemm_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, Ig
     return false;
 }
 
-// FP32 frame block-reduce modes as split-BF16 products (k_frame_rows): unit
-// steps, square filters; `rw` output rows a wave.
+// FP32 and split-BF16 frame block-reduce modes as split-BF16 products
+// (k_frame_rows): square filters, unit steps, 2x up-sampled input or every
+// second output; `rw` output rows a wave.
 bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw) {
     if (d->mode != COGCONV_PROJECT_FRAME_BLOCK_REDUCE_SUM && d->mode != COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM)
         return false;
-    if (d->precision != COGCONV_FP32 || d->in0.dims != 2 || g.FH != g.FW || !frame_rows_supported(g.FH) ||
-        g.upAr != 1 || g.upAc != 1 || g.dnR != 1 || g.dnC != 1)
-        return false;
+    if (d->in0.dims != 2 || g.FH != g.FW || g.hR != g.hC || g.upAr != g.upAc || g.dnR != g.dnC) return false;
+    int phases = 1;
     IgemmCfg c;
     std::memset(&c, 0, sizeof c);
-    c.lds_bytes = frame_rows_lds_bytes(g.FH, rw);
+    if (g.upAr == 1 && g.dnR == 1) {
+        c.variant = FR_UNIT;
+    } else if (false && g.upAr == 1 && g.dnR == 2) {
+        c.variant = FR_DOWN;
+    } else if (false && g.upAr == 2 && g.dnR == 1) {
+        c.variant = g.hR & 1 ? FR_UP1 : FR_UP0;
+        phases = 2;
+    } else {
+        return false;
+    }
+    c.lds_bytes = frame_rows_lds_bytes(g.FH, rw, c.variant, d->precision);
     if (c.lds_bytes == 0 || c.lds_bytes > 160 * 1024) return false;
     c.MB = rw;
     c.Mout = m.T / m.N;
     c.mTiles = (c.Mout + 31) / 32;
-    c.tilesR = (g.OH + 4 * rw - 1) / (4 * rw);
-    c.tilesC = (g.OW + 31) / 32;
+    const int th = 4 * rw / phases;  // rows (of a phase) of a block
+    c.tilesR = ((g.OH + phases - 1) / phases + th - 1) / th;
+    c.tilesC = ((g.OW + phases - 1) / phases + 31) / 32;
     c.RC = (m.R + 15) / 16 * 16;
+    c.vec4 = d->precision != COGCONV_FP32 && g.W % 4 == 0 && g.dnR == 1 && rw <= 2;  // 16-byte staging (of aligned fields)
     // 32-bit buffer offsets: an image with its planes padded to whole chunks,
     // and 32 output planes.
     if ((long)c.RC * g.H * g.W * 4 >= (1L << 31) || (long)32 * g.OH * g.OW * 4 >= (1L << 31)) return false;
-    // A packed bank within the no-allocation launch's scratch array, so that the
-    // plans it took keep running there.
-    if (frame_rows_workspace_bytes(c, g.FH) > (64UL << 20)) return false;
+    // FP32: a packed bank within the no-allocation launch's scratch array, so that
+    // the plans it took keep running there.
+    if (frame_rows_workspace_bytes(c, g.FH, d->precision) > (d->precision == COGCONV_FP32 ? 64UL << 20 : 1UL << 31))
+        return false;
     *out = c;
     return true;
 }
 
-// Estimated time (us, two launches) of the split-BF16 frame kernel, and of the
-// FP32 MFMA frame kernel (one launch) on the same op: a launch floor, plus the
-// longer of one block's serial time and the whole grid's time at full load.  A
-// chunk costs its staging and its MFMA cycles at 2.4 GHz.  The constants fit 557
-// measured calls (sides 24 to 256, 3 to 64 planes, 1 to 64 outputs, batches 1 to
-// 32, filters 3x3 to 9x9); choosing the faster estimate loses 2% against always
-// knowing the faster kernel, and gains 1.34x over the FP32 MFMA kernel alone.
-double frame_rows_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    const double blocks = (double)c.tilesR * c.tilesC * c.mTiles * m.B, chunks = c.RC / 16;
-    const double mfma = c.MB * g.FH * g.FW * 6 * 32 / 2400.0;  // one wave's, six products of 32 cycles a tap and row
-    const double serial = chunks * (2.0 + mfma);
-    const double load = blocks / 256 * chunks * (1.7 * mfma + 0.002 * (4 * c.MB + g.FH - 1) * (31 + g.FW));
-    return 7.9 + std::max(serial, load);
+// Estimated time (us) of one call: a launch floor, plus the longer of one block's
+// serial time and the whole grid's time at full load.  A chunk of planes costs its
+// staging and its MFMA time `mfma` (one wave's at 2.4 GHz); `px` staged pixels.
+struct CallTime {
+    double launch, chunk, mfma, block, mfmaLoad, pxLoad;
+    double us(double blocks, double chunks, double m, double px) const {
+        return launch + std::max(chunks * (chunk + mfma * m), blocks / 256 * (block + chunks * (mfmaLoad * m + pxLoad * px)));
+    }
+};
+
+// The constants fit calls measured on this card (sides 24 to 256, 3 to 64 planes, 1
+// to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log error 0.1 to 0.12 rms).
+// FP32 against the MFMA kernel, 200 calls: the faster estimate is 2% from always
+// knowing the faster kernel, the split form alone 15%, 1.15x the MFMA kernel.
+// Split-BF16 (250 calls) and BF16 / FP16 (400): 2% from the best rows a wave.
+double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
+    static const CallTime fit[] = {{8.7, 1.33, 1.36, 0.09, 1.58, 0.0021},   // FP32
+                                   {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // BF16
+                                   {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // FP16
+                                   {6.4, 1.23, 1.52, 0.43, 1.57, 0.0013}};  // split-BF16
+    const double products = d->precision == COGCONV_FP32 ? 6 : (d->precision == COGCONV_SPLIT_BF16 ? 3 : 1);
+    const double mfma = g.FH * g.FW * c.MB * products * 32 / 2400.0;  // 32 cycles each
+    return fit[d->precision].us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
+                                (4.0 * c.MB + g.FH - 1) * (31 + g.FW));
 }
 
 double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    const double blocks = (double)c.tilesR * c.tilesC * c.mTiles * m.B, chunks = (m.R + c.RC - 1) / c.RC;
+    static const CallTime fit = {4.3, 1.14, 2.45, 1.20, 2.52, 0.0050};
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
-    const double serial = chunks * (4.7 + mfma);
-    const double load = blocks / 256 * chunks * (2.7 * mfma + 0.0072 * c.RC / 16 * (7 + g.FH) * (31 + g.FW));
-    return 4.9 + std::max(serial, load);
+    return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
+                  c.RC / 16.0 * (7 + g.FH) * (31 + g.FW));
 }
 
 SmallCfg choose_small(const Geom& g, const PlaneMap& m, long blocks = 4096) {
@@ -846,7 +869,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         if (fc) v.f = *fc;
         switch (kind) {
         case KK_IGEMM_LP: v.workspace = igemm_lp_workspace_bytes(v.i, g.FH, desc->precision); break;
-        case KK_FRAME_ROWS: v.workspace = frame_rows_workspace_bytes(v.i, g.FH); break;
+        case KK_FRAME_ROWS: v.workspace = frame_rows_workspace_bytes(v.i, g.FH, desc->precision); break;
         case KK_FA_IGEMM:
         case KK_FA_IGEMM_LP: v.workspace = (size_t)v.f.splits * v.f.K * m.N * outPts * sizeof(float); break;
         case KK_SMALL_OUTPUT: v.workspace = (size_t)v.s.splits * m.nOut * outPts * sizeof(float); break;
@@ -935,6 +958,23 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         if (rows) return;
         IgemmCfg lp;
         if (!choose_igemm_lp(desc, g, m, &lp)) return;
+        // k_frame_rows wherever it is built (3x3 to 9x9, unit steps, its offsets in 31
+        // bits): faster than k_igemm_lp in 97% of 650 measured calls, 1.5x on average
+        // and at most 1.25x slower.  One kernel's configurations only, so that
+        // candidates agree bit for bit.
+        IgemmCfg fr[3];
+        bool frOk[3];
+        int first = -1;
+        for (int i = 0; i < 3; i++) {
+            frOk[i] = choose_frame_rows(desc, g, m, &fr[i], 1 << i);
+            if (frOk[i] && (first < 0 || frame_rows_us(desc, g, m, fr[i]) < frame_rows_us(desc, g, m, fr[first]))) first = i;
+        }
+        if (first >= 0) {
+            add(KK_FRAME_ROWS, nullptr, nullptr, &fr[first], nullptr);
+            for (int i = 0; i < 3; i++)
+                if (frOk[i]) add(KK_FRAME_ROWS, nullptr, nullptr, &fr[i], nullptr);
+            return;
+        }
         add(KK_IGEMM_LP, nullptr, nullptr, &lp, nullptr);
         const int mbMax = lp.MB;
         for (int mb : {4, 2, 1}) {
@@ -975,10 +1015,11 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     for (int i = 0; i < 3; i++) {
         rows_ok[i] = choose_frame_rows(desc, g, m, &rows[i], i == 0 ? 1 : (i == 1 ? 2 : 8));
         if (!rows_ok[i]) continue;
-        if (rows_first < 0 || frame_rows_us(g, m, rows[i]) < frame_rows_us(g, m, rows[rows_first])) rows_first = i;
+        if (rows_first < 0 || frame_rows_us(desc, g, m, rows[i]) < frame_rows_us(desc, g, m, rows[rows_first]))
+            rows_first = i;
     }
     if (rows_first >= 0 && igemm_ok &&
-        frame_rows_us(g, m, rows[rows_first]) > 0.95 * igemm_frame_us(g, m, ig))
+        frame_rows_us(desc, g, m, rows[rows_first]) > 0.95 * igemm_frame_us(g, m, ig))
         rows_first = -1;
     PhaseSet up;
     const bool up_ok = choose_igemm_up(desc, g, m, &up);
@@ -1079,7 +1120,9 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
     if (e) return e;
     std::vector<Variant> vars;
     enumerate_variants(desc, g, m, vars);
-    const auto offered = [&](int i) { return !(serving && vars[i].kind == KK_FRAME_ROWS); };
+    const auto offered = [&](int i) {
+        return !(serving && vars[i].kind == KK_FRAME_ROWS && desc->precision == COGCONV_FP32);
+    };
     if (vars.empty())
         return fail(COGCONV_ERR_UNSUPPORTED,
                     "precision %d is offered for ProjectFrame/BackProjectFrame with block reduction on 2-D fields with "
@@ -1272,10 +1315,15 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
         break;
     }
     case KK_FRAME_ROWS:
-        snprintf(buf, len, "igemm_f32x3 %s out=%dx%dx%d tile=%dx32 rows=%d threads=256 lds=%zu",
-                 mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB, plan->icfg.MB,
+    {
+        static const char* const names[] = {"igemm_f32x3", "igemm_bf16x1", "igemm_fp16x1", "igemm_bf16x2"};
+        snprintf(buf, len, "%s%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=256%s lds=%zu",
+                 names[plan->desc.precision],
+                 g.upAr == 2 ? "_up2" : (g.dnR == 2 ? "_down2" : ""), mode_name(plan->desc.mode), plan->m.nOut, g.OH,
+                 g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, plan->icfg.vec4 ? " ld16" : "",
                  plan->icfg.lds_bytes);
         break;
+    }
     case KK_IGEMM_UP: {
         if (plan->ps.f.on) {
             static const char* pn[] = {"f32", "bf16", "fp16", "split_bf16"};
@@ -1331,26 +1379,46 @@ extern "C" int cogconv_plan_describe(cogconv_plan plan, char* buf, size_t len) {
     return COGCONV_OK;
 }
 
+namespace {
+
+// Plans whose launch packs operand 2 into the workspace and reads it only there.
+// (The FP32 split form also reads the filters as they are, where it computes an
+// output again.)
+bool packs_operand(const cogconv_plan_s* plan) {
+    return plan->kind == KK_IGEMM_LP || (plan->kind == KK_FRAME_ROWS && plan->desc.precision != COGCONV_FP32);
+}
+
+hipError_t launch_packing(const cogconv_plan_s* plan, const float* in0, const float* in1, float* out, void* workspace,
+                          hipStream_t s, LpStage stage) {
+    return plan->kind == KK_FRAME_ROWS ? launch_frame_rows(plan->desc.precision, plan->g, plan->m, plan->icfg, in0, in1,
+                                                           out, workspace, s, stage)
+                                       : launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, in0, in1,
+                                                         out, workspace, s, stage);
+}
+
+}  // namespace
+
 extern "C" int cogconv_plan_pack_operand(cogconv_plan plan, const float* in1, void* workspace, cogconv_stream stream,
                                          int32_t* packed) {
     clear_error();
     if (!plan || !packed) return fail(COGCONV_ERR_INVALID_ARG, "null argument");
     *packed = 0;
-    if (plan->kind != KK_IGEMM_LP) return COGCONV_OK;
+    if (!packs_operand(plan)) return COGCONV_OK;
     if (!in1 || !workspace) return fail(COGCONV_ERR_INVALID_ARG, "null operand or workspace");
-    const hipError_t e = launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, nullptr, in1, nullptr,
-                                         workspace, reinterpret_cast<hipStream_t>(stream), LP_PACK_ONLY);
+    const hipError_t e = launch_packing(plan, nullptr, in1, nullptr, workspace, reinterpret_cast<hipStream_t>(stream),
+                                        LP_PACK_ONLY);
     if (int st = check_hip(e, "operand pack")) return st;
     *packed = 1;
     return COGCONV_OK;
 }
 
 std::string cogconv_plan_pack_key(const cogconv_plan_s* plan) {
-    if (!plan || plan->kind != KK_IGEMM_LP) return std::string();
-    // What k_pack_filters_lp reads: precision, mode, orientation, taps, planes
-    // and the padded output / input-plane counts of the kernel configuration.
-    const int key[] = {plan->desc.precision, plan->m.mode, plan->g.flip, plan->g.FH, plan->g.FW, plan->m.N,
-                       plan->m.T, plan->m.R, plan->icfg.Mout, plan->icfg.mTiles * 16 * plan->icfg.MB, plan->icfg.RC};
+    if (!plan || !packs_operand(plan)) return std::string();
+    // What k_pack_filters_lp (k_pack_rows) reads: precision, mode, orientation, taps,
+    // planes and the padded output / input-plane counts of the kernel configuration.
+    const int key[] = {plan->kind, plan->desc.precision, plan->m.mode, plan->g.flip, plan->g.FH, plan->g.FW, plan->m.N,
+                       plan->m.T, plan->m.R, plan->icfg.Mout,
+                       plan->icfg.mTiles * (plan->kind == KK_FRAME_ROWS ? 32 : 16 * plan->icfg.MB), plan->icfg.RC};
     return std::string(reinterpret_cast<const char*>(key), sizeof key);
 }
 
@@ -1358,9 +1426,9 @@ extern "C" int cogconv_launch_packed(cogconv_plan plan, const float* in0, float*
                                      cogconv_stream stream) {
     clear_error();
     if (!plan || !in0 || !out || !workspace) return fail(COGCONV_ERR_INVALID_ARG, "null plan or buffer");
-    if (plan->kind != KK_IGEMM_LP) return fail(COGCONV_ERR_INVALID_ARG, "plan does not pack operand 2");
-    const hipError_t e = launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, in0, nullptr, out,
-                                         workspace, reinterpret_cast<hipStream_t>(stream), LP_RUN_ONLY);
+    if (!packs_operand(plan)) return fail(COGCONV_ERR_INVALID_ARG, "plan does not pack operand 2");
+    const hipError_t e = launch_packing(plan, in0, nullptr, out, workspace, reinterpret_cast<hipStream_t>(stream),
+                                        LP_RUN_ONLY);
     return check_hip(e, "convolution launch");
 }
 
@@ -1391,7 +1459,8 @@ int launch_all(cogconv_plan plan, const float* in0, const float* in1, float* out
                             LP_PACK_AND_RUN, ep);
         break;
     case KK_FRAME_ROWS:
-        e = launch_frame_rows(plan->g, plan->m, plan->icfg, in0, in1, out, workspace, s, ep);
+        e = launch_frame_rows(plan->desc.precision, plan->g, plan->m, plan->icfg, in0, in1, out, workspace, s,
+                              LP_PACK_AND_RUN, ep);
         break;
     case KK_IGEMM_UP:
         if (plan->ps.f.on && plan->desc.precision != COGCONV_FP32) {
@@ -1453,8 +1522,8 @@ int cogconv::launch_table(cogconv_plan plan, const cogconv_image_io* device_tabl
         e = launch_igemm_lp(plan->desc.precision, plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, workspace, s,
                             packed ? LP_RUN_ONLY : LP_PACK_AND_RUN, plan->epi, device_table, x16);
     else if (plan->kind == KK_FRAME_ROWS)
-        e = launch_frame_rows(plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, workspace, s, plan->epi,
-                              device_table);
+        e = launch_frame_rows(plan->desc.precision, plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, workspace, s,
+                              packed ? LP_RUN_ONLY : LP_PACK_AND_RUN, plan->epi, device_table, x16);
     else
         e = launch_igemm_f32(plan->g, plan->m, plan->icfg, nullptr, in1, nullptr, s, plan->epi, device_table);
     return check_hip(e, "table launch");
@@ -1474,7 +1543,7 @@ extern "C" int cogconv_launch_table(cogconv_plan plan, const cogconv_image_io* h
     if (!plan || !host_table || !device_table) return fail(COGCONV_ERR_INVALID_ARG, "null plan or table");
     if (!plan_table_capable(plan))
         return fail(COGCONV_ERR_UNSUPPORTED, "table launches are offered for the MFMA frame plans (no up-sampling)");
-    if (packed && plan->kind != KK_IGEMM_LP) return fail(COGCONV_ERR_INVALID_ARG, "plan does not pack operand 2");
+    if (packed && !packs_operand(plan)) return fail(COGCONV_ERR_INVALID_ARG, "plan does not pack operand 2");
     if (!packed && !in1) return fail(COGCONV_ERR_INVALID_ARG, "null operand 2");
     if ((plan->workspace || packed) && !workspace)
         return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);

@@ -1,6 +1,7 @@
-"""The split-BF16 form of the FP32 frame modes (igemm_f32x3 plans): parity with
-the FP64 oracle at the edges of its tiles, every candidate bit for bit alike,
-operands outside the split's range, unaligned buffers and request tables."""
+"""The row-walking frame kernel: the split-BF16 form of the FP32 frame modes
+(igemm_f32x3 plans) and its BF16, FP16 and split-BF16 forms.  Parity with the FP64
+oracle at the edges of its tiles, every candidate bit for bit alike, operands
+outside the split's range, unaligned buffers and request tables."""
 import numpy as np
 import pytest
 
@@ -87,6 +88,78 @@ def test_magnitudes_beyond_the_split(scale):
         # all terms positive: the oracle's magnitude sum is the result itself
         assert np.abs(launch(p, a, k) - ref).max() <= 1e-5 * ref.max()
         assert np.all(np.abs(launch(p, a, k) - ref) <= 1e-5 * mag)
+
+
+@pytest.mark.parametrize("xs,ws", [(1e-36, 1e8), (1e10, 1e-37), (1e-33, 1e30)])
+def test_small_operands_with_large_ones(xs, ws):
+    """One operand too small for its low BF16 terms, the other large enough that
+    the results are not small: still FP32 accuracy."""
+    rng = np.random.default_rng(8)
+    a = (rng.uniform(0.5, 1, (18, 20, 40)) * xs).astype(np.float32)
+    k = (rng.uniform(0.5, 1, (34 * 18, 5, 5)) * ws).astype(np.float32)
+    od, cd = desc_pair(O.PF_BRS, O.CLAMP, O.XCORR, O.NONE, 1, 1, a.shape, k.shape)
+    rows, _ = candidates(cd)
+    ref, mag = oracle_ref(od, a, k)
+    for p in rows:
+        print("CASE small and large", xs, ws, p.description, flush=True)
+        assert np.all(np.abs(launch(p, a, k) - ref) <= 1e-5 * mag)
+
+
+def rounded(a, precision):
+    if precision == L.FP16:
+        return a.astype(np.float16).astype(np.float32)
+    bits = a.view(np.uint32).astype(np.uint64)
+    return ((bits + 0x7FFF + ((bits >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("precision", (L.BF16, L.FP16, L.SPLIT_BF16))
+@pytest.mark.parametrize("mode,border,B,N,K,H,W,F", [
+    (O.PF_BRS, O.CLAMP, 1, 3, 2, 5, 4, 3),       # one column group a row, clamped on both sides
+    (O.BPF_BRS, O.CLAMP, 2, 17, 33, 9, 36, 5),   # a group past the tile, one plane and output past their blocks
+    (O.PF_BRS, O.CYCLIC, 1, 40, 9, 17, 8, 9),    # wrapped by more than a group on both sides
+    (O.PF_BRS, O.ZERO, 2, 16, 32, 16, 64, 7),    # whole tiles
+    (O.BPF_BRS, O.FULL, 1, 33, 5, 7, 28, 9),
+    (O.PF_BRS, O.VALID, 3, 8, 20, 18, 44, 3),
+    (O.PF_BRS, O.ZERO, 1, 20, 12, 8, 33, 3),     # rows of an odd width: no 16-byte loads
+    (O.BPF_BRS, O.CYCLIC, 1, 50, 7, 5, 6, 7),    # the filter larger than the field
+])
+def test_low_precision_every_candidate(precision, mode, border, B, N, K, H, W, F):
+    """BF16 and FP16: FP32 summation error only, against the oracle on the rounded
+    operands.  Split-BF16 drops the product of the low terms, 2^-16 of a product
+    at most.  Aligned and unaligned fields give the same bits (16-byte and 4-byte
+    staging), and so does the packed launch."""
+    if precision == L.SPLIT_BF16 and F > 5:
+        return
+    rng = np.random.default_rng(F * 1000 + H * 10 + precision)
+    a = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    k = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    orient = O.CONV if mode == O.BPF_BRS else O.XCORR
+    od, cd = desc_pair(mode, border, orient, O.NONE, 1, B, a.shape, k.shape, precision=precision)
+    if precision == L.SPLIT_BF16:
+        ref, mag = oracle_ref(od, a, k)
+        tol = 2.0 ** -16 + 2e-6
+    else:
+        ref, mag = oracle_ref(od, rounded(a, precision), rounded(k, precision))
+        tol = 2e-6
+    first = None
+    for v in range(L.variant_count(cd)):
+        p = L.Plan(cd, v)
+        print("CASE low precision", mode, border, p.description, flush=True)
+        assert "x1" in p.description or "x2" in p.description
+        for off in (0, 1):
+            got = launch(p, a, k, off=off)
+            assert np.all(np.abs(got - ref) <= tol * mag), (p.description, off)
+            first = got if first is None else first
+            assert np.array_equal(got, first), (p.description, off)
+        ba, bk, ws = L.DeviceBuffer.from_array(a), L.DeviceBuffer.from_array(k), L.DeviceBuffer(p.workspace_bytes)
+        bo = L.DeviceBuffer(4 * int(np.prod(p.out_shape)))
+        assert p.pack_operand(bk, ws)
+        p.launch_packed(ba, bo, ws)
+        L.synchronize()
+        assert np.array_equal(bo.download(p.out_shape), first)
+        for x in (ba, bk, ws, bo):
+            x.close()
+        p.close()
 
 
 def test_non_finite_operands():
