@@ -36,7 +36,8 @@
 //
 // Measured against the kernels it replaced (us a call): FP32 9x9, 32 -> 32 planes,
 // 8 images 256x256: 730 -> 331; split-BF16 3x3, 64 -> 64 planes, 32 images 128x128:
-// 170 -> 122; BF16 and FP16 3x3 to 9x9 over 400 random calls (3 to 64 planes, 24 to
+// 170 -> 122; FP32 2x up-sampled 7x7, 32 -> 32 planes, 8 images 256x256: 485 -> 262 (its
+// bound now: 126 of matrix cores at their peak, 55 of output stores); BF16 and FP16 3x3 to 9x9 over 400 random calls (3 to 64 planes, 24 to
 // 256 a side): 1.5x.  What bounds it: the matrix cores at FP32 (70% of their peak
 // at 9x9); for one term the latency of staging and of the filter stream.
 #include <algorithm>

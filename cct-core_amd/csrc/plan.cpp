@@ -579,7 +579,7 @@ bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
         c.variant = FR_UNIT;
     } else if (false && g.upAr == 1 && g.dnR == 2) {
         c.variant = FR_DOWN;
-    } else if (false && g.upAr == 2 && g.dnR == 1) {
+    } else if (g.upAr == 2 && g.dnR == 1) {
         c.variant = g.hR & 1 ? FR_UP1 : FR_UP0;
         phases = 2;
     } else {
@@ -621,13 +621,19 @@ struct CallTime {
 // FP32 against the MFMA kernel, 200 calls: the faster estimate is 2% from always
 // knowing the faster kernel, the split form alone 15%, 1.15x the MFMA kernel.
 // Split-BF16 (250 calls) and BF16 / FP16 (400): 2% from the best rows a wave.
+// 2x up-sampled (300 calls, estimates within 10%): 4% from the faster kernel, 1.21x
+// the FP32 MFMA one.
 double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
     static const CallTime fit[] = {{8.7, 1.33, 1.36, 0.09, 1.58, 0.0021},   // FP32
                                    {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // BF16
                                    {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // FP16
                                    {6.4, 1.23, 1.52, 0.43, 1.57, 0.0013}};  // split-BF16
+    static const CallTime up = {8.6, 0.90, 1.69, 1.00, 1.41, 0.0045};
     const double products = d->precision == COGCONV_FP32 ? 6 : (d->precision == COGCONV_SPLIT_BF16 ? 3 : 1);
     const double mfma = g.FH * g.FW * c.MB * products * 32 / 2400.0;  // 32 cycles each
+    if (g.upAr == 2)  // half the taps a wave, half the waves' rows a block
+        return up.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma / 2,
+                     (2.0 * c.MB + (g.FH - 1) / 2) * (32 + (g.FW - 1) / 2));
     return fit[d->precision].us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
                                 (4.0 * c.MB + g.FH - 1) * (31 + g.FW));
 }
@@ -637,6 +643,13 @@ double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
     return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
                   c.RC / 16.0 * (7 + g.FH) * (31 + g.FW));
+}
+
+double up2q_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
+    static const CallTime fit = {4.8, 1.25, 2.75, 2.78, 3.04, 0.0022};
+    const double mfma = c.MB * g.FH * g.FW / 2.0 * (c.RC / 4) * 4 * 32 / 2400.0;
+    return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
+                  c.RC / 16.0 * c.tileRows * c.tileCols);
 }
 
 SmallCfg choose_small(const Geom& g, const PlaneMap& m, long blocks = 4096) {
@@ -1030,17 +1043,20 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     // the autotuner times both routes.
     const bool fft_first = fft_ok && !rt_ok && (long)g.FH * g.FW >= 31L * 31;
     // Heuristic default.
-    // The fused up-sampled launch first: all four phases from one staged window,
+    // Up-sampled: the fused FP32 MFMA launch where the split form is not estimated
+    // faster by more than the estimates' error: all four phases from one staged window,
     // one output block and two blocks a CU (2x 7x7, 32 -> 32 planes of 256 x 256:
     // 0.49 ms, against 0.54 ms for two output blocks at one block a CU and
     // 0.74 ms for the four phase launches).
     PhaseSet upq = up;
     const bool upq_ok = up_ok && (choose_igemm_up2q(g, m, up, &upq.f, 1, 0, 80 * 1024, true) ||
                                   choose_igemm_up2q(g, m, up, &upq.f));
+    if (rows_first >= 0 && upq_ok && frame_rows_us(desc, g, m, rows[rows_first]) > 0.9 * up2q_us(g, m, upq.f.c))
+        rows_first = -1;
     if (fft_first) add_fft(fc);
+    else if (rows_first >= 0) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[rows_first], nullptr);
     else if (upq_ok) add_up(upq);
     else if (up_ok) add_up(up);
-    else if (rows_first >= 0) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[rows_first], nullptr);
     else if (igemm_ok) add(KK_IGEMM, nullptr, nullptr, &ig, nullptr);
     else if (fa_ok) add(KK_FA_IGEMM, nullptr, nullptr, nullptr, &fa);
     else if (small_out) add(KK_SMALL_OUTPUT, nullptr, &sm, nullptr, nullptr);
@@ -1317,10 +1333,9 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
     case KK_FRAME_ROWS:
     {
         static const char* const names[] = {"igemm_f32x3", "igemm_bf16x1", "igemm_fp16x1", "igemm_bf16x2"};
-        snprintf(buf, len, "%s%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=256%s lds=%zu",
-                 names[plan->desc.precision],
-                 g.upAr == 2 ? "_up2" : (g.dnR == 2 ? "_down2" : ""), mode_name(plan->desc.mode), plan->m.nOut, g.OH,
-                 g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, plan->icfg.vec4 ? " ld16" : "",
+        const char* name = g.upAr == 2 ? "igemm_f32_up2x3" : names[plan->desc.precision];
+        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=256%s lds=%zu",
+                 name, mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, plan->icfg.vec4 ? " ld16" : "",
                  plan->icfg.lds_bytes);
         break;
     }

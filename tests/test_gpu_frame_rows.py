@@ -74,6 +74,49 @@ def test_every_candidate(mode, border, B, N, K, H, W, F):
         p.close()
 
 
+@pytest.mark.parametrize("border,B,N,K,H,W,F,orient", [
+    (O.ZERO, 1, 1, 1, 2, 3, 3, O.XCORR),        # one sample of some phases
+    (O.CYCLIC, 2, 16, 32, 8, 32, 3, O.CONV),    # whole tiles at every row count
+    (O.FULL, 1, 17, 33, 9, 33, 5, O.XCORR),     # odd output sizes, one row, column, plane, output past the tiles
+    (O.VALID, 1, 7, 5, 12, 40, 5, O.XCORR),
+    (O.ZERO, 2, 20, 9, 7, 31, 7, O.XCORR),      # odd halo
+    (O.FULL, 1, 33, 40, 5, 18, 7, O.CONV),      # even halo
+    (O.CYCLIC, 1, 5, 3, 3, 4, 9, O.XCORR),      # the filter larger than the stored field
+    (O.VALID, 1, 18, 20, 17, 35, 9, O.XCORR),
+])
+def test_upsampled_every_candidate(border, B, N, K, H, W, F, orient):
+    """2x up-sampled input (igemm_f32_up2x3): parity, every candidate alike, an
+    epilogue applied as afterwards, and non-finite samples reaching exactly the
+    outputs they reach in the FP32 MFMA kernel (no inserted zero multiplies them)."""
+    rng = np.random.default_rng(F * 100 + H + W)
+    mode = O.BPF_BRS if orient == O.CONV else O.PF_BRS
+    a = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    k = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    od, cd = desc_pair(mode, border, orient, O.UP, 2, B, a.shape, k.shape)
+    plans = [L.Plan(cd, v) for v in range(L.variant_count(cd))]
+    rows = [p for p in plans if p.description.startswith("igemm_f32_up2x3")]
+    mfma = [p for p in plans if "fused" in p.description]
+    assert len(rows) == 2
+    ref, mag = oracle_ref(od, a, k)
+    b = a.copy()
+    b[0, H // 2, W // 2], b[N - 1, 0, W - 1] = np.inf, np.nan
+    first = None
+    for i, p in enumerate(rows):
+        print("CASE up rows", border, p.description, flush=True)
+        got = launch(p, a, k, off=i)
+        assert_parity(got, ref, mag, what=p.description)
+        first = got if first is None else first
+        assert np.array_equal(got, first), p.description
+        if mfma:
+            want = launch(mfma[0], b, k)
+            bad = launch(p, b, k)
+            assert np.array_equal(np.isnan(bad), np.isnan(want)) and np.array_equal(np.isinf(bad), np.isinf(want))
+        p.set_epilogue(L.make_epilogue([(L.EPI_MUL_CONST, 3.0, 0), (L.EPI_MAX_CONST, 0.5, 0)]))
+        assert np.array_equal(launch(p, a, k), np.maximum(got * np.float32(3.0), np.float32(0.5)))
+    for p in plans:
+        p.close()
+
+
 @pytest.mark.parametrize("scale", (1e-36, 1e-30, 1e30))
 def test_magnitudes_beyond_the_split(scale):
     """Operands whose low BF16 terms underflow, and large ones: as exact as near 1."""
