@@ -55,6 +55,11 @@ constexpr int FR_RC = 16;  // planes of a staged chunk (one MFMA k slice)
 // Operands below this may lose bits of their last BF16 term (under 2^-126).
 constexpr float FR_SMALL = 0x1p-102f;
 
+// Whether every 32-pixel run of an output tile is a whole 128-byte line.
+__host__ __device__ __forceinline__ bool stream_rows(int OW, const float* out) {
+    return (OW & 31) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0;
+}
+
 // BF16 terms of an operand.
 constexpr int fr_terms(int prec) { return prec == COGCONV_FP32 ? 3 : (prec == COGCONV_SPLIT_BF16 ? 2 : 1); }
 
@@ -202,8 +207,11 @@ __device__ __forceinline__ float frame_point(const Geom& g, const PlaneMap& m, c
     return s;
 }
 
-template <int F, int RW, int OCC, int S, int PREC, bool VEC>
-__global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, IgemmCfg c, const float* __restrict__ X,
+// VEC: 16-byte staging loads.  STORES: 0 picks the stores' cache policy at run time;
+// at four rows a wave, where the two forms side by side spill, 1 is the cached
+// and 2 the streamed one.
+template <int F, int RW, int MW, int OCC, int S, int PREC, bool VEC, int STORES>
+__global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m, IgemmCfg c, const float* __restrict__ X,
                                                          const float* __restrict__ Wt,
                                                          const typename LpType<PREC>::T* __restrict__ Wp,
                                                          float* __restrict__ O,
@@ -219,38 +227,42 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
 
     // Output-plane blocks of one tile are adjacent block indices (same XCD).
     int bid = xcd_swizzle(blockIdx.x, gridDim.x);
-    const int mt = bid % c.mTiles;
-    bid /= c.mTiles;
+    const int mGroups = (c.mTiles + MW - 1) / MW;
+    const int mg = bid % mGroups * MW;
+    bid /= mGroups;
     const int tc = bid % c.tilesC;
     bid /= c.tilesC;
     const int tr = bid % c.tilesR;
     const int b = bid / c.tilesR;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    // A wave's output block; one past the last works on the last and stores nothing.
+    const int mOwn = mg + (MW > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0), mt = min(mOwn, c.mTiles - 1);
     const int half = lane >> 5, l32 = lane & 31;
     const int pair = wave & 1;  // FR_UP
     const int row0 = (Z::UP ? wave >> 1 : wave) * RW;
     const int Mout = c.Mout, m0 = mt * 32;
+    constexpr int NTH = 256 * MW;
     const int HW = g.H * g.W, OHW = g.OH * g.OW;
     const float* Xb = tab ? tab[b].in0 : X + (size_t)b * m.N * HW;
     float* Ob = tab ? tab[b].out : O + (size_t)b * Mout * OHW;
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(Xb, (uint32_t)m.N * HW * 4u);  // the plan bounds this by 2^31
 
-    // Staging units of this thread, numbers tid, tid + 256, ...: a pixel (all 16
+    // Staging units of this thread, numbers tid, tid + 256 MW, ...: a pixel (all 16
     // planes of a chunk), or (VEC) 8 planes of an aligned group of 4 columns, which
     // a row of W % 4 == 0 columns holds or leaves out as a whole.  Byte offsets
     // within a plane with the border applied, or out of range (reads 0).
-    constexpr int NS = VEC ? (2 * Z::NG * Z::TR + 255) / 256 : (NPIX + 255) / 256;
+    constexpr int NS = VEC ? (2 * Z::NG * Z::TR + NTH - 1) / NTH : (NPIX + NTH - 1) / NTH;
     // The next chunk's loads run under this one's MFMAs where registers allow.
-    constexpr bool AHEAD = NS <= (VEC ? 1 : S == FR_DOWN ? 3 : 2);
+    constexpr bool AHEAD = NS <= (VEC ? 1 : S == FR_DOWN ? 3 : 2) && !(MW == 2 && RW == 4 && T == 1);
     const int y0 = tr * Z::TH * Z::STEP - (Z::UP ? g.hR >> 1 : g.hR);
     const int x0 = tc * 32 * Z::STEP - (Z::UP ? g.hC >> 1 : g.hC);
     int pOff[NS];
     int pix[VEC ? NS : 1];          // VEC: 4 * (half * T * NPIX + pixel of the group's first column) + clamp
 #pragma unroll
     for (int k = 0; k < NS; k++) {
-        const int u = tid + 256 * k;
+        const int u = tid + NTH * k;
         int ty, x;
         bool live;
         if constexpr (VEC) {
@@ -314,7 +326,7 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
     };
     // Filters held: a tap column, loaded one ahead, or all F of a chunk (DEEP, where
     // they fit registers), loaded a chunk ahead.
-    constexpr bool DEEP = S == FR_UNIT && F == 3 && T == 1;
+    constexpr bool DEEP = S == FR_UNIT && F == 3 && T == 1 && MW * RW < 8;
     V a[DEEP ? F : 1][NT][T];
     auto fragment = [&](int at, int i, int t) __attribute__((always_inline)) {
         return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(wr, at, (NP * i * T + t) * FRAG, 0));
@@ -377,7 +389,7 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
     // A chunk is staged in batches of loads: every plane of the thread's units (one
     // memory round trip) where they are loaded ahead, otherwise (VEC) a unit at a
     // time, or a half of the planes of at most 8 pixels.
-    constexpr int NB = AHEAD ? NS : VEC ? 1 : NS <= 8 ? NS : 4, HB = AHEAD && !VEC ? 2 : 1;
+    constexpr int NB = AHEAD ? NS : VEC ? 1 : NS <= 8 ? NS : 4, HB = !VEC && NS <= (S == FR_DOWN ? 3 : 2) ? 2 : 1;
     float v[NB][VEC ? 1 : 8 * HB];
     floatx4 v4[NB][VEC ? 8 : 1];
     auto load = [&](int ch, int h0, int k0) __attribute__((always_inline)) {
@@ -385,7 +397,7 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
         for (int k = 0; k < NB; k++) {
             if (k0 + k >= NS) continue;
             if constexpr (VEC) {
-                const int r8 = ch * FR_RC + 8 * (tid + 256 * (k0 + k) >= Z::NG * Z::TR);
+                const int r8 = ch * FR_RC + 8 * (tid + NTH * (k0 + k) >= Z::NG * Z::TR);
 #pragma unroll
                 for (int q = 0; q < 8; q++) {
                     // The plane is per lane (the two halves meet in a wave): plane, then a scalar one.
@@ -426,7 +438,7 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
         };
 #pragma unroll
         for (int k = 0; k < NB; k++) {
-            const int u = tid + 256 * (k0 + k);
+            const int u = tid + NTH * (k0 + k);
             if (k0 + k >= NS) continue;
             if constexpr (VEC) {
                 if (u >= 2 * Z::NG * Z::TR) continue;
@@ -568,50 +580,65 @@ __global__ __launch_bounds__(256, OCC) void k_frame_rows(Geom g, PlaneMap m, Ige
         }
     }
     const __amdgpu_buffer_rsrc_t orr = buffer_rsrc(Ob + (size_t)m0 * OHW, (uint32_t)min(32, Mout - m0) * OHW * 4u);
-    // Streamed, but for an up-sampled output: the waves of a pair write every other column.
-    constexpr int CACHE = Z::UP ? 0 : LOAD_NT;
+    // Streamed (non-temporal) where a row of 32 pixels is a whole 128-byte line, so
+    // that the output does not push the input out of L2; through the caches where
+    // lines are shared by two tiles, or by the two waves of an up-sampled pair.
+    // (BF16 3x3, 64 -> 64 planes, 32 images: 128x128 100 us streamed, 102 cached, and with
+    // 32 input planes 46 and 75; 136x136 135 and 122.)
+    auto put = [&](auto POLICY) __attribute__((always_inline)) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int mo = 8 * (v >> 2) + (v & 3);
-        const bool ok = m0 + mo + 4 * half < Mout;
+        for (int v = 0; v < 16; v++) {
+            const int mo = 8 * (v >> 2) + (v & 3);
+            const bool ok = m0 + mo + 4 * half < Mout && mOwn == mt;
 #pragma unroll
-        for (int q = 0; q < NA; q++) {
-            const int orow = out_row(q), ocol = out_col(q);
-            const int vo = ok && orow < g.OH && ocol < g.OW ? (4 * half * OHW + orow * g.OW + ocol) * 4 : STAGE_OOB;
-            const float sum = acc[q][v];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), orr, vo, mo * OHW * 4, CACHE);
+            for (int q = 0; q < NA; q++) {
+                const int orow = out_row(q), ocol = out_col(q);
+                const int vo = ok && orow < g.OH && ocol < g.OW ? (4 * half * OHW + orow * g.OW + ocol) * 4 : STAGE_OOB;
+                const float sum = acc[q][v];
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), orr, vo, mo * OHW * 4, POLICY);
+            }
         }
-    }
+    };
+    if constexpr (STORES || Z::UP)
+        put(std::integral_constant<int, STORES == 2 ? LOAD_NT : 0>());
+    else if (stream_rows(g.OW, Ob))
+        put(std::integral_constant<int, LOAD_NT>());
+    else
+        put(std::integral_constant<int, 0>());
 }
 
-// The configurations built: (filter, rows a wave, waves a SIMD, sampling, precision).
-#define FR_LP(X, P)                                                                                                 \
-    X(3, 1, 4, FR_UNIT, P) X(3, 2, 4, FR_UNIT, P) X(3, 4, 3, FR_UNIT, P) X(5, 1, 4, FR_UNIT, P) X(5, 2, 4, FR_UNIT, P) \
-    X(5, 4, 3, FR_UNIT, P) X(7, 1, 4, FR_UNIT, P) X(7, 2, 3, FR_UNIT, P) X(7, 4, 3, FR_UNIT, P)                      \
-    X(9, 1, 4, FR_UNIT, P) X(9, 2, 3, FR_UNIT, P) X(9, 4, 3, FR_UNIT, P)
-#define FR_UP(X, F, S) X(F, 1, F < 9 ? 3 : 2, S, COGCONV_FP32) X(F, 2, 2, S, COGCONV_FP32)
-#define FR_CASES(X)                                                                                                 \
-    X(3, 1, 3, FR_UNIT, COGCONV_FP32) X(5, 1, 3, FR_UNIT, COGCONV_FP32) X(7, 1, 2, FR_UNIT, COGCONV_FP32)           \
-    X(9, 1, 2, FR_UNIT, COGCONV_FP32) X(3, 2, 3, FR_UNIT, COGCONV_FP32) X(5, 2, 2, FR_UNIT, COGCONV_FP32)           \
-    X(7, 2, 2, FR_UNIT, COGCONV_FP32) X(9, 2, 2, FR_UNIT, COGCONV_FP32) X(9, 8, 1, FR_UNIT, COGCONV_FP32)           \
-    FR_UP(X, 3, FR_UP0) FR_UP(X, 3, FR_UP1) FR_UP(X, 5, FR_UP0) FR_UP(X, 7, FR_UP0) FR_UP(X, 7, FR_UP1)              \
-    FR_UP(X, 9, FR_UP0)                                                                                             \
-    X(3, 1, 2, FR_DOWN, COGCONV_FP32) X(5, 1, 2, FR_DOWN, COGCONV_FP32) X(7, 1, 2, FR_DOWN, COGCONV_FP32)           \
-    X(9, 1, 2, FR_DOWN, COGCONV_FP32)                                                                               \
-    X(3, 1, 3, FR_UNIT, COGCONV_SPLIT_BF16) X(3, 2, 3, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
-    X(3, 4, 2, FR_UNIT, COGCONV_SPLIT_BF16) X(5, 1, 3, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
-    X(5, 2, 3, FR_UNIT, COGCONV_SPLIT_BF16) X(5, 4, 2, FR_UNIT, COGCONV_SPLIT_BF16)                                 \
-    FR_LP(X, COGCONV_BF16) FR_LP(X, COGCONV_FP16)
+// The configurations built: (filter, rows a wave, output blocks a workgroup, waves a SIMD, sampling, precision).
+#define FR_LP(X, P)                                                                                                \
+    X(3, 1, 1, 4, FR_UNIT, P) X(3, 2, 1, 4, FR_UNIT, P) X(3, 4, 1, 3, FR_UNIT, P) X(3, 2, 2, 4, FR_UNIT, P)        \
+    X(3, 4, 2, 4, FR_UNIT, P) X(5, 1, 1, 4, FR_UNIT, P) X(5, 2, 1, 4, FR_UNIT, P) X(5, 4, 1, 3, FR_UNIT, P)        \
+    X(7, 1, 1, 4, FR_UNIT, P) X(7, 2, 1, 3, FR_UNIT, P) X(7, 4, 1, 3, FR_UNIT, P) X(9, 1, 1, 4, FR_UNIT, P)        \
+    X(9, 2, 1, 3, FR_UNIT, P) X(9, 4, 1, 3, FR_UNIT, P)
+#define FR_SPLIT(X, F, P) X(F, 1, 1, 3, FR_UNIT, P) X(F, 2, 1, 3, FR_UNIT, P) X(F, 4, 1, 2, FR_UNIT, P)
+#define FR_UNIT32(X, P)                                                                                            \
+    X(3, 1, 1, 3, FR_UNIT, P) X(3, 2, 1, 3, FR_UNIT, P) X(5, 1, 1, 3, FR_UNIT, P) X(5, 2, 1, 2, FR_UNIT, P)        \
+    X(7, 1, 1, 2, FR_UNIT, P) X(7, 2, 1, 2, FR_UNIT, P) X(9, 1, 1, 2, FR_UNIT, P) X(9, 2, 1, 2, FR_UNIT, P)        \
+    X(9, 8, 1, 1, FR_UNIT, P)
+#define FR_UP2(X, F, S, P) X(F, 1, 1, F < 9 ? 3 : 2, S, P) X(F, 2, 1, 2, S, P)
+#define FR_UP(X, P)                                                                                                \
+    FR_UP2(X, 3, FR_UP0, P) FR_UP2(X, 3, FR_UP1, P) FR_UP2(X, 5, FR_UP0, P) FR_UP2(X, 7, FR_UP0, P)                \
+    FR_UP2(X, 7, FR_UP1, P) FR_UP2(X, 9, FR_UP0, P)
+#define FR_DOWN2(X, P)                                                                                             \
+    X(3, 1, 1, 2, FR_DOWN, P) X(5, 1, 1, 2, FR_DOWN, P) X(7, 1, 1, 2, FR_DOWN, P) X(9, 1, 1, 2, FR_DOWN, P)
+#define FR_CASES(X)                                                                                                \
+    FR_UNIT32(X, COGCONV_FP32) FR_UP(X, COGCONV_FP32) FR_DOWN2(X, COGCONV_FP32) FR_LP(X, COGCONV_BF16)             \
+    FR_LP(X, COGCONV_FP16) FR_SPLIT(X, 3, COGCONV_SPLIT_BF16) FR_SPLIT(X, 5, COGCONV_SPLIT_BF16)
 
 // Where 16-byte staging loads pay (at four rows a wave their registers cost a block a CU).
 static constexpr bool fr_vec(int RW, int S, int prec) { return S == FR_UNIT && prec != COGCONV_FP32 && RW <= 2; }
 
-static constexpr int fr_key(int F, int RW, int S, int prec) { return ((prec * 4 + S) * 16 + F) * 16 + RW; }
+static constexpr int fr_stores(int RW, bool stream) { return RW < 4 || RW == 8 ? 0 : 1 + stream; }
 
-size_t frame_rows_lds_bytes(int F, int RW, int S, int prec) {
-    switch (fr_key(F, RW, S, prec)) {
-#define FR_LDS(F, RW, OCC, S, PREC) \
-    case fr_key(F, RW, S, PREC): return FrameRows<F, RW, S, fr_terms(PREC)>::LDS;
+static constexpr int fr_key(int F, int RW, int MW, int S, int prec) { return (((prec * 4 + S) * 16 + F) * 16 + RW) * 2 + MW - 1; }
+
+size_t frame_rows_lds_bytes(int F, int RW, int MW, int S, int prec) {
+    switch (fr_key(F, RW, MW, S, prec)) {
+#define FR_LDS(F, RW, MW, OCC, S, PREC) \
+    case fr_key(F, RW, MW, S, PREC): return FrameRows<F, RW, S, fr_terms(PREC)>::LDS;
         FR_CASES(FR_LDS)
 #undef FR_LDS
     default: return 0;
@@ -625,7 +652,7 @@ size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F, int prec) {
 hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
                              const float* w, float* out, void* ws, hipStream_t s, int stage, const Epi& ep,
                              const cogconv_image_io* tab, bool x16) {
-    const long blocks = (long)c.tilesC * c.tilesR * c.mTiles * m.B;
+    const long blocks = (long)c.tilesC * c.tilesR * ((c.mTiles + c.splits - 1) / c.splits) * m.B;
     if (blocks <= 0 || blocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
     if (prec == COGCONV_FP32 && stage != LP_PACK_AND_RUN) return hipErrorInvalidValue;  // the redo reads w itself
     if (stage != LP_RUN_ONLY) {
@@ -647,17 +674,22 @@ hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const I
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || stage == LP_PACK_ONLY) return e;
     }
-    const dim3 grid((unsigned)blocks), block(256);
+    const dim3 grid((unsigned)blocks), block(256 * c.splits);
     const bool vec = c.vec4 && (tab ? x16 : (reinterpret_cast<uintptr_t>(x) & 15) == 0);
-    switch (fr_key(g.FH, c.MB, c.variant, prec)) {
-#define FR_LAUNCH(F, RW, OCC, S, PREC)                                                                             \
-    case fr_key(F, RW, S, PREC):                                                                                   \
-        hipLaunchKernelGGL((vec ? k_frame_rows<F, RW, OCC, S, PREC, fr_vec(RW, S, PREC)>                           \
-                                : k_frame_rows<F, RW, OCC, S, PREC, false>),                                       \
-                           grid, block, c.lds_bytes, s, g, m, c, x, w, static_cast<const LpType<PREC>::T*>(ws), out, tab, ep); \
+    const bool stream = !tab && stream_rows(g.OW, out);
+    switch (fr_key(g.FH, c.MB, c.splits, c.variant, prec)) {
+#define FR_FORM(F, RW, MW, OCC, S, PREC, VEC, STREAM) k_frame_rows<F, RW, MW, OCC, S, PREC, VEC, fr_stores(RW, STREAM)>
+#define FR_LAUNCH(F, RW, MW, OCC, S, PREC)                                                                         \
+    case fr_key(F, RW, MW, S, PREC):                                                                               \
+        hipLaunchKernelGGL((vec      ? FR_FORM(F, RW, MW, OCC, S, PREC, fr_vec(RW, S, PREC), false)                \
+                            : stream ? FR_FORM(F, RW, MW, OCC, S, PREC, false, true)                               \
+                                     : FR_FORM(F, RW, MW, OCC, S, PREC, false, false)),                            \
+                           grid, block, c.lds_bytes, s, g, m, c, x, w, static_cast<const LpType<PREC>::T*>(ws),    \
+                           out, tab, ep);                                                                          \
         break;
         FR_CASES(FR_LAUNCH)
 #undef FR_LAUNCH
+#undef FR_FORM
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -568,7 +568,7 @@ bool choose_igemm_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, Ig
 // FP32 and split-BF16 frame block-reduce modes as split-BF16 products
 // (k_frame_rows): square filters, unit steps, 2x up-sampled input or every
 // second output; `rw` output rows a wave.
-bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw) {
+bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw, int mw = 1) {
     if (d->mode != COGCONV_PROJECT_FRAME_BLOCK_REDUCE_SUM && d->mode != COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM)
         return false;
     if (d->in0.dims != 2 || g.FH != g.FW || g.hR != g.hC || g.upAr != g.upAc || g.dnR != g.dnC) return false;
@@ -577,7 +577,7 @@ bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     std::memset(&c, 0, sizeof c);
     if (g.upAr == 1 && g.dnR == 1) {
         c.variant = FR_UNIT;
-    } else if (false && g.upAr == 1 && g.dnR == 2) {
+    } else if (g.upAr == 1 && g.dnR == 2) {
         c.variant = FR_DOWN;
     } else if (g.upAr == 2 && g.dnR == 1) {
         c.variant = g.hR & 1 ? FR_UP1 : FR_UP0;
@@ -585,11 +585,13 @@ bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     } else {
         return false;
     }
-    c.lds_bytes = frame_rows_lds_bytes(g.FH, rw, c.variant, d->precision);
+    c.lds_bytes = frame_rows_lds_bytes(g.FH, rw, mw, c.variant, d->precision);
     if (c.lds_bytes == 0 || c.lds_bytes > 160 * 1024) return false;
     c.MB = rw;
     c.Mout = m.T / m.N;
+    c.splits = mw;
     c.mTiles = (c.Mout + 31) / 32;
+    if (mw > c.mTiles) return false;
     const int th = 4 * rw / phases;  // rows (of a phase) of a block
     c.tilesR = ((g.OH + phases - 1) / phases + th - 1) / th;
     c.tilesC = ((g.OW + phases - 1) / phases + 31) / 32;
@@ -616,33 +618,39 @@ struct CallTime {
     }
 };
 
-// The constants fit calls measured on this card (sides 24 to 256, 3 to 64 planes, 1
-// to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log error 0.1 to 0.12 rms).
-// FP32 against the MFMA kernel, 200 calls: the faster estimate is 2% from always
-// knowing the faster kernel, the split form alone 15%, 1.15x the MFMA kernel.
-// Split-BF16 (250 calls) and BF16 / FP16 (400): 2% from the best rows a wave.
-// 2x up-sampled (300 calls, estimates within 10%): 4% from the faster kernel, 1.21x
-// the FP32 MFMA one.
+// The constants fit calls measured on this card with operands from memory (sides 24
+// to 256, 3 to 64 planes, 1 to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log
+// error 0.1 to 0.14 rms).  FP32 against the MFMA kernel: the faster estimate is 2%
+// from always knowing the faster kernel, 1.14x the MFMA kernel on 250 calls (1.15x
+// with an output step of 2, 157 calls; 1.21x up-sampled, 300 calls).  BF16 / FP16 (500
+// calls): 2% from the best configuration; split-BF16 (260): 3%.
 double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit[] = {{8.7, 1.33, 1.36, 0.09, 1.58, 0.0021},   // FP32
-                                   {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // BF16
-                                   {7.0, 1.27, 1.96, 0.07, 1.25, 0.0030},   // FP16
-                                   {6.4, 1.23, 1.52, 0.43, 1.57, 0.0013}};  // split-BF16
+    static const CallTime fit[] = {{8.9, 1.24, 1.34, 0.02, 1.56, 0.0028},   // FP32
+                                   {6.6, 1.23, 2.10, 0.45, 1.18, 0.0034},   // BF16
+                                   {6.6, 1.23, 2.10, 0.45, 1.18, 0.0034},   // FP16
+                                   {6.6, 1.03, 1.61, 0.43, 1.35, 0.0027}};  // split-BF16
+    static const CallTime down = {6.9, 1.82, 2.82, 1.66, 3.48, 0.0005};
     static const CallTime up = {8.6, 0.90, 1.69, 1.00, 1.41, 0.0045};
     const double products = d->precision == COGCONV_FP32 ? 6 : (d->precision == COGCONV_SPLIT_BF16 ? 3 : 1);
     const double mfma = g.FH * g.FW * c.MB * products * 32 / 2400.0;  // 32 cycles each
     if (g.upAr == 2)  // half the taps a wave, half the waves' rows a block
         return up.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma / 2,
                      (2.0 * c.MB + (g.FH - 1) / 2) * (32 + (g.FW - 1) / 2));
-    return fit[d->precision].us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
-                                (4.0 * c.MB + g.FH - 1) * (31 + g.FW));
+    if (g.dnR == 2)
+        return down.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
+                       (8.0 * c.MB - 2 + g.FH) * (62 + g.FW));
+    // In 256-thread units: a workgroup of two output blocks stages its pixels once.
+    const int groups = (c.mTiles + c.splits - 1) / c.splits;
+    return fit[d->precision].us((double)c.tilesR * c.tilesC * groups * c.splits * m.B, c.RC / 16, mfma,
+                                (4.0 * c.MB + g.FH - 1) * (31 + g.FW) / c.splits);
 }
 
 double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit = {4.3, 1.14, 2.45, 1.20, 2.52, 0.0050};
+    static const CallTime unit = {4.3, 1.32, 2.40, 1.13, 2.52, 0.0052}, down = {3.7, 1.93, 3.11, 2.19, 2.84, 0.0038};
+    const CallTime& fit = g.dnR == 2 ? down : unit;
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
     return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
-                  c.RC / 16.0 * (7 + g.FH) * (31 + g.FW));
+                  c.RC / 16.0 * (7 * g.dnR + g.FH) * (31 * g.dnC + g.FW));
 }
 
 double up2q_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
@@ -975,17 +983,20 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         // bits): faster than k_igemm_lp in 97% of 650 measured calls, 1.5x on average
         // and at most 1.25x slower.  One kernel's configurations only, so that
         // candidates agree bit for bit.
-        IgemmCfg fr[3];
-        bool frOk[3];
-        int first = -1;
-        for (int i = 0; i < 3; i++) {
-            frOk[i] = choose_frame_rows(desc, g, m, &fr[i], 1 << i);
-            if (frOk[i] && (first < 0 || frame_rows_us(desc, g, m, fr[i]) < frame_rows_us(desc, g, m, fr[first]))) first = i;
-        }
-        if (first >= 0) {
+        // Rows a wave and output blocks a workgroup (two for 3x3 BF16 / FP16: each
+        // pixel staged once for 64 outputs, 64 -> 64 planes, 32 images 128x128
+        // 101 -> 85 us; 5x5 122 -> 117, split-BF16 level, not built).
+        static const int forms[][2] = {{1, 1}, {2, 1}, {4, 1}, {2, 2}, {4, 2}};
+        IgemmCfg fr[5];
+        int n = 0, first = 0;
+        for (const auto& f : forms)
+            if (choose_frame_rows(desc, g, m, &fr[n], f[0], f[1])) {
+                if (frame_rows_us(desc, g, m, fr[n]) < frame_rows_us(desc, g, m, fr[first])) first = n;
+                n++;
+            }
+        if (n) {
             add(KK_FRAME_ROWS, nullptr, nullptr, &fr[first], nullptr);
-            for (int i = 0; i < 3; i++)
-                if (frOk[i]) add(KK_FRAME_ROWS, nullptr, nullptr, &fr[i], nullptr);
+            for (int i = 0; i < n; i++) add(KK_FRAME_ROWS, nullptr, nullptr, &fr[i], nullptr);
             return;
         }
         add(KK_IGEMM_LP, nullptr, nullptr, &lp, nullptr);
@@ -1334,8 +1345,8 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
     {
         static const char* const names[] = {"igemm_f32x3", "igemm_bf16x1", "igemm_fp16x1", "igemm_bf16x2"};
         const char* name = g.upAr == 2 ? "igemm_f32_up2x3" : names[plan->desc.precision];
-        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=256%s lds=%zu",
-                 name, mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, plan->icfg.vec4 ? " ld16" : "",
+        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=%d%s lds=%zu",
+                 name, mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, 256 * plan->icfg.splits, plan->icfg.vec4 ? " ld16" : "",
                  plan->icfg.lds_bytes);
         break;
     }

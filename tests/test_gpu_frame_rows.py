@@ -24,7 +24,7 @@ def candidates(cd):
     plans = [L.Plan(cd, v) for v in range(L.variant_count(cd))]
     rows = [p for p in plans if p.description.startswith("igemm_f32x3")]
     mfma = [p for p in plans if p.description.startswith("igemm_f32 ")]
-    return rows, mfma[0]
+    return rows, mfma[0] if mfma else None
 
 
 def launch(plan, a, k, off=0):
@@ -117,6 +117,36 @@ def test_upsampled_every_candidate(border, B, N, K, H, W, F, orient):
         p.close()
 
 
+@pytest.mark.parametrize("border,B,N,K,H,W,F", [
+    (O.CLAMP, 1, 1, 1, 2, 4, 3),       # one output row and two columns
+    (O.CYCLIC, 2, 16, 32, 16, 128, 3), # whole tiles
+    (O.ZERO, 1, 17, 33, 18, 66, 5),    # one output row, column, plane and block past the tiles
+    (O.VALID, 1, 40, 9, 30, 40, 7),
+    (O.ZERO, 2, 9, 20, 22, 26, 9),
+    (O.CYCLIC, 1, 5, 3, 4, 6, 9),      # the filter larger than the field
+])
+def test_output_step_every_candidate(border, B, N, K, H, W, F):
+    """Every second output: parity, and non-finite samples reaching exactly the
+    outputs they reach in the FP32 MFMA kernel."""
+    rng = np.random.default_rng(F * 100 + H + W)
+    a = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    k = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    od, cd = desc_pair(O.PF_BRS, border, O.XCORR, O.DOWN, 2, B, a.shape, k.shape)
+    rows, _ = candidates(cd)
+    other = [L.Plan(cd, v) for v in range(L.variant_count(cd))]
+    other = [p for p in other if p.description.startswith(("igemm_f32 ", "direct"))]
+    assert rows
+    ref, mag = oracle_ref(od, a, k)
+    b = a.copy()
+    b[0, H // 2, W // 2], b[N - 1, 0, W - 1] = np.inf, np.nan
+    want = launch(other[0], b, k)
+    for i, p in enumerate(rows):
+        print("CASE down rows", border, p.description, flush=True)
+        assert_parity(launch(p, a, k, off=i + 1), ref, mag, what=p.description)
+        bad = launch(p, b, k)
+        assert np.array_equal(np.isnan(bad), np.isnan(want)) and np.array_equal(np.isinf(bad), np.isinf(want))
+
+
 @pytest.mark.parametrize("scale", (1e-36, 1e-30, 1e30))
 def test_magnitudes_beyond_the_split(scale):
     """Operands whose low BF16 terms underflow, and large ones: as exact as near 1."""
@@ -165,6 +195,7 @@ def rounded(a, precision):
     (O.PF_BRS, O.VALID, 3, 8, 20, 18, 44, 3),
     (O.PF_BRS, O.ZERO, 1, 20, 12, 8, 33, 3),     # rows of an odd width: no 16-byte loads
     (O.BPF_BRS, O.CYCLIC, 1, 50, 7, 5, 6, 7),    # the filter larger than the field
+    (O.PF_BRS, O.CLAMP, 1, 24, 70, 33, 64, 3),   # three output blocks in workgroups of two, whole-line rows
 ])
 def test_low_precision_every_candidate(precision, mode, border, B, N, K, H, W, F):
     """BF16 and FP16: FP32 summation error only, against the oracle on the rounded
