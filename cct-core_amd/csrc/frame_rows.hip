@@ -210,7 +210,9 @@ __device__ __forceinline__ float frame_point(const Geom& g, const PlaneMap& m, c
 // VEC: 16-byte staging loads.  STORES: 0 picks the stores' cache policy at run time;
 // at four rows a wave, where the two forms side by side spill, 1 is the cached
 // and 2 the streamed one.
-template <int F, int RW, int MW, int OCC, int S, int PREC, bool VEC, int STORES>
+// INLINE: the workgroup packs its filters itself, chunk by chunk, into LDS: no
+// packed bank, one launch.
+template <int F, int RW, int MW, int OCC, int S, int PREC, bool VEC, int STORES, bool INLINE>
 __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m, IgemmCfg c, const float* __restrict__ X,
                                                          const float* __restrict__ Wt,
                                                          const typename LpType<PREC>::T* __restrict__ Wp,
@@ -326,11 +328,13 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     };
     // Filters held: a tap column, loaded one ahead, or all F of a chunk (DEEP, where
     // they fit registers), loaded a chunk ahead.
-    constexpr bool DEEP = S == FR_UNIT && F == 3 && T == 1 && MW * RW < 8;
+    constexpr bool DEEP = S == FR_UNIT && F == 3 && T == 1 && MW * RW < 8 && !INLINE;
     V a[DEEP ? F : 1][NT][T];
+    unsigned char* sFilt = fr_smem + Z::LDS;  // INLINE: the chunk's fragments, in the bank's order
     auto fragment = [&](int at, int i, int t) __attribute__((always_inline)) {
         return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(wr, at, (NP * i * T + t) * FRAG, 0));
     };
+    if (!INLINE)
 #pragma unroll
     for (int k = 0; k < (DEEP ? F : 1); k++)
 #pragma unroll
@@ -342,8 +346,9 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
                          (size_t)mt * chunks * F * F;
     bool smallW = false;
     if (EXACT) {
-        for (int i = lane; i < chunks * F * F; i += 64) smallW |= range[i].y != 0;
-        if (tid < 2) sRange[tid] = 0u;
+        if (!INLINE)
+            for (int i = lane; i < chunks * F * F; i += 64) smallW |= range[i].y != 0;
+        if (tid < 4) sRange[tid] = 0u;
         __syncthreads();  // before the first chunk's stores
     }
 
@@ -355,6 +360,12 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         const int d = DEEP ? k : 0;
         const int off = S == FR_DOWN ? (j & 1) * Z::HC + (j >> 1) : Z::off(j);
         const unsigned char* bp = fr_smem + rdBase + (Z::off(SET) * TC + off) * 16;
+        if (INLINE)
+#pragma unroll
+            for (int i = 0; i < N; i++)
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    a[0][i][t] = *reinterpret_cast<const V*>(sFilt + ((k * F + i) * T + t) * FRAG + lane * 16);
 #pragma unroll
         for (int y = 0; y < Z::STEP * (RW - 1) + N; y++) {
             V bv[T];
@@ -374,7 +385,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
                         else low[EXACT ? at : 0] = fr_mfma<PREC>(a[d][i][ta], bv[tb], low[EXACT ? at : 0]);
                     }
             // A tap row that has met its last row gives its registers to the next tap column's.
-            if (y >= Z::STEP * (RW - 1)) {
+            if (!INLINE && y >= Z::STEP * (RW - 1)) {
                 const int i = y - Z::STEP * (RW - 1);
 #pragma unroll
                 for (int t = 0; t < T; t++) a[d][i][t] = fragment(next, i, t);
@@ -470,7 +481,55 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         }
         if (EXACT && any_small(least) && lane == 0) sRange[0] = 1u;
     };
+    // INLINE: unit u of a chunk is 8 planes of one output and tap, tap fastest (the
+    // order of the filters in memory); FB units of a thread at a time.
+    constexpr int FN = F * F * 64, FU = (FN + NTH - 1) / NTH, FB = FU <= 3 ? FU : 4;
+    float fv[INLINE ? FB : 1][8];
+    unsigned mostW = 0u;
+    const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
+    const int planeW = (bpf ? m.T / m.N : 1) * F * F * 4;  // bytes between an output's planes
+    const __amdgpu_buffer_rsrc_t fr = buffer_rsrc(Wt, (uint32_t)m.T * F * F * 4u);
+    auto load_filters = [&](int ch, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < FB; k++) {
+            const int u = tid + NTH * (k0 + k);
+            const int t = u % (F * F), mm = u / (F * F) & 31, h = u / (F * F) >> 5;
+            const bool live = k0 + k < FU && u < FN && m0 + mm < Mout;
+            const int at = ((bpf ? m0 + mm : (m0 + mm) * m.N) * F * F + t) * 4 + 8 * h * planeW;
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                fv[INLINE ? k : 0][q] = buffer_load_f32(fr, live && ch * FR_RC + 8 * h + q < m.R ? at : STAGE_OOB,
+                                                        (ch * FR_RC + q) * planeW);
+        }
+    };
+    auto store_filters = [&](int k0) __attribute__((always_inline)) {
+        unsigned least = ~0u;
+#pragma unroll
+        for (int k = 0; k < FB; k++) {
+            const int u = tid + NTH * (k0 + k);
+            if (k0 + k >= FU || u >= FN) continue;
+            const int t = u % (F * F), pos = g.flip ? F * F - 1 - t : t;  // tap row pos / F, column pos % F
+            V s[T];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const float w = fv[INLINE ? k : 0][q];
+                if (EXACT) {
+                    mostW = max(mostW, magnitude(w));
+                    least = min(least, magnitude(w) - 1u);
+                }
+                E t3[T];
+                split_terms<T>(w, t3);
+#pragma unroll
+                for (int e = 0; e < T; e++) s[e][q] = t3[e];
+            }
+#pragma unroll
+            for (int e = 0; e < T; e++)
+                *reinterpret_cast<V*>(sFilt + ((pos % F * F + pos / F) * T + e) * FRAG + u / (F * F) * 16) = s[e];
+        }
+        if (EXACT && any_small(least) && lane == 0) sRange[2] = 1u;
+    };
     if (AHEAD) load(0, 0, 0);
+    if (INLINE && FB == FU) load_filters(0, 0);
     for (int ch = 0; ch < chunks; ch++) {
         if (ch) __syncthreads();
         if (AHEAD) {
@@ -484,9 +543,21 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
                     store(h, k0);
                 }
         }
+        if (INLINE) {
+            if (FB == FU) {
+                store_filters(0);
+            } else {
+#pragma unroll 1
+                for (int k0 = 0; k0 < FU; k0 += FB) {
+                    load_filters(ch, k0);
+                    store_filters(k0);
+                }
+            }
+        }
         __syncthreads();
         if (AHEAD && ch + 1 < chunks) load(ch + 1, 0, 0);
-        constexpr int UNROLL = DEEP ? F : 1;
+        if (INLINE && FB == FU && ch + 1 < chunks) load_filters(ch + 1, 0);
+        constexpr int UNROLL = DEEP || (INLINE && F == 3) ? F : 1;
 #pragma unroll UNROLL
         for (int k = 0; k < (Z::UP ? kOdd : F); k++) column(ch, k, std::integral_constant<int, 0>());
         if constexpr (Z::UP)
@@ -514,10 +585,17 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         float bound = 1.f;
         if (sRange[0]) {
             unsigned wMost = 0u;
-            for (int i = lane; i < chunks * F * F; i += 64) wMost = max(wMost, range[i].x);
+            if (INLINE) {
+                mostW = wave_max(mostW);
+                if (lane == 0) atomicMax(&sRange[3], mostW);
+                __syncthreads();
+                wMost = sRange[3];
+            } else {
+                for (int i = lane; i < chunks * F * F; i += 64) wMost = max(wMost, range[i].x);
+            }
             bound += __uint_as_float(min(wave_max(wMost), FINITE));
         }
-        if (__any(smallW)) {  // the same in every wave
+        if (INLINE ? sRange[2] != 0 : __any(smallW)) {  // the same in every wave
             most = wave_max(most);
             if (lane == 0) atomicMax(&sRange[1], most);
             __syncthreads();
@@ -631,6 +709,17 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
 // Where 16-byte staging loads pay (at four rows a wave their registers cost a block a CU).
 static constexpr bool fr_vec(int RW, int S, int prec) { return S == FR_UNIT && prec != COGCONV_FP32 && RW <= 2; }
 
+// Where a workgroup may pack its own filters.  3x3: 1.20x the packed form's time on
+// 158 small and middle calls (BF16, FP16, split-BF16; 4 images 75x96, 7 -> 8 planes:
+// 7.3 -> 4.8 us), 5x5 BF16 / FP16 1.07x where it wins.  Not built: 7x7 (0.64x: 49
+// scattered taps a workgroup and chunk), 5x5 split-BF16 (1.02x where it wins), FP32
+// (1.03x).
+static constexpr bool fr_inline(int F, int RW, int MW, int S, int prec) {
+    return S == FR_UNIT && MW == 1 && prec != COGCONV_FP32 &&
+           (F == 3 ? RW <= 2 : F == 5 && RW == 1 && prec != COGCONV_SPLIT_BF16);
+}
+bool frame_rows_inline(int F, int RW, int MW, int S, int prec) { return fr_inline(F, RW, MW, S, prec); }
+
 static constexpr int fr_stores(int RW, bool stream) { return RW < 4 || RW == 8 ? 0 : 1 + stream; }
 
 static constexpr int fr_key(int F, int RW, int MW, int S, int prec) { return (((prec * 4 + S) * 16 + F) * 16 + RW) * 2 + MW - 1; }
@@ -655,7 +744,8 @@ hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const I
     const long blocks = (long)c.tilesC * c.tilesR * ((c.mTiles + c.splits - 1) / c.splits) * m.B;
     if (blocks <= 0 || blocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
     if (prec == COGCONV_FP32 && stage != LP_PACK_AND_RUN) return hipErrorInvalidValue;  // the redo reads w itself
-    if (stage != LP_RUN_ONLY) {
+    const bool own = c.ring && stage == LP_PACK_AND_RUN;
+    if (stage != LP_RUN_ONLY && !own) {
         const long total = (long)c.mTiles * (c.RC / FR_RC) * g.FH * g.FW * 64;
         const dim3 grid((unsigned)std::min((total + 255) / 256, 4096L)), block(256);
         switch (prec) {
@@ -676,15 +766,19 @@ hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const I
     }
     const dim3 grid((unsigned)blocks), block(256 * c.splits);
     const bool vec = c.vec4 && (tab ? x16 : (reinterpret_cast<uintptr_t>(x) & 15) == 0);
+    const size_t lds = c.lds_bytes + (own ? (size_t)g.FH * g.FW * fr_terms(prec) * 1024 : 0);
     const bool stream = !tab && stream_rows(g.OW, out);
     switch (fr_key(g.FH, c.MB, c.splits, c.variant, prec)) {
-#define FR_FORM(F, RW, MW, OCC, S, PREC, VEC, STREAM) k_frame_rows<F, RW, MW, OCC, S, PREC, VEC, fr_stores(RW, STREAM)>
+#define FR_FORM(F, RW, MW, OCC, S, PREC, VEC, STREAM, OWN) \
+    k_frame_rows<F, RW, MW, OCC, S, PREC, VEC, fr_stores(RW, STREAM), OWN && fr_inline(F, RW, MW, S, PREC)>
 #define FR_LAUNCH(F, RW, MW, OCC, S, PREC)                                                                         \
     case fr_key(F, RW, MW, S, PREC):                                                                               \
-        hipLaunchKernelGGL((vec      ? FR_FORM(F, RW, MW, OCC, S, PREC, fr_vec(RW, S, PREC), false)                \
-                            : stream ? FR_FORM(F, RW, MW, OCC, S, PREC, false, true)                               \
-                                     : FR_FORM(F, RW, MW, OCC, S, PREC, false, false)),                            \
-                           grid, block, c.lds_bytes, s, g, m, c, x, w, static_cast<const LpType<PREC>::T*>(ws),    \
+        hipLaunchKernelGGL((own ? (vec ? FR_FORM(F, RW, MW, OCC, S, PREC, fr_vec(RW, S, PREC), false, true)        \
+                                       : FR_FORM(F, RW, MW, OCC, S, PREC, false, false, true))                     \
+                            : vec    ? FR_FORM(F, RW, MW, OCC, S, PREC, fr_vec(RW, S, PREC), false, false)         \
+                            : stream ? FR_FORM(F, RW, MW, OCC, S, PREC, false, true, false)                        \
+                                     : FR_FORM(F, RW, MW, OCC, S, PREC, false, false, false)),                     \
+                           grid, block, lds, s, g, m, c, x, w, static_cast<const LpType<PREC>::T*>(ws),    \
                            out, tab, ep);                                                                          \
         break;
         FR_CASES(FR_LAUNCH)

@@ -320,6 +320,7 @@ hipError_t launch_igemm_lp(int precision, const Geom& g, const PlaneMap& m, cons
 // (the FP32 form packs on every launch).
 enum FrameRowsSampling { FR_UNIT = 0, FR_UP0 = 1, FR_UP1 = 2, FR_DOWN = 3 };
 size_t frame_rows_lds_bytes(int F, int RW, int MW, int sampling, int precision);  // 0: not built
+bool frame_rows_inline(int F, int RW, int MW, int sampling, int precision);  // plain launches may pack in the kernel (c.ring)
 size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F, int precision);
 hipError_t launch_frame_rows(int precision, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
                              const float* w, float* out, void* ws, hipStream_t s, int stage = LP_PACK_AND_RUN,

@@ -568,7 +568,8 @@ bool choose_igemm_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, Ig
 // FP32 and split-BF16 frame block-reduce modes as split-BF16 products
 // (k_frame_rows): square filters, unit steps, 2x up-sampled input or every
 // second output; `rw` output rows a wave.
-bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw, int mw = 1) {
+bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw, int mw = 1,
+                       bool own = false) {
     if (d->mode != COGCONV_PROJECT_FRAME_BLOCK_REDUCE_SUM && d->mode != COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM)
         return false;
     if (d->in0.dims != 2 || g.FH != g.FW || g.hR != g.hC || g.upAr != g.upAc || g.dnR != g.dnC) return false;
@@ -587,6 +588,9 @@ bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     }
     c.lds_bytes = frame_rows_lds_bytes(g.FH, rw, mw, c.variant, d->precision);
     if (c.lds_bytes == 0 || c.lds_bytes > 160 * 1024) return false;
+    if (own && (!frame_rows_inline(g.FH, rw, mw, c.variant, d->precision) || (long)m.T * g.FH * g.FW * 4 >= (1L << 31)))
+        return false;
+    c.ring = own;  // plain launches pack their filters in the kernel
     c.MB = rw;
     c.Mout = m.T / m.N;
     c.splits = mw;
@@ -623,7 +627,8 @@ struct CallTime {
 // error 0.1 to 0.14 rms).  FP32 against the MFMA kernel: the faster estimate is 2%
 // from always knowing the faster kernel, 1.14x the MFMA kernel on 250 calls (1.15x
 // with an output step of 2, 157 calls; 1.21x up-sampled, 300 calls).  BF16 / FP16 (500
-// calls): 2% from the best configuration; split-BF16 (260): 3%.
+// calls): 2% from the best configuration; split-BF16 (260): 3%; packing in the kernel
+// where it is estimated faster gains another 1.07x and 1.10x.
 double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
     static const CallTime fit[] = {{8.9, 1.24, 1.34, 0.02, 1.56, 0.0028},   // FP32
                                    {6.6, 1.23, 2.10, 0.45, 1.18, 0.0034},   // BF16
@@ -639,6 +644,13 @@ double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, co
     if (g.dnR == 2)
         return down.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
                        (8.0 * c.MB - 2 + g.FH) * (62 + g.FW));
+    // A workgroup that packs its own filters: one launch, its staging in the chunk.
+    static const CallTime lpInline = {3.7, 0.16, 8.93, 0.36, 4.55, 0.0007},
+                          splitInline = {3.7, 0.78, 3.01, 0.10, 1.88, 0.0018};
+    if (c.ring)
+        return (products == 3 ? splitInline : lpInline)
+            .us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
+                (4.0 * c.MB + g.FH - 1) * (31 + g.FW) + 32.0 * g.FH * g.FW);
     // In 256-thread units: a workgroup of two output blocks stages its pixels once.
     const int groups = (c.mTiles + c.splits - 1) / c.splits;
     return fit[d->precision].us((double)c.tilesR * c.tilesC * groups * c.splits * m.B, c.RC / 16, mfma,
@@ -983,14 +995,14 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         // bits): faster than k_igemm_lp in 97% of 650 measured calls, 1.5x on average
         // and at most 1.25x slower.  One kernel's configurations only, so that
         // candidates agree bit for bit.
-        // Rows a wave and output blocks a workgroup (two for 3x3 BF16 / FP16: each
+        // Rows a wave, output blocks a workgroup, filters packed in the kernel (two blocks for 3x3 BF16 / FP16: each
         // pixel staged once for 64 outputs, 64 -> 64 planes, 32 images 128x128
         // 101 -> 85 us; 5x5 122 -> 117, split-BF16 level, not built).
-        static const int forms[][2] = {{1, 1}, {2, 1}, {4, 1}, {2, 2}, {4, 2}};
-        IgemmCfg fr[5];
+        static const int forms[][3] = {{1, 1, 0}, {2, 1, 0}, {4, 1, 0}, {2, 2, 0}, {4, 2, 0}, {1, 1, 1}, {2, 1, 1}};
+        IgemmCfg fr[7];
         int n = 0, first = 0;
         for (const auto& f : forms)
-            if (choose_frame_rows(desc, g, m, &fr[n], f[0], f[1])) {
+            if (choose_frame_rows(desc, g, m, &fr[n], f[0], f[1], f[2])) {
                 if (frame_rows_us(desc, g, m, fr[n]) < frame_rows_us(desc, g, m, fr[first])) first = n;
                 n++;
             }
@@ -1345,9 +1357,9 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
     {
         static const char* const names[] = {"igemm_f32x3", "igemm_bf16x1", "igemm_fp16x1", "igemm_bf16x2"};
         const char* name = g.upAr == 2 ? "igemm_f32_up2x3" : names[plan->desc.precision];
-        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=%d%s lds=%zu",
+        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=%d%s%s lds=%zu",
                  name, mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, 256 * plan->icfg.splits, plan->icfg.vec4 ? " ld16" : "",
-                 plan->icfg.lds_bytes);
+                 plan->icfg.ring ? " inline" : "", plan->icfg.lds_bytes);
         break;
     }
     case KK_IGEMM_UP: {

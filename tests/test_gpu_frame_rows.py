@@ -196,6 +196,8 @@ def rounded(a, precision):
     (O.PF_BRS, O.ZERO, 1, 20, 12, 8, 33, 3),     # rows of an odd width: no 16-byte loads
     (O.BPF_BRS, O.CYCLIC, 1, 50, 7, 5, 6, 7),    # the filter larger than the field
     (O.PF_BRS, O.CLAMP, 1, 24, 70, 33, 64, 3),   # three output blocks in workgroups of two, whole-line rows
+    (O.BPF_BRS, O.ZERO, 1, 35, 33, 10, 12, 3),   # filters packed in the kernel: partial chunk and block, both
+    (O.BPF_BRS, O.ZERO, 2, 19, 3, 9, 31, 5),     # orientations
 ])
 def test_low_precision_every_candidate(precision, mode, border, B, N, K, H, W, F):
     """BF16 and FP16: FP32 summation error only, against the oracle on the rounded
@@ -215,9 +217,10 @@ def test_low_precision_every_candidate(precision, mode, border, B, N, K, H, W, F
     else:
         ref, mag = oracle_ref(od, rounded(a, precision), rounded(k, precision))
         tol = 2e-6
-    first = None
+    first, inline = None, 0
     for v in range(L.variant_count(cd)):
         p = L.Plan(cd, v)
+        inline += "inline" in p.description
         print("CASE low precision", mode, border, p.description, flush=True)
         assert "x1" in p.description or "x2" in p.description
         for off in (0, 1):
@@ -234,6 +237,7 @@ def test_low_precision_every_candidate(precision, mode, border, B, N, K, H, W, F
         for x in (ba, bk, ws, bo):
             x.close()
         p.close()
+    assert inline == (2 if F == 3 else int(F == 5 and precision != L.SPLIT_BF16))
 
 
 def test_non_finite_operands():
