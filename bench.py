@@ -225,6 +225,8 @@ def timed_steps(L, ops, stream, steps, warmup):
 def roofline(plan, ms, peak_tflops, name, reps, traffic_file):
     """Roofline object for one launch of `plan` taking `ms`: compute-bound when
     its algorithmic FLOP/byte is above the ridge of `peak_tflops` and HBM."""
+    if "x3 " in plan.description:
+        peak_tflops = round(PEAK_BF16_TFLOPS / 6, 1)  # FP32 as six BF16 products
     ai = plan.flops / plan.bytes
     ridge = peak_tflops * 1e12 / (PEAK_HBM_GBS * 1e9)
     if ai >= ridge:
