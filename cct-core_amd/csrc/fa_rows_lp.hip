@@ -1,4 +1,4 @@
-// Row-streaming BF16 / FP16 FilterAdjointBlockReduceSum for BorderValid,
+// Row-streaming BF16 / FP16 / FP32 FilterAdjointBlockReduceSum for BorderValid,
 // unit steps, cross-correlation orientation (the weight gradient of a
 // stride-1 layer):
 //
@@ -30,6 +30,12 @@
 // split's partial,
 // ws[s][k][n][i][j]; the partials are summed afterwards in split order
 // (launch_reduce_partials), so the result does not depend on timing.
+//
+// FP32 operands are three BF16 terms each, six products, the low ones in
+// accumulators of their own (see frame_rows.hip): 1x1 and 3x3 dW.  Bound by the matrix
+// cores and the LDS stores of three terms; 16 images 173x256, 22 -> 2 planes: 178 us on
+// the FP32 MFMA kernel, 84 us here, relative error 5.2e-7 and 2.3e-7; 10 images
+// 201x256, 45 -> 10: 259 and 124 us.  In one accumulator the error reached 4e-6.
 #include "lp.h"
 #include "stage.h"
 
@@ -54,12 +60,23 @@ __device__ __forceinline__ void load4(__amdgpu_buffer_rsrc_t r, int vo, float (&
     v[3] = q.w;
 }
 
-// Four rounded elements, as the 8-byte half of an 8-element LDS slot.
+// Four elements, as the 8-byte half of an 8-element LDS slot of each of their
+// terms, `stride` elements apart.
 template <int PREC>
-__device__ __forceinline__ void store4(typename LpType<PREC>::T* dst, const float (&v)[4]) {
+__device__ __forceinline__ void store4(typename LpType<PREC>::T* dst, int stride, const float (&v)[4]) {
     typedef typename LpType<PREC>::T T;
     typedef T T4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<T4*>(dst) = T4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
+    constexpr int NT = lp_terms(PREC);
+    T4 q[NT];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        T t[NT];
+        split_terms<NT>(v[e], t);
+#pragma unroll
+        for (int k = 0; k < NT; k++) q[k][e] = t[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NT; k++) *reinterpret_cast<T4*>(dst + k * stride) = q[k];
 }
 
 // Elements j .. j + 7 of the 16-element run cur ++ nxt (16-bit elements).
@@ -95,10 +112,14 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
     constexpr int NT = NB * 16;        // x planes of the tile
     constexpr int RB = OD + 1;         // x rows in the ring
     constexpr int P = OD * OD;
+    constexpr int TM = lp_terms(PREC);  // BF16 terms of an operand
+    constexpr bool EXACT = TM == 3;
     extern __shared__ __attribute__((aligned(16))) unsigned char fr_smem[];
-    T* sD = reinterpret_cast<T*>(fr_smem);  // [2][4][KT][8]: dy rows, double-buffered
-    T* sX = sD + 2 * 4 * KT * 8;            // [RB][FR_XS][NT][8]: x row ring
-    T* sJunk = sX + RB * FR_XS * NT * 8;    // [8]: where lanes without a piece store theirs
+    constexpr int DT = 2 * 4 * KT * 8, XT = RB * FR_XS * NT * 8;  // elements of one term
+    T* sD = reinterpret_cast<T*>(fr_smem);  // [terms][2][4][KT][8]: dy rows, double-buffered
+    T* sX = sD + TM * DT;                   // [terms][RB][FR_XS][NT][8]: x row ring
+    T* sJunk = sX + TM * XT;                // [8]: where lanes without a piece store theirs
+    unsigned mostD = 0u, mostX = 0u, leastD = ~0u, leastX = ~0u;  // EXACT: magnitudes staged (see any_small)
 
     const int tiles = c.nTiles * c.kTiles;
     const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -174,7 +195,14 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
             float m[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) m[e] = dPix[d] + e < dyW ? v[d][e] : 0.f;
-            store4<PREC>(dUnit[d] ? sD + buf * 4 * KT * 8 + dDst[d] : sJunk, m);
+            if (EXACT) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    mostD = max(mostD, magnitude(m[e]));
+                    leastD = min(leastD, magnitude(m[e]) - 1u);
+                }
+            }
+            store4<PREC>(dUnit[d] ? sD + buf * 4 * KT * 8 + dDst[d] : sJunk, dUnit[d] ? DT : 0, m);
         }
     };
     auto load_x = [&](int y, bool on, float (&v)[XP][4]) {
@@ -188,17 +216,28 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
             float m[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) m[e] = xPix[d] + e < W ? v[d][e] : 0.f;
-            store4<PREC>(xUnit[d] ? sX + row * FR_XS * NT * 8 + xDst[d] : sJunk, m);
+            if (EXACT) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    mostX = max(mostX, magnitude(m[e]));
+                    leastX = min(leastX, magnitude(m[e]) - 1u);
+                }
+            }
+            store4<PREC>(xUnit[d] ? sX + row * FR_XS * NT * 8 + xDst[d] : sJunk, xUnit[d] ? XT : 0, m);
         }
     };
 
-    floatx4 acc[KBW][OD][OD];
+    // EXACT: the products with a low term sum apart (see k_frame_rows).
+    floatx4 acc[KBW][OD][OD], low[EXACT ? KBW : 1][EXACT ? OD : 1][EXACT ? OD : 1];
 #pragma unroll
     for (int kb = 0; kb < KBW; kb++)
 #pragma unroll
         for (int i = 0; i < OD; i++)
 #pragma unroll
-            for (int j = 0; j < OD; j++) acc[kb][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < OD; j++) {
+                acc[kb][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                if (EXACT) low[EXACT ? kb : 0][EXACT ? i : 0][EXACT ? j : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
 
     // Rows y0 .. y1 - 1, streamed down with a fresh prologue.
     auto stream = [&](const int y0, const int y1) {
@@ -237,22 +276,40 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                 load_dy(y + FR_PD, y + FR_PD < y1, qd[u]);
                 load_x(y + FR_PD + OD - 1, y + FR_PD < y1, qx[u]);
                 const T* dBuf = sD + (t & 1) * 4 * KT * 8;
-                V a[KBW];
+                V a[KBW][TM];
 #pragma unroll
                 for (int kb = 0; kb < KBW; kb++)
-                    a[kb] = *reinterpret_cast<const V*>(dBuf + (g4 * KT + (kh * KBW + kb) * 16 + l16) * 8);
+#pragma unroll
+                    for (int q = 0; q < TM; q++)
+                        a[kb][q] = *reinterpret_cast<const V*>(dBuf + q * DT + (g4 * KT + (kh * KBW + kb) * 16 + l16) * 8);
 #pragma unroll
                 for (int i = 0; i < OD; i++) {
                     int rr = ring0 + i;
                     rr -= rr >= RB ? RB : 0;
                     const T* xRow = sX + (rr * FR_XS * NT + nb * 16 + l16) * 8;
-                    const V cur = *reinterpret_cast<const V*>(xRow + g4 * NT * 8);
-                    const V nxt = *reinterpret_cast<const V*>(xRow + (g4 + 1) * NT * 8);
+                    V cur[TM], nxt[TM];
+#pragma unroll
+                    for (int q = 0; q < TM; q++) {
+                        cur[q] = *reinterpret_cast<const V*>(xRow + q * XT + g4 * NT * 8);
+                        nxt[q] = *reinterpret_cast<const V*>(xRow + q * XT + (g4 + 1) * NT * 8);
+                    }
                     auto tap = [&](auto jc) {
                         constexpr int J = decltype(jc)::value;
-                        const V bj = window<J>(cur, nxt);
+                        // The products with term indexes summing to less than TM, smallest first.
 #pragma unroll
-                        for (int kb = 0; kb < KBW; kb++) acc[kb][i][J] = lp_mfma<PREC>(a[kb], bj, acc[kb][i][J]);
+                        for (int q = TM - 1; q >= 0; q--) {
+                            const V bj = window<J>(cur[q], nxt[q]);
+#pragma unroll
+                            for (int r = TM - 1 - q; r >= 0; r--)
+#pragma unroll
+                                for (int kb = 0; kb < KBW; kb++) {
+                                    if (!EXACT || q + r == 0)
+                                        acc[kb][i][J] = lp_mfma<PREC>(a[kb][r], bj, acc[kb][i][J]);
+                                    else
+                                        low[EXACT ? kb : 0][EXACT ? i : 0][EXACT ? J : 0] = lp_mfma<PREC>(
+                                            a[kb][r], bj, low[EXACT ? kb : 0][EXACT ? i : 0][EXACT ? J : 0]);
+                                }
+                        }
                     };
                     tap(std::integral_constant<int, 0>{});
                     if constexpr (OD > 1) {
@@ -291,6 +348,14 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
     const int off = run > 0 ? (b * 11) % run : 0;
     stream(yBeg + off, yEnd);
     if (off) stream(yBeg, yBeg + off);
+    if (EXACT) {
+#pragma unroll
+        for (int kb = 0; kb < KBW; kb++)
+#pragma unroll
+            for (int i = 0; i < OD; i++)
+#pragma unroll
+                for (int j = 0; j < OD; j++) acc[kb][i][j] += low[EXACT ? kb : 0][EXACT ? i : 0][EXACT ? j : 0];
+    }
     // The split's partial: ws[s][k][n][i][j] (every (k, n, i, j) of the tile,
     // zeros for a block without rows).
     const size_t total = (size_t)K * N * P;
@@ -309,11 +374,65 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                     for (int j = 0; j < OD; j++) o[i * OD + j] = acc[kb][i][j][v];
             }
         }
+    if constexpr (EXACT) {
+        // As in k_frame_rows: partials that are not finite, or so small that lost
+        // products or terms may matter, are summed again by FP32 multiply-adds.
+        unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem);  // the last step ended with a barrier
+        if (tid < 4) sRange[tid] = 0u;
+        __syncthreads();
+        mostD = wave_max(mostD);
+        mostX = wave_max(mostX);
+        const bool smallD = any_small(leastD), smallX = any_small(leastX);
+        if (lane == 0) {
+            atomicMax(&sRange[0], mostD);
+            atomicMax(&sRange[1], mostX);
+            if (smallD) sRange[2] = 1u;
+            if (smallX) sRange[3] = 1u;
+        }
+        __syncthreads();
+        constexpr unsigned FINITE = 0x7f7fffffu;
+        float bound = 1.f;
+        if (sRange[3]) bound += __uint_as_float(min(sRange[0], FINITE));
+        if (sRange[2]) bound += __uint_as_float(min(sRange[1], FINITE));
+        const float tiny = 0x1p-100f * 32.f * (float)max(run, 1) * bound;
+        float z = 0.f;
+        bool redo = false;
+#pragma unroll
+        for (int kb = 0; kb < KBW; kb++)
+#pragma unroll
+            for (int i = 0; i < OD; i++)
+#pragma unroll
+                for (int j = 0; j < OD; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float q = acc[kb][i][j][v];
+                        z = fmaf(q, 0.f, z);
+                        redo |= fabsf(q) < tiny && q != 0.f;
+                    }
+        if (__any(redo || z != z)) {
+            // Each thread reads back its own stores.
+#pragma unroll 1
+            for (int e = 0; e < KBW * 4 * P; e++) {
+                const int ij = e % P, k = kt * KT + (kh * KBW + e / P / 4) * 16 + 4 * g4 + e / P % 4;
+                if (k >= K || n >= N) continue;
+                float* o = out + ((size_t)k * N + n) * P + ij;
+                const float q = fabsf(*o);
+                if (q < __builtin_inff() && (q >= tiny || q == 0.f)) continue;
+                const float* dp = DY + ((size_t)b * K + k) * dyH * dyW;
+                const float* xp = X + ((size_t)b * N + n) * H * W + ij % OD;
+                float sum = 0.f;
+                for (int y = yBeg; y < yEnd; y++)
+                    for (int x = x0; x < min(x0 + 32, dyW); x++)
+                        sum = fmaf(dp[y * dyW + x], xp[(y + ij / OD) * W + x], sum);
+                *o = sum;
+            }
+        }
+    }
 }
 
-size_t fa_rows_lp_lds_bytes(const FaCfg& c, int OD) {
+size_t fa_rows_lp_lds_bytes(const FaCfg& c, int OD, int precision) {
     const int KT = c.kh * c.kbw * 16, NT = c.nb * 16;
-    return (size_t)2 * 4 * KT * 16 + (size_t)(OD + 1) * FR_XS * NT * 16 + 16;  // + the junk slot
+    return lp_terms(precision) * ((size_t)2 * 4 * KT * 16 + (size_t)(OD + 1) * FR_XS * NT * 16) + 16;  // + the junk slot
 }
 
 // Tiles offered (x-plane blocks NB, dy-plane block groups KH, dy-plane blocks a wave KBW).
@@ -325,7 +444,7 @@ static void fa_rows_launch2(const Geom& g, const PlaneMap& m, const FaCfg& c, co
     // (5x5 dW: one dy block a wave, as the planner requires.)
 #define FR_CASE(NB_, KH_, KBW_)                                                                                  \
     case NB_ * 100 + KH_ * 10 + KBW_:                                                                           \
-        if constexpr (OD != 5 || KBW_ == 1)                                                                     \
+        if constexpr ((OD != 5 || KBW_ == 1) && (PREC != COGCONV_FP32 || (OD != 5 && KBW_ == 1 && NB_ < 4)))      \
             hipLaunchKernelGGL((k_fa_rows_lp<PREC, OD, KBW_, NB_, KH_>), grid, block, c.lds_bytes, s, g, m, c, x, dy, \
                                ws);                                                                              \
         break;
@@ -361,6 +480,7 @@ hipError_t launch_fa_rows_lp(int precision, const Geom& g, const PlaneMap& m, co
     const dim3 grid((unsigned)blocks);
     hipError_t e;
     switch (precision) {
+    case COGCONV_FP32: e = fa_rows_launch1<COGCONV_FP32>(g, m, c, x, dy, ws, s, grid); break;
     case COGCONV_BF16: e = fa_rows_launch1<COGCONV_BF16>(g, m, c, x, dy, ws, s, grid); break;
     case COGCONV_FP16: e = fa_rows_launch1<COGCONV_FP16>(g, m, c, x, dy, ws, s, grid); break;
     default: return hipErrorInvalidValue;

@@ -52,16 +52,10 @@ namespace cogconv {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int FR_RC = 16;  // planes of a staged chunk (one MFMA k slice)
-// Operands below this may lose bits of their last BF16 term (under 2^-126).
-constexpr float FR_SMALL = 0x1p-102f;
-
 // Whether every 32-pixel run of an output tile is a whole 128-byte line.
 __host__ __device__ __forceinline__ bool stream_rows(int OW, const float* out) {
     return (OW & 31) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0;
 }
-
-// BF16 terms of an operand.
-constexpr int fr_terms(int prec) { return prec == COGCONV_FP32 ? 3 : (prec == COGCONV_SPLIT_BF16 ? 2 : 1); }
 
 // How taps meet the staged samples.
 //   FR_UNIT  unit steps: output row r sees tap row i at staged row r + i.
@@ -93,16 +87,6 @@ struct FrameRows {
     static constexpr int LDS = 2 * T * NPIX * 16 + 16;          // and the tile's extreme magnitudes
 };
 
-// Splits x into T terms: term t rounds what the earlier ones left.
-template <int T, class E>
-__device__ __forceinline__ void split_terms(float x, E (&t)[T]) {
-#pragma unroll
-    for (int k = 0; k < T; k++) {
-        t[k] = (E)x;
-        if (k + 1 < T) x -= (float)t[k];
-    }
-}
-
 template <int PREC>
 __device__ __forceinline__ floatx16 fr_mfma(typename LpType<PREC>::V a, typename LpType<PREC>::V b, floatx16 c) {
     if constexpr (PREC == COGCONV_FP16)
@@ -111,21 +95,10 @@ __device__ __forceinline__ floatx16 fr_mfma(typename LpType<PREC>::V a, typename
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ unsigned wave_max(unsigned v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, d));
-    return v;
-}
-
-__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
-
-// Whether any lane's operands go under FR_SMALL; `least`: the smallest magnitude(x) - 1, which puts zeros last.
-__device__ __forceinline__ bool any_small(unsigned least) { return __any(least < __float_as_uint(FR_SMALL) - 1u); }
-
 // Packed bank: [32-plane output block][16-plane chunk][tap column j][tap row i][term][lane][8], where lane l
 // holds output plane l % 32 and input planes 8 (l / 32) .. + 7 (zeros past the planes), taps flipped for the
 // convolution orientation.  After it, for the FP32 plans, one uint2 a [block][chunk][j][i]: the fragment's largest
-// magnitude (bits), and whether it holds operands under FR_SMALL.
+// magnitude (bits), and whether it holds operands under LP_SMALL.
 template <int PREC, int T>
 __global__ void k_pack_rows(Geom g, PlaneMap m, int Mout, int chunks, long total, const float* __restrict__ Wt,
                             typename LpType<PREC>::T* __restrict__ Wp) {
@@ -218,7 +191,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
                                                          const typename LpType<PREC>::T* __restrict__ Wp,
                                                          float* __restrict__ O,
                                                          const cogconv_image_io* __restrict__ tab, Epi e) {
-    constexpr int T = fr_terms(PREC);
+    constexpr int T = lp_terms(PREC);
     typedef FrameRows<F, RW, S, T> Z;
     typedef typename LpType<PREC>::T E;
     typedef typename LpType<PREC>::V V;
@@ -341,7 +314,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         for (int i = 0; i < NT; i++)
 #pragma unroll
             for (int t = 0; t < T; t++) a[k][i][t] = fragment(DEEP ? lane * 16 + k * COLB : next_column(-1, F - 1), i, t);
-    // EXACT: whether the bank (smallW) and the tile (sRange[0]) hold operands under FR_SMALL.
+    // EXACT: whether the bank (smallW) and the tile (sRange[0]) hold operands under LP_SMALL.
     const uint2* range = reinterpret_cast<const uint2*>(Wp + (size_t)c.mTiles * chunks * F * F * T * 512) +
                          (size_t)mt * chunks * F * F;
     bool smallW = false;
@@ -577,7 +550,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     // reaches them as inf * 0 or inf - inf of its terms), and those so small that
     // products or terms under BF16's and FP32's normal range may matter to
     // them: each of the n products of a pair of operands loses at most 2^-123,
-    // and where the tile (the bank) holds operands under FR_SMALL, whose
+    // and where the tile (the bank) holds operands under LP_SMALL, whose
     // last term may be lost, 2^-125 of the bank's (the tile's) largest.
     float tiny = 0x1p-100f * (float)(chunks * FR_RC * F * F);
     if (EXACT) {
@@ -727,7 +700,7 @@ static constexpr int fr_key(int F, int RW, int MW, int S, int prec) { return (((
 size_t frame_rows_lds_bytes(int F, int RW, int MW, int S, int prec) {
     switch (fr_key(F, RW, MW, S, prec)) {
 #define FR_LDS(F, RW, MW, OCC, S, PREC) \
-    case fr_key(F, RW, MW, S, PREC): return FrameRows<F, RW, S, fr_terms(PREC)>::LDS;
+    case fr_key(F, RW, MW, S, PREC): return FrameRows<F, RW, S, lp_terms(PREC)>::LDS;
         FR_CASES(FR_LDS)
 #undef FR_LDS
     default: return 0;
@@ -735,7 +708,7 @@ size_t frame_rows_lds_bytes(int F, int RW, int MW, int S, int prec) {
 }
 
 size_t frame_rows_workspace_bytes(const IgemmCfg& c, int F, int prec) {
-    return (size_t)c.mTiles * (c.RC / FR_RC) * F * F * (fr_terms(prec) * 1024 + sizeof(uint2));
+    return (size_t)c.mTiles * (c.RC / FR_RC) * F * F * (lp_terms(prec) * 1024 + sizeof(uint2));
 }
 
 hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
@@ -751,7 +724,7 @@ hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const I
         switch (prec) {
 #define FR_PACK(PREC)                                                                                              \
     case PREC:                                                                                                     \
-        hipLaunchKernelGGL((k_pack_rows<PREC, fr_terms(PREC)>), grid, block, 0, s, g, m, c.Mout, c.RC / FR_RC, total, w, \
+        hipLaunchKernelGGL((k_pack_rows<PREC, lp_terms(PREC)>), grid, block, 0, s, g, m, c.Mout, c.RC / FR_RC, total, w, \
                            static_cast<LpType<PREC>::T*>(ws));                                                     \
         break;
             FR_PACK(COGCONV_FP32)
@@ -766,7 +739,7 @@ hipError_t launch_frame_rows(int prec, const Geom& g, const PlaneMap& m, const I
     }
     const dim3 grid((unsigned)blocks), block(256 * c.splits);
     const bool vec = c.vec4 && (tab ? x16 : (reinterpret_cast<uintptr_t>(x) & 15) == 0);
-    const size_t lds = c.lds_bytes + (own ? (size_t)g.FH * g.FW * fr_terms(prec) * 1024 : 0);
+    const size_t lds = c.lds_bytes + (own ? (size_t)g.FH * g.FW * lp_terms(prec) * 1024 : 0);
     const bool stream = !tab && stream_rows(g.OW, out);
     switch (fr_key(g.FH, c.MB, c.splits, c.variant, prec)) {
 #define FR_FORM(F, RW, MW, OCC, S, PREC, VEC, STREAM, OWN) \

@@ -290,7 +290,7 @@ hipError_t launch_fa_igemm_f32(const Geom& g, const PlaneMap& m, const FaCfg& c,
 hipError_t launch_reduce_partials(const float* ws, float* out, int splits, long total, long points, hipStream_t s,
                                   const Epi& e);
 size_t fa_igemm_lp_lds_bytes(const FaCfg& c, int OW, int precision);
-size_t fa_rows_lp_lds_bytes(const FaCfg& c, int OD);
+size_t fa_rows_lp_lds_bytes(const FaCfg& c, int OD, int precision);
 hipError_t launch_fa_rows_lp(int precision, const Geom& g, const PlaneMap& m, const FaCfg& c, const float* x,
                              const float* dy, float* out, float* ws, hipStream_t s, const Epi& ep);
 hipError_t launch_fa_igemm_lp(int precision, const Geom& g, const PlaneMap& m, const FaCfg& c, const float* x,

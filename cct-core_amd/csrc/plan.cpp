@@ -455,7 +455,7 @@ bool choose_fa_rows_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
                        int kbw = 0, int rowSplits = 0) {
     if (d->mode != COGCONV_FILTER_ADJOINT_BLOCK_REDUCE_SUM || d->border != COGCONV_BORDER_VALID || d->in0.dims != 2)
         return false;
-    if (d->precision != COGCONV_BF16 && d->precision != COGCONV_FP16) return false;
+    if (d->precision == COGCONV_SPLIT_BF16) return false;
     if (g.flip || g.upFr != 1 || g.upFc != 1 || g.upAr != 1 || g.upAc != 1 || g.dnR != 1 || g.dnC != 1) return false;
     if (g.OH != g.OW || (g.OH != 1 && g.OH != 3 && g.OH != 5)) return false;
     FaCfg c;
@@ -475,6 +475,8 @@ bool choose_fa_rows_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     const int sel = nb * 100 + kh * 10 + kbw;
     if (sel != 222 && sel != 221 && sel != 142 && sel != 141 && sel != 422 && sel != 421 && sel != 414) return false;
     if (g.OH == 5 && kbw != 1) return false;
+    // FP32: twice the accumulators (5x5 dW and larger tiles spill or lose a block a CU).
+    if (d->precision == COGCONV_FP32 && (g.OH == 5 || kbw != 1 || nb > 2)) return false;
     c.nb = nb;
     c.kh = kh;
     c.kbw = kbw;
@@ -496,7 +498,8 @@ bool choose_fa_rows_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     c.rowSplits = rowSplits;
     c.rowsPer = (g.FH + rowSplits - 1) / rowSplits;
     c.splits = m.B * c.chunks * rowSplits;
-    c.lds_bytes = fa_rows_lp_lds_bytes(c, g.OH);
+    c.lds_bytes = fa_rows_lp_lds_bytes(c, g.OH, d->precision);
+    if (c.lds_bytes > 160 * 1024) return false;
     *out = c;
     return true;
 }
@@ -663,6 +666,32 @@ double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
     return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
                   c.RC / 16.0 * (7 * g.dnR + g.FH) * (31 * g.dnC + g.FW));
+}
+
+// FP32 FilterAdjoint as split-BF16 products (k_fa_rows_lp): a launch floor, the
+// longer of one block's walk and the grid's at full load (in blocks of four waves
+// over 256 CUs), and the partials' writing and summing; and the FP32 MFMA kernel.
+// 139 measured calls (1x1 and 3x3, sides 24 to 256, log error 0.17 and 0.15 rms); at 0.8
+// of the other's estimate it takes 53 of 252 further calls, 1.42x faster on them (4
+// slower, at worst 0.69x), with 0.7 times the MFMA kernel's relative error.
+double fa_rows_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
+    const double points = (double)g.OH * g.OW, waves = c.nb * c.kh;
+    const double blocks = (double)c.nTiles * c.kTiles * c.splits * waves / 1024;
+    const double mfma = points * c.kbw * 6 * 16 / 2400.0;  // one wave's a row
+    const double staged = (c.kh * c.kbw * 16 * 32.0 + c.nb * 16 * 40.0) / waves / 64;
+    return 8.5 + std::max(c.rowsPer * (0.61 + 1.79 * mfma), blocks * (1.04 + c.rowsPer * (2.27 * mfma + 0.021 * staged + 0.11))) +
+           0.55e-6 * 4 * c.splits * c.K * m.N * points;
+}
+
+double fa_igemm_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
+    const double points = (double)g.OH * g.OW;
+    const int cw = std::min(c.CW, (g.FWe + 3) / 4 * 4), planes = std::min(m.N, (int)((16 * c.CBW + points - 1) / points) + 1);
+    const long chunks = (long)m.B * ((g.FHe + c.RR - 1) / c.RR) * ((g.FWe + c.CW - 1) / c.CW);
+    const double items = (double)((chunks + c.splits - 1) / c.splits);
+    const double mfma = (double)c.MB * c.CBW * c.RR * (cw / 4) * 32 / 4 / 2400.0;
+    const double staged = (c.RR * (double)c.K + (c.RR + g.OH - 1) * (double)planes) * cw * 4e-3;  // KB
+    return 5.3 + std::max(1.0, (double)c.colGroups * c.splits / 256) * items * (4.34 + 1.44 * mfma + 0.025 * staged) +
+           0.45e-6 * 4 * c.splits * c.K * m.N * points;
 }
 
 double up2q_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
@@ -1033,6 +1062,27 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     const bool igemm_ok = ig.MB > 0;
     FaCfg fa;
     const bool fa_ok = choose_fa_igemm(desc, g, m, &fa);
+    // FilterAdjoint as split-BF16 products, where estimated faster by more than the
+    // estimates' error; partials within the no-allocation launch's scratch array.
+    std::vector<FaCfg> fx;
+    int fx_first = -1;
+    static const int fx_tiles[][3] = {{2, 2, 1}, {1, 4, 1}};  // larger tiles: 0.7 to 0.95x these
+    for (const auto& t : fx_tiles) {  // of each tile the row split estimated best
+        FaCfg best;
+        bool any = false;
+        for (int rsp = 1; rsp <= 64; rsp *= 2) {
+            FaCfg c;
+            if (!choose_fa_rows_lp(desc, g, m, &c, t[0], t[1], t[2], rsp) ||
+                (size_t)c.splits * c.K * m.N * outPts * sizeof(float) > (64UL << 20))
+                continue;
+            if (!any || fa_rows_us(g, m, c) < fa_rows_us(g, m, best)) best = c;
+            any = true;
+        }
+        if (!any) continue;
+        if (fx_first < 0 || fa_rows_us(g, m, best) < fa_rows_us(g, m, fx[fx_first])) fx_first = (int)fx.size();
+        fx.push_back(best);
+    }
+    if (fx_first >= 0 && fa_ok && fa_rows_us(g, m, fx[fx_first]) > 0.8 * fa_igemm_us(g, m, fa)) fx_first = -1;
     const SmallCfg sm = choose_small(g, m);
     const DirectCfg dr = choose_direct(g, 4);
     DirectCfg drt[3];
@@ -1081,6 +1131,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     else if (upq_ok) add_up(upq);
     else if (up_ok) add_up(up);
     else if (igemm_ok) add(KK_IGEMM, nullptr, nullptr, &ig, nullptr);
+    else if (fx_first >= 0 && fa_ok) add(KK_FA_IGEMM_LP, nullptr, nullptr, nullptr, &fx[fx_first]);
     else if (fa_ok) add(KK_FA_IGEMM, nullptr, nullptr, nullptr, &fa);
     else if (small_out) add(KK_SMALL_OUTPUT, nullptr, &sm, nullptr, nullptr);
     else if (rt_ok) add(KK_DIRECT_RT, &drt[rt_first], nullptr, nullptr, nullptr);
@@ -1096,7 +1147,9 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
                 if (c.MB > 0) add(KK_IGEMM, nullptr, nullptr, &c, nullptr);
             }
     }
+    for (const FaCfg& c : fx) add(KK_FA_IGEMM_LP, nullptr, nullptr, nullptr, &c);
     if (fa_ok) {
+        add(KK_FA_IGEMM, nullptr, nullptr, nullptr, &fa);
         for (int cw : {0, 32, 16})
             for (int cbw : {3, 6, 9})
                 for (int parts : {128, 256, 512, 1024})
@@ -1160,7 +1213,8 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
     std::vector<Variant> vars;
     enumerate_variants(desc, g, m, vars);
     const auto offered = [&](int i) {
-        return !(serving && vars[i].kind == KK_FRAME_ROWS && desc->precision == COGCONV_FP32);
+        return !(serving && desc->precision == COGCONV_FP32 &&
+                 (vars[i].kind == KK_FRAME_ROWS || vars[i].kind == KK_FA_IGEMM_LP));
     };
     if (vars.empty())
         return fail(COGCONV_ERR_UNSUPPORTED,
@@ -1380,10 +1434,11 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
     }
     case KK_FA_IGEMM_LP: {
         static const char* pn[] = {"fp32", "bf16", "fp16", "split_bf16"};
+        static const char* rn[] = {"fa_igemm_f32x3", "fa_rows_bf16", "fa_rows_fp16", ""};
         if (plan->fcfg.rows) {
             const FaCfg& f = plan->fcfg;
-            snprintf(buf, len, "fa_rows_%s %s out=%dx%dx%d tile=%dx%d waves=%d chunks=%d rowsplits=%d splits=%d lds=%zu",
-                     pn[plan->desc.precision], mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW,
+            snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx%d waves=%d chunks=%d rowsplits=%d splits=%d lds=%zu",
+                     rn[plan->desc.precision], mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW,
                      f.kh * f.kbw * 16, f.nb * 16, f.nb * f.kh, f.chunks, f.rowSplits, f.splits, f.lds_bytes);
             break;
         }
