@@ -113,6 +113,9 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
     const int m0 = mt * MT;
     const int y0 = tr * 8 * g.dnR - g.hR;
     const int x0 = tc * 32 * g.dnC - g.hC;
+    // Read now, under the staging: fetched at the stores it costs a small launch a scalar load's latency.
+    int epiOps = e.n;
+    asm volatile("" : "+s"(epiOps));
     const int TRp = c.tileRows, TCp = c.tileCols;
     const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
     const int L = m.T / m.N;
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
     // With an epilogue every output takes the tile path, whose stores apply it
     // to values read back from LDS (16 images 64x64x16 -> 32, 3x3, bias and
     // rectifier: 23.6 us when the threads re-read their own global stores).
-    const bool vec = e.n == 0 && ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 3) == 0 &&
+    const bool vec = epiOps == 0 && ph.oStride == 1 && ((ph.OWf | ph.oCol0) & 3) == 0 &&
                      (reinterpret_cast<uintptr_t>(O) & 15) == 0;
     if (vec) {  // block-uniform
         floatx4* red4 = reinterpret_cast<floatx4*>(smem);  // [rw][MB][4][64]
@@ -269,7 +272,7 @@ __global__ __launch_bounds__(512) void k_igemm_f32(Geom g, PlaneMap m, IgemmCfg 
             for (int pb = 0; pb < 4; pb++) *tile(mb, pb) = acc[mb][pb] + *tile(mb, pb);
     }
     __syncthreads();
-    if (e.n) {
+    if (epiOps) {
         // Whole 32-column rows, eight elements of a thread per epilogue pass; four
         // where eight would take more registers than the rest of the kernel.
         const int col = tid & 31, ocol = tc * 32 + col;
