@@ -496,6 +496,8 @@ __device__ __forceinline__ void up2q_body(const Geom& g, const PlaneMap& m, cons
     const int m0 = mt * MT;
     const int y0 = tr * 8 - u.hU;
     const int x0 = tc * 32 - u.wU;
+    int epiOps = e.n;  // read now, under the staging
+    asm volatile("" : "+s"(epiOps));
     const int TRp = c.tileRows, TCp = c.tileCols;
     const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
     const int L = m.T / m.N;
@@ -587,7 +589,7 @@ __device__ __forceinline__ void up2q_body(const Geom& g, const PlaneMap& m, cons
     }
     // The epilogue rewrites the thread's own stores (still in L2), so the
     // accumulators above stay in registers whatever its code size.
-    if (e.n) {
+    if (epiOps) {
         for (int t = 0; t < MB * 4; t++) {
             const int mb = t >> 2, pb = t & 3;
             const int mm = m0 + mb * 16 + l16;
