@@ -1604,7 +1604,8 @@ extern "C" int cogconv_launch(cogconv_plan plan, const float* in0, const float* 
 }
 
 bool cogconv::plan_table_capable(const cogconv_plan_s* plan) {
-    return plan->kind == KK_IGEMM_LP || plan->kind == KK_FRAME_ROWS ||
+    // (An up-sampled plan takes no table whichever kernel it runs.)
+    return plan->kind == KK_IGEMM_LP || (plan->kind == KK_FRAME_ROWS && plan->g.upAr == 1) ||
            (plan->kind == KK_IGEMM && plan->m.mode != COGCONV_PLANE_BY_PLANE);
 }
 
