@@ -376,7 +376,8 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
         }
     if constexpr (EXACT) {
         // As in k_frame_rows: partials that are not finite, or so small that lost
-        // products or terms may matter, are summed again by FP32 multiply-adds.
+        // products or terms may matter (0 where small operands were staged, whose
+        // terms may all be lost), are summed again by FP32 multiply-adds.
         unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem);  // the last step ended with a barrier
         if (tid < 4) sRange[tid] = 0u;
         __syncthreads();
@@ -395,6 +396,7 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
         if (sRange[3]) bound += __uint_as_float(min(sRange[0], FINITE));
         if (sRange[2]) bound += __uint_as_float(min(sRange[1], FINITE));
         const float tiny = 0x1p-100f * 32.f * (float)max(run, 1) * bound;
+        const bool zeros = sRange[2] != 0 || sRange[3] != 0;
         float z = 0.f;
         bool redo = false;
 #pragma unroll
@@ -407,7 +409,7 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                     for (int v = 0; v < 4; v++) {
                         const float q = acc[kb][i][j][v];
                         z = fmaf(q, 0.f, z);
-                        redo |= fabsf(q) < tiny && q != 0.f;
+                        redo |= fabsf(q) < tiny && (q != 0.f || zeros);
                     }
         if (__any(redo || z != z)) {
             // Each thread reads back its own stores.
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                 if (k >= K || n >= N) continue;
                 float* o = out + ((size_t)k * N + n) * P + ij;
                 const float q = fabsf(*o);
-                if (q < __builtin_inff() && (q >= tiny || q == 0.f)) continue;
+                if (q < __builtin_inff() && (q >= tiny || (q == 0.f && !zeros))) continue;
                 const float* dp = DY + ((size_t)b * K + k) * dyH * dyW;
                 const float* xp = X + ((size_t)b * N + n) * H * W + ij % OD;
                 float sum = 0.f;

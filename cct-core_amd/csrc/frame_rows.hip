@@ -551,11 +551,15 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     // products or terms under BF16's and FP32's normal range may matter to
     // them: each of the n products of a pair of operands loses at most 2^-123,
     // and where the tile (the bank) holds operands under LP_SMALL, whose
-    // last term may be lost, 2^-125 of the bank's (the tile's) largest.
+    // last term may be lost, 2^-125 of the bank's (the tile's) largest.  Operands
+    // under 2^-134 lose every term, so where the tile or the bank holds small ones
+    // a sum of exactly 0 is such an output too (elsewhere it is a sum of zeros).
     float tiny = 0x1p-100f * (float)(chunks * FR_RC * F * F);
+    bool zeros = false;
     if (EXACT) {
         constexpr unsigned FINITE = 0x7f7fffffu;
         float bound = 1.f;
+        zeros = sRange[0] != 0 || (INLINE ? sRange[2] != 0 : __any(smallW));
         if (sRange[0]) {
             unsigned wMost = 0u;
             if (INLINE) {
@@ -585,7 +589,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
             for (int v = 0; v < 16; v++) {
                 acc[r][v] += low[EXACT ? r : 0][v];
                 z = fmaf(acc[r][v], 0.f, z);
-                redo |= fabsf(acc[r][v]) < tiny && acc[r][v] != 0.f;
+                redo |= fabsf(acc[r][v]) < tiny && (acc[r][v] != 0.f || zeros);
             }
     }
     if (e.n || __any(redo || z != z)) {  // wave-uniform
@@ -609,7 +613,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
             for (int k = 0; k < 8; k++) {
                 const int mm = m0 + mo0 + 8 * (k >> 2) + (k & 3);
                 const float a = fabsf(v[k]);
-                if (EXACT && mm < Mout && (!(a < __builtin_inff()) || (a < tiny && v[k] != 0.f))) again |= 1u << k;
+                if (EXACT && mm < Mout && (!(a < __builtin_inff()) || (a < tiny && (v[k] != 0.f || zeros)))) again |= 1u << k;
                 pl[k] = b * Mout + min(mm, Mout - 1);
                 pt[k] = prow * g.OW + pc;
             }

@@ -1,0 +1,75 @@
+"""The FP32 plans that run as split-BF16 products (igemm_f32x3, igemm_f32_up2x3 and
+fa_igemm_f32x3) on operands outside the split's range: subnormal ones, whose BF16
+terms all vanish, in every sampling the split forms take."""
+import numpy as np
+import pytest
+
+import cogconv._lib as L
+import oracle as O
+from gpuhelp import desc_pair, oracle_ref, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    L.init(0)
+    yield
+    L.synchronize()
+
+
+# (mode, border, sampling, step, filter): batch 1, 18 -> 34 planes, 20x40
+FORMS = {
+    "unit": (O.PF_BRS, O.CLAMP, O.NONE, 1, 5),
+    "up": (O.PF_BRS, O.ZERO, O.UP, 2, 5),
+    "down": (O.PF_BRS, O.CLAMP, O.DOWN, 2, 5),
+    "weight_grad": (O.FA_BRS, O.VALID, O.NONE, 1, 3),
+}
+N, K, H, W = 18, 34, 20, 40
+
+
+def split_plans(form):
+    """Descriptors, operand shapes and the split variants of a form."""
+    mode, border, sampling, step, F = FORMS[form]
+    xs = (N, H, W)
+    ws = (K, H - F + 1, W - F + 1) if mode == O.FA_BRS else (K * N, F, F)
+    od, cd = desc_pair(mode, border, O.XCORR, sampling, step, 1, xs, ws)
+    split = []
+    for v in range(L.variant_count(cd)):
+        p = L.Plan(cd, v)
+        if "x3 " in p.description:
+            split.append((v, p.description))
+        p.close()
+    assert split
+    return od, cd, xs, ws, split
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("sx,sw", [(1e-41, 1e30), (1e30, 1e-41), (1e-44, 1e36)])
+def test_operands_that_vanish_in_the_split(form, sx, sw):
+    """Operands under 2^-134 round to 0 as BF16, and so do their remainders: the
+    results, far from 0, are FP32 sums of them all the same."""
+    rng = np.random.default_rng(11)
+    od, cd, xs, ws, split = split_plans(form)
+    x = (rng.uniform(0.5, 1, xs) * sx).astype(np.float32)
+    w = (rng.uniform(0.5, 1, ws) * sw).astype(np.float32)
+    ref, mag = oracle_ref(od, x, w)
+    for v, name in split:
+        print("CASE vanishing", form, sx, sw, name, flush=True)
+        assert np.all(np.abs(run_gpu(cd, x, w, variant=v) - ref) <= 1e-5 * mag), name
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_vanishing_operands_beside_others(form):
+    """A field of zeros with subnormal samples in some columns and ordinary ones in
+    others: every output that only subnormal samples reach is their sum."""
+    rng = np.random.default_rng(12)
+    od, cd, xs, ws, split = split_plans(form)
+    x = np.zeros(xs, np.float32)
+    x[:, :, 3::16] = rng.uniform(0.5, 1, x[:, :, 3::16].shape) * 1e-41
+    x[:, 10:, 11::16] = rng.uniform(0.5, 1, x[:, 10:, 11::16].shape)
+    w = (rng.uniform(0.5, 1, ws) * 1e30).astype(np.float32)
+    ref, mag = oracle_ref(od, x, w)
+    for v, name in split:
+        print("CASE vanishing beside others", form, name, flush=True)
+        assert np.all(np.abs(run_gpu(cd, x, w, variant=v) - ref) <= 1e-5 * mag), name
