@@ -114,6 +114,7 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
     constexpr int P = OD * OD;
     constexpr int TM = lp_terms(PREC);  // BF16 terms of an operand
     constexpr bool EXACT = TM == 3;
+    static_assert(!EXACT || KBW == 1, "the FP32 redo sums one dy block a wave");
     extern __shared__ __attribute__((aligned(16))) unsigned char fr_smem[];
     constexpr int DT = 2 * 4 * KT * 8, XT = RB * FR_XS * NT * 8;  // elements of one term
     T* sD = reinterpret_cast<T*>(fr_smem);  // [terms][2][4][KT][8]: dy rows, double-buffered
@@ -356,6 +357,85 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
 #pragma unroll
                 for (int j = 0; j < OD; j++) acc[kb][i][j] += low[EXACT ? kb : 0][EXACT ? i : 0][EXACT ? j : 0];
     }
+    if constexpr (EXACT) {
+        // As in k_frame_rows: partials that are not finite, or so small that lost
+        // products or terms may matter (0 where small operands were staged, whose
+        // terms may all be lost), are summed again by FP32 MFMAs.
+        unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem);  // the last step ended with a barrier
+        if (tid < 4) sRange[tid] = 0u;
+        __syncthreads();
+        mostD = wave_max(mostD);
+        mostX = wave_max(mostX);
+        const bool smallD = any_small(leastD), smallX = any_small(leastX);
+        if (lane == 0) {
+            atomicMax(&sRange[0], mostD);
+            atomicMax(&sRange[1], mostX);
+            if (smallD) sRange[2] = 1u;
+            if (smallX) sRange[3] = 1u;
+        }
+        __syncthreads();
+        constexpr unsigned FINITE = 0x7f7fffffu;
+        float bound = 1.f;
+        if (sRange[3]) bound += __uint_as_float(min(sRange[0], FINITE));
+        if (sRange[2]) bound += __uint_as_float(min(sRange[1], FINITE));
+        float tiny = 0x1p-100f * 32.f * (float)max(run, 1) * bound;
+        const bool zeros = sRange[2] != 0 || sRange[3] != 0;
+        float z = 0.f;
+        bool redo = false;
+#pragma unroll
+        for (int kb = 0; kb < KBW; kb++)
+#pragma unroll
+            for (int i = 0; i < OD; i++)
+#pragma unroll
+                for (int j = 0; j < OD; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float q = acc[kb][i][j][v];
+                        z = fmaf(q, 0.f, z);
+                        redo |= fabsf(q) < tiny && (q != 0.f || zeros);
+                    }
+        if (__any(redo || z != z)) {  // wave-uniform
+            // 16 dy planes x 16 x planes by v_mfma_f32_16x16x4 on operands as they are in
+            // memory; lane group g4 holds pixels 8 g4 .. + 7 of the chunk's row, one a
+            // product.  Bound by the loads of 64 separate lines: 16 images 100x256, 22 -> 2
+            // planes, a tenth of the samples NaN, 158 us (1.36 ms with a lane summing each of
+            // its outputs by itself; 69 us without NaNs).
+#pragma unroll
+            for (int i = 0; i < OD; i++)
+#pragma unroll
+                for (int j = 0; j < OD; j++) low[0][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            const int k = kt * KT + kh * 16 + l16, n = nt * NT + nb * 16 + l16, p0 = x0 + 8 * g4;
+            const int left = min(x0 + 32, dyW) - p0;  // pixels from p0 on (past them, in the next row, 0 multiplies 0)
+            const int dOff = k < K ? 4 * (k * dyH * dyW + p0) : FR_OOB, xOff = n < N ? 4 * (n * H * W + p0) : FR_OOB;
+#pragma unroll 1
+            for (int y = yBeg; y < yEnd; y++) {
+                float d[8];
+                buffer_load_row<8>(dyr, dOff + 4 * y * dyW, 0, d);
+#pragma unroll
+                for (int i = 0; i < OD; i++) {
+                    float q[8 + OD - 1];
+                    buffer_load_row<8 + OD - 1>(xr, xOff + 4 * (y + i) * W, 0, q);
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+#pragma unroll
+                        for (int j = 0; j < OD; j++)
+                            low[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(e < left ? d[e] : 0.f, e < left ? q[e + j] : 0.f,
+                                                                               low[0][i][j], 0, 0, 0);
+                }
+            }
+            asm volatile("" : "+v"(tiny));  // (compared anew: the masks of the first comparison would spill)
+#pragma unroll
+            for (int i = 0; i < OD; i++)
+#pragma unroll
+                for (int j = 0; j < OD; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float a = acc[0][i][j][v];
+                        if (!(fabsf(a) < __builtin_inff()) || (fabsf(a) < tiny && (a != 0.f || zeros)))
+                            acc[0][i][j][v] = low[0][i][j][v];
+                    }
+        }
+    }
     // The split's partial: ws[s][k][n][i][j] (every (k, n, i, j) of the tile,
     // zeros for a block without rows).
     const size_t total = (size_t)K * N * P;
@@ -374,62 +454,6 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                     for (int j = 0; j < OD; j++) o[i * OD + j] = acc[kb][i][j][v];
             }
         }
-    if constexpr (EXACT) {
-        // As in k_frame_rows: partials that are not finite, or so small that lost
-        // products or terms may matter (0 where small operands were staged, whose
-        // terms may all be lost), are summed again by FP32 multiply-adds.
-        unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem);  // the last step ended with a barrier
-        if (tid < 4) sRange[tid] = 0u;
-        __syncthreads();
-        mostD = wave_max(mostD);
-        mostX = wave_max(mostX);
-        const bool smallD = any_small(leastD), smallX = any_small(leastX);
-        if (lane == 0) {
-            atomicMax(&sRange[0], mostD);
-            atomicMax(&sRange[1], mostX);
-            if (smallD) sRange[2] = 1u;
-            if (smallX) sRange[3] = 1u;
-        }
-        __syncthreads();
-        constexpr unsigned FINITE = 0x7f7fffffu;
-        float bound = 1.f;
-        if (sRange[3]) bound += __uint_as_float(min(sRange[0], FINITE));
-        if (sRange[2]) bound += __uint_as_float(min(sRange[1], FINITE));
-        const float tiny = 0x1p-100f * 32.f * (float)max(run, 1) * bound;
-        const bool zeros = sRange[2] != 0 || sRange[3] != 0;
-        float z = 0.f;
-        bool redo = false;
-#pragma unroll
-        for (int kb = 0; kb < KBW; kb++)
-#pragma unroll
-            for (int i = 0; i < OD; i++)
-#pragma unroll
-                for (int j = 0; j < OD; j++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const float q = acc[kb][i][j][v];
-                        z = fmaf(q, 0.f, z);
-                        redo |= fabsf(q) < tiny && (q != 0.f || zeros);
-                    }
-        if (__any(redo || z != z)) {
-            // Each thread reads back its own stores.
-#pragma unroll 1
-            for (int e = 0; e < KBW * 4 * P; e++) {
-                const int ij = e % P, k = kt * KT + (kh * KBW + e / P / 4) * 16 + 4 * g4 + e / P % 4;
-                if (k >= K || n >= N) continue;
-                float* o = out + ((size_t)k * N + n) * P + ij;
-                const float q = fabsf(*o);
-                if (q < __builtin_inff() && (q >= tiny || (q == 0.f && !zeros))) continue;
-                const float* dp = DY + ((size_t)b * K + k) * dyH * dyW;
-                const float* xp = X + ((size_t)b * N + n) * H * W + ij % OD;
-                float sum = 0.f;
-                for (int y = yBeg; y < yEnd; y++)
-                    for (int x = x0; x < min(x0 + 32, dyW); x++)
-                        sum = fmaf(dp[y * dyW + x], xp[(y + ij / OD) * W + x], sum);
-                *o = sum;
-            }
-        }
-    }
 }
 
 size_t fa_rows_lp_lds_bytes(const FaCfg& c, int OD, int precision) {

@@ -142,44 +142,6 @@ __global__ void k_pack_rows(Geom g, PlaneMap m, int Mout, int chunks, long total
     }
 }
 
-// One output element by plain FP32 multiply-adds, four planes a tap as in the FP32
-// MFMA kernel (taps off the field multiply 0, as everywhere else; no inserted zero
-// of an up-sampled field multiplies).
-__device__ __forceinline__ float frame_point(const Geom& g, const PlaneMap& m, const float* Xb, const float* Wt, int mm,
-                                             int orow, int ocol) {
-    const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
-    const int L = m.T / m.N, taps = g.FH * g.FW;
-    const bool up = g.upAr == 2;
-    float s = 0.f;
-    for (int r0 = 0; r0 < m.R; r0 += 4)
-        for (int i = 0; i < g.FH; i++)
-            for (int j = 0; j < g.FW; j++) {
-                int y = orow * g.dnR - g.hR + i, c = ocol * g.dnC - g.hC + j;
-                if (up) {
-                    if ((y | c) & 1) continue;
-                    y >>= 1;
-                    c >>= 1;
-                }
-                bool in = (unsigned)y < (unsigned)g.H && (unsigned)c < (unsigned)g.W;
-                if (g.border == COGCONV_BORDER_CYCLIC) {
-                    y %= g.H;
-                    y += y < 0 ? g.H : 0;
-                    c %= g.W;
-                    c += c < 0 ? g.W : 0;
-                    in = true;
-                } else if (g.border == COGCONV_BORDER_CLAMP) {
-                    y = min(max(y, 0), g.H - 1);
-                    c = min(max(c, 0), g.W - 1);
-                    in = true;
-                }
-                const int t = g.flip ? taps - 1 - (i * g.FW + j) : i * g.FW + j;
-                for (int r = r0; r < min(r0 + 4, m.R); r++)
-                    s = fmaf(Wt[(size_t)(bpf ? r * L + mm : mm * m.N + r) * taps + t],
-                             in ? Xb[((size_t)r * g.H + y) * g.W + c] : 0.f, s);
-            }
-    return s;
-}
-
 // VEC: 16-byte staging loads.  STORES: 0 picks the stores' cache policy at run time;
 // at four rows a wave, where the two forms side by side spill, 1 is the cached
 // and 2 the streamed one.
@@ -545,7 +507,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     auto out_col = [&](int q) __attribute__((always_inline)) {
         return NP * ocol0 + (Z::UP ? q / RW ^ pair ^ Z::P : 0);
     };
-    // Two kinds of outputs are computed again below, by plain FP32 multiply-adds:
+    // Two kinds of outputs are computed again below, by FP32 MFMAs:
     // non-finite ones (an infinite or NaN operand, or one that rounds to infinity,
     // reaches them as inf * 0 or inf - inf of its terms), and those so small that
     // products or terms under BF16's and FP32's normal range may matter to
@@ -580,19 +542,85 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         }
         tiny *= bound;
     }
-    float z = 0.f;
-    bool redo = false;
-    if (EXACT) {
+    if constexpr (EXACT) {
+        float z = 0.f;
+        bool redo = false;
 #pragma unroll
         for (int r = 0; r < NA; r++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                acc[r][v] += low[EXACT ? r : 0][v];
+                acc[r][v] += low[r][v];
                 z = fmaf(acc[r][v], 0.f, z);
                 redo |= fabsf(acc[r][v]) < tiny && (acc[r][v] != 0.f || zeros);
             }
+        if (__any(redo || z != z)) {  // wave-uniform
+            // The wave's outputs once more, v_mfma_f32_32x32x2 on operands as they are in
+            // memory, two planes a tap (taps off the field multiply 0, as everywhere else;
+            // no inserted zero of an up-sampled field multiplies).  A field masked with
+            // infinities brings every wave here.  Bound by the scattered filter loads (64 lines
+            // of L1 each, for NA rows): one 128x128 image, 32 -> 32 planes, 9x9, a tenth of the
+            // samples NaN, 144 us (5.7 ms with a lane summing each of its outputs by itself; 49
+            // us without NaNs).
+#pragma unroll
+            for (int r = 0; r < NA; r++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) low[r][v] = 0.f;
+            const int mm = m0 + l32;
+            const int aOff = mm < Mout ? (bpf ? mm : mm * m.N) * F * F * 4 + half * planeW : STAGE_OOB;
+            int co[F];  // byte offset of tap column j's sample in a row, of the lane's plane
+#pragma unroll
+            for (int j = 0; j < F; j++) {
+                const int x = Z::UP ? (2 * ocol0 + ((g.hC + j) & 1) - g.hC + j) >> 1 : Z::STEP * ocol0 - g.hC + j;
+                co[j] = stage_col_offset(g, x) + half * HW * 4;
+            }
+#pragma unroll 1
+            for (int r0 = 0; r0 < m.R; r0 += 2) {
+                const bool live = r0 + half < m.R;
+#pragma unroll 1
+                for (int i = 0; i < F; i++) {
+                    float w[F], a[F];
+                    const int row = (g.flip ? F - 1 - i : i) * F * 4;
+                    buffer_load_row<F>(fr, live ? aOff : STAGE_OOB, r0 * planeW + row, w);
+#pragma unroll
+                    for (int j = 0; j < F; j++) a[j] = g.flip ? w[F - 1 - j] : w[j];
+#pragma unroll
+                    for (int q = 0; q < NA; q++) {
+                        int y = Z::STEP * out_row(q) - g.hR + i;
+                        if (Z::UP && (y & 1)) continue;
+                        y = Z::UP ? y >> 1 : y;
+                        bool in = (unsigned)y < (unsigned)g.H;
+                        if (g.border == COGCONV_BORDER_CYCLIC) {
+                            y %= g.H;
+                            y += y < 0 ? g.H : 0;
+                            in = true;
+                        } else {
+                            in = in || g.border == COGCONV_BORDER_CLAMP;
+                            y = min(max(y, 0), g.H - 1);
+                        }
+                        float x[F];
+#pragma unroll
+                        for (int j = 0; j < F; j++)
+                            x[j] = buffer_load_f32(xr, in && live ? co[j] + 4 * y * g.W : STAGE_OOB, 4 * r0 * HW);
+#pragma unroll
+                        for (int j = 0; j < F; j++) {
+                            // The tap columns of the accumulator's column phase (out_col).
+                            if (Z::UP && ((g.hC + j) & 1) != ((q / RW ^ pair ^ Z::P) & 1)) continue;
+                            low[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], x[j], low[q], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+            asm volatile("" : "+v"(tiny));  // (compared anew: the masks of the first comparison would spill)
+#pragma unroll
+            for (int r = 0; r < NA; r++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float a = acc[r][v];
+                    if (!(fabsf(a) < __builtin_inff()) || (fabsf(a) < tiny && (a != 0.f || zeros))) acc[r][v] = low[r][v];
+                }
+        }
     }
-    if (e.n || __any(redo || z != z)) {  // wave-uniform
+    if (e.n) {
         // Eight planes of a row at a time in a runtime loop (16 spill registers at
         // three waves a SIMD).
 #pragma unroll 1
@@ -600,32 +628,19 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
             float v[8];
             int pl[8], pt[8];
             const int mo0 = 16 * (t & 1) + 4 * half;  // plane of v[k]: mo0 + 8 (k / 4) + k % 4
-            const int orow = out_row(t >> 1), ocol = out_col(t >> 1);
-            const int prow = min(orow, g.OH - 1), pc = min(ocol, g.OW - 1);
+            const int prow = min(out_row(t >> 1), g.OH - 1), pc = min(out_col(t >> 1), g.OW - 1);
 #pragma unroll
             for (int q = 0; q < 2 * NA; q++) {
                 if (q != t) continue;  // wave-uniform: the accumulators keep compile-time indexes
 #pragma unroll
                 for (int k = 0; k < 8; k++) v[k] = acc[q >> 1][8 * (q & 1) + k];
             }
-            unsigned again = 0;
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const int mm = m0 + mo0 + 8 * (k >> 2) + (k & 3);
-                const float a = fabsf(v[k]);
-                if (EXACT && mm < Mout && (!(a < __builtin_inff()) || (a < tiny && (v[k] != 0.f || zeros)))) again |= 1u << k;
-                pl[k] = b * Mout + min(mm, Mout - 1);
+                pl[k] = b * Mout + min(m0 + mo0 + 8 * (k >> 2) + (k & 3), Mout - 1);
                 pt[k] = prow * g.OW + pc;
             }
-            if (orow >= g.OH || ocol >= g.OW) again = 0;
-            while (again) {
-                const int k = __builtin_ctz(again);
-                again &= again - 1;
-                const float s = frame_point(g, m, Xb, Wt, m0 + mo0 + 8 * (k >> 2) + (k & 3), prow, pc);
-#pragma unroll
-                for (int q = 0; q < 8; q++) v[q] = q == k ? s : v[q];
-            }
-            if (e.n) epi_eval_n<8>(e, v, pl, pt);
+            epi_eval_n<8>(e, v, pl, pt);
 #pragma unroll
             for (int q = 0; q < 2 * NA; q++) {
                 if (q != t) continue;

@@ -19,6 +19,31 @@ __device__ __forceinline__ float buffer_load_f32(__amdgpu_buffer_rsrc_t r, int v
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vbytes, sbytes, 0));
 }
 
+// N floats in a row from one byte offset (4-byte alignment will do), 16 bytes a load.
+template <int N>
+__device__ __forceinline__ void buffer_load_row(__amdgpu_buffer_rsrc_t r, int vbytes, int sbytes, float (&v)[N]) {
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    typedef float floatx2 __attribute__((ext_vector_type(2)));
+    constexpr int W = N / 4 * 4;
+#pragma unroll
+    for (int k = 0; k < W; k += 4) {
+        const floatx4 q = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, vbytes + 4 * k, sbytes, 0));
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[k + e] = q[e];
+    }
+    if constexpr (N - W == 3) {
+        const auto q = __builtin_amdgcn_raw_buffer_load_b96(r, vbytes + 4 * W, sbytes, 0);
+#pragma unroll
+        for (int e = 0; e < 3; e++) v[W + e] = __uint_as_float(q[e]);
+    } else if constexpr (N - W == 2) {
+        const floatx2 q = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(r, vbytes + 4 * W, sbytes, 0));
+        v[W] = q[0];
+        v[W + 1] = q[1];
+    } else if constexpr (N - W == 1) {
+        v[W] = buffer_load_f32(r, vbytes + 4 * W, sbytes);
+    }
+}
+
 // Cache policy of the loads that stage input fields in the BF16 / FP16 frame
 // kernels and the FP32 FilterAdjoint: non-temporal (nt), so that the streamed
 // field does not push out of the L2 what every block re-reads (the packed

@@ -1,6 +1,9 @@
 """The FP32 plans that run as split-BF16 products (igemm_f32x3, igemm_f32_up2x3 and
 fa_igemm_f32x3) on operands outside the split's range: subnormal ones, whose BF16
-terms all vanish, in every sampling the split forms take."""
+terms all vanish, in every sampling the split forms take, and the time a field
+full of non-finite samples takes."""
+import time
+
 import numpy as np
 import pytest
 
@@ -73,3 +76,40 @@ def test_vanishing_operands_beside_others(form):
     for v, name in split:
         print("CASE vanishing beside others", form, name, flush=True)
         assert np.all(np.abs(run_gpu(cd, x, w, variant=v) - ref) <= 1e-5 * mag), name
+
+
+@pytest.mark.parametrize("mode,B,N,K,H,W,F", [
+    (O.PF_BRS, 1, 32, 32, 128, 128, 9),
+    (O.FA_BRS, 16, 22, 2, 100, 256, 3),
+])
+@pytest.mark.parametrize("value", (np.nan, -np.inf, np.finfo(np.float32).min))
+def test_masked_fields_keep_their_speed(mode, B, N, K, H, W, F, value):
+    """A tenth of the samples NaN, infinite or the lowest float: every output is
+    computed a second time, by the matrix cores as well (it took 117 and 20 times as
+    long when each lane summed its outputs by itself, and takes 3 now)."""
+    rng = np.random.default_rng(13)
+    x = rng.uniform(-1, 1, (B * N, H, W)).astype(np.float32)
+    ws = (B * K, H - F + 1, W - F + 1) if mode == O.FA_BRS else (K * N, F, F)
+    w = rng.uniform(-1, 1, ws).astype(np.float32)
+    _, cd = desc_pair(mode, O.VALID if mode == O.FA_BRS else O.CLAMP, O.XCORR, O.NONE, 1, B, x.shape, ws)
+    plan = L.Plan(cd)
+    assert "x3 " in plan.description
+    print("CASE masked field", value, plan.description, flush=True)
+    bw, bo = L.DeviceBuffer.from_array(w), L.DeviceBuffer(4 * int(np.prod(plan.out_shape)))
+    wk = L.DeviceBuffer(plan.workspace_bytes)
+    best = []
+    for a in (x, np.where(rng.random(x.shape) < 0.1, np.float32(value), x)):
+        ba = L.DeviceBuffer.from_array(a)
+        times = []
+        for _ in range(8):
+            L.synchronize()
+            start = time.perf_counter()
+            plan.launch(ba, bw, bo, wk)
+            L.synchronize()
+            times.append(time.perf_counter() - start)
+        best.append(min(times))
+        ba.close()
+    for b in (bw, bo, wk):
+        b.close()
+    plan.close()
+    assert best[1] <= 8 * best[0]
