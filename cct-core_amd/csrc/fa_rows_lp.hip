@@ -381,7 +381,7 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
         float tiny = 0x1p-100f * 32.f * (float)max(run, 1) * bound;
         const bool zeros = sRange[2] != 0 || sRange[3] != 0;
         float z = 0.f;
-        bool redo = false;
+        unsigned least = ~0u;  // the smallest magnitude but 0, as 2 bits - 1
 #pragma unroll
         for (int kb = 0; kb < KBW; kb++)
 #pragma unroll
@@ -392,9 +392,23 @@ __global__ __launch_bounds__(64 * NB * KH) void k_fa_rows_lp(Geom g, PlaneMap m,
                     for (int v = 0; v < 4; v++) {
                         const float q = acc[kb][i][j][v];
                         z = fmaf(q, 0.f, z);
-                        redo |= fabsf(q) < tiny && (q != 0.f || zeros);
+                        least = min(least, (__float_as_uint(q) << 1) - 1u);
                     }
-        if (__any(redo || z != z)) {  // wave-uniform
+        bool redo = z != z;
+        if (zeros || least < (__float_as_uint(tiny) << 1) - 1u) {
+#pragma unroll
+            for (int kb = 0; kb < KBW; kb++)
+#pragma unroll
+                for (int i = 0; i < OD; i++)
+#pragma unroll
+                    for (int j = 0; j < OD; j++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const float q = acc[kb][i][j][v];
+                            redo |= fabsf(q) < tiny && (q != 0.f || zeros);
+                        }
+        }
+        if (__builtin_expect(__any(redo), 0)) {  // wave-uniform
             // 16 dy planes x 16 x planes by v_mfma_f32_16x16x4 on operands as they are in
             // memory; lane group g4 holds pixels 8 g4 .. + 7 of the chunk's row, one a
             // product.  Bound by the loads of 64 separate lines: 16 images 100x256, 22 -> 2

@@ -544,16 +544,23 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     }
     if constexpr (EXACT) {
         float z = 0.f;
-        bool redo = false;
+        unsigned least = ~0u;  // the smallest magnitude but 0, as 2 bits - 1
 #pragma unroll
         for (int r = 0; r < NA; r++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 acc[r][v] += low[r][v];
                 z = fmaf(acc[r][v], 0.f, z);
-                redo |= fabsf(acc[r][v]) < tiny && (acc[r][v] != 0.f || zeros);
+                least = min(least, (__float_as_uint(acc[r][v]) << 1) - 1u);
             }
-        if (__any(redo || z != z)) {  // wave-uniform
+        bool redo = z != z;
+        if (zeros || least < (__float_as_uint(tiny) << 1) - 1u) {
+#pragma unroll
+            for (int r = 0; r < NA; r++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) redo |= fabsf(acc[r][v]) < tiny && (acc[r][v] != 0.f || zeros);
+        }
+        if (__builtin_expect(__any(redo), 0)) {  // wave-uniform
             // The wave's outputs once more, v_mfma_f32_32x32x2 on operands as they are in
             // memory, two planes a tap (taps off the field multiply 0, as everywhere else;
             // no inserted zero of an up-sampled field multiplies).  A field masked with
