@@ -353,9 +353,9 @@ int noalloc_setup(int device);
 // (tune.cpp): the tuned variant index for `desc` on the current device and the
 // description it had when it was timed.
 int plan_variant_count(const cogconv_desc* desc, int* count);
-// cogconv_plan_create for the serving loop: FP32 plans keep to the kernels
-// without a workspace, which its admission budget has no room set aside for,
-// and whose choice does not depend on how many requests are stacked.
+// cogconv_plan_create for the serving loop: FP32 plans are chosen as if the split-BF16
+// forms were not there, whose packed banks its admission budget has no room set
+// aside for, and which are chosen by how many requests are stacked.
 int plan_create_serving(const cogconv_desc* desc, cogconv_plan* plan);
 bool tune_cache_lookup(const cogconv_desc* desc, int* variant, std::string* name);
 

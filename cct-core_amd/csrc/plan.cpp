@@ -917,7 +917,9 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len);
 // The candidate configurations for `desc`, the heuristic choice first.  The
 // list depends on the descriptor only, so an index into it is a stable
 // autotuning result (the tuner also keeps the description to check it).
-void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap& m, std::vector<Variant>& out) {
+// `plain`: without the split-BF16 forms of FP32 (the serving loop).
+void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap& m, std::vector<Variant>& out,
+                        bool plain) {
     out.clear();
     const long outPts = (long)g.OH * g.OW;
     std::vector<std::string> seen;
@@ -1072,7 +1074,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         bool any = false;
         for (int rsp = 1; rsp <= 64; rsp *= 2) {
             FaCfg c;
-            if (!choose_fa_rows_lp(desc, g, m, &c, t[0], t[1], t[2], rsp) ||
+            if (plain || !choose_fa_rows_lp(desc, g, m, &c, t[0], t[1], t[2], rsp) ||
                 (size_t)c.splits * c.K * m.N * outPts * sizeof(float) > (64UL << 20))
                 continue;
             if (!any || fa_rows_us(g, m, c) < fa_rows_us(g, m, best)) best = c;
@@ -1099,7 +1101,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     bool rows_ok[3];
     int rows_first = -1;
     for (int i = 0; i < 3; i++) {
-        rows_ok[i] = choose_frame_rows(desc, g, m, &rows[i], i == 0 ? 1 : (i == 1 ? 2 : 8));
+        rows_ok[i] = !plain && choose_frame_rows(desc, g, m, &rows[i], i == 0 ? 1 : (i == 1 ? 2 : 8));
         if (!rows_ok[i]) continue;
         if (rows_first < 0 || frame_rows_us(desc, g, m, rows[i]) < frame_rows_us(desc, g, m, rows[rows_first]))
             rows_first = i;
@@ -1139,6 +1141,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     // Alternatives.
     for (int i = 0; i < 3; i++)
         if (rows_ok[i]) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[i], nullptr);
+    if (rows_first >= 0 && up_ok && !upq_ok) add_up(up);
     if (igemm_ok) {
         add(KK_IGEMM, nullptr, nullptr, &ig, nullptr);
         for (int mb : {4, 2, 1})
@@ -1189,6 +1192,9 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     if (fft_ok && !fft_first) add_fft(fc);
 }
 
+// Whether a plan of `desc` leaves the split-BF16 forms of FP32 out.
+bool plain_only(const cogconv_desc* desc, bool serving) { return serving && desc->precision == COGCONV_FP32; }
+
 bool kind_matches_algo(int kind, int algo) {
     switch (algo) {
     case COGCONV_ALGO_DIRECT: return kind == KK_DIRECT || kind == KK_DIRECT_RT || kind == KK_FFT;
@@ -1211,11 +1217,7 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
     int e = analyse(desc, &out, &g, &m);
     if (e) return e;
     std::vector<Variant> vars;
-    enumerate_variants(desc, g, m, vars);
-    const auto offered = [&](int i) {
-        return !(serving && desc->precision == COGCONV_FP32 &&
-                 (vars[i].kind == KK_FRAME_ROWS || vars[i].kind == KK_FA_IGEMM_LP));
-    };
+    enumerate_variants(desc, g, m, vars, plain_only(desc, serving));
     if (vars.empty())
         return fail(COGCONV_ERR_UNSUPPORTED,
                     "precision %d is offered for ProjectFrame/BackProjectFrame with block reduction on 2-D fields with "
@@ -1233,7 +1235,7 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
         if (desc->algo == COGCONV_ALGO_SMALL_OUTPUT && outPts > 4096)
             return fail(COGCONV_ERR_UNSUPPORTED, "small-output kernel needs an output plane of at most 4096 points");
         for (int i = 0; i < (int)vars.size() && pick < 0; i++)
-            if (kind_matches_algo(vars[i].kind, desc->algo) && offered(i)) pick = i;
+            if (kind_matches_algo(vars[i].kind, desc->algo)) pick = i;
         if (pick < 0)
             return fail(COGCONV_ERR_UNSUPPORTED,
                         "implicit GEMM needs a block-reduce frame mode with a square 1/3/5/7/9 filter on 2-D fields "
@@ -1241,10 +1243,9 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
                         "planes per image in dy");
     } else {
         pick = 0;
-        while (!offered(pick) && pick + 1 < (int)vars.size()) pick++;
         int tuned;
         std::string tunedName;
-        if (tune_cache_lookup(desc, &tuned, &tunedName) && tuned < (int)vars.size() && offered(tuned)) {
+        if (tune_cache_lookup(desc, &tuned, &tunedName) && tuned < (int)vars.size()) {
             // Accept the cached index only if it still names the same configuration.
             cogconv_plan_s tmp;
             std::memset(&tmp, 0, sizeof tmp);
@@ -1305,7 +1306,7 @@ int cogconv::plan_variant_count(const cogconv_desc* desc, int* count) {
     int e = analyse(desc, &out, &g, &m);
     if (e) return e;
     std::vector<Variant> vars;
-    enumerate_variants(desc, g, m, vars);
+    enumerate_variants(desc, g, m, vars, plain_only(desc, false));
     *count = (int)vars.size();
     return COGCONV_OK;
 }
