@@ -917,7 +917,8 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len);
 // The candidate configurations for `desc`, the heuristic choice first.  The
 // list depends on the descriptor only, so an index into it is a stable
 // autotuning result (the tuner also keeps the description to check it).
-// `plain`: without the split-BF16 forms of FP32 (the serving loop).
+// `plain`: without the split-BF16 forms of FP32 and the row-walking frame kernel,
+// as the implicit-GEMM hint asks and, for FP32, the serving loop.
 void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap& m, std::vector<Variant>& out,
                         bool plain) {
     out.clear();
@@ -1033,7 +1034,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         IgemmCfg fr[7];
         int n = 0, first = 0;
         for (const auto& f : forms)
-            if (choose_frame_rows(desc, g, m, &fr[n], f[0], f[1], f[2])) {
+            if (!plain && choose_frame_rows(desc, g, m, &fr[n], f[0], f[1], f[2])) {
                 if (frame_rows_us(desc, g, m, fr[n]) < frame_rows_us(desc, g, m, fr[first])) first = n;
                 n++;
             }
@@ -1192,8 +1193,10 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     if (fft_ok && !fft_first) add_fft(fc);
 }
 
-// Whether a plan of `desc` leaves the split-BF16 forms of FP32 out.
-bool plain_only(const cogconv_desc* desc, bool serving) { return serving && desc->precision == COGCONV_FP32; }
+// Whether a plan of `desc` leaves out the forms that enumerate_variants calls not plain.
+bool plain_only(const cogconv_desc* desc, bool serving) {
+    return desc->algo == COGCONV_ALGO_IMPLICIT_GEMM || (serving && desc->precision == COGCONV_FP32);
+}
 
 bool kind_matches_algo(int kind, int algo) {
     switch (algo) {
@@ -1201,7 +1204,7 @@ bool kind_matches_algo(int kind, int algo) {
     case COGCONV_ALGO_SMALL_OUTPUT: return kind == KK_SMALL_OUTPUT;
     case COGCONV_ALGO_IMPLICIT_GEMM:
         return kind == KK_IGEMM || kind == KK_FA_IGEMM || kind == KK_IGEMM_LP || kind == KK_FA_IGEMM_LP ||
-               kind == KK_IGEMM_UP || kind == KK_FRAME_ROWS;
+               kind == KK_IGEMM_UP;
     default: return true;
     }
 }
@@ -1408,13 +1411,14 @@ void describe_into(const cogconv_plan_s* plan, char* buf, size_t len) {
                  plan->icfg.vec4 ? " ld16" : "", plan->icfg.trg, plan->icfg.ring ? " ring" : "", plan->icfg.lds_bytes);
         break;
     }
-    case KK_FRAME_ROWS:
-    {
+    case KK_FRAME_ROWS: {
         static const char* const names[] = {"igemm_f32x3", "igemm_bf16x1", "igemm_fp16x1", "igemm_bf16x2"};
-        const char* name = g.upAr == 2 ? "igemm_f32_up2x3" : names[plan->desc.precision];
-        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d ring threads=%d%s%s lds=%zu",
-                 name, mode_name(plan->desc.mode), plan->m.nOut, g.OH, g.OW, 4 * plan->icfg.MB / g.upAr, plan->icfg.MB, 256 * plan->icfg.splits, plan->icfg.vec4 ? " ld16" : "",
-                 plan->icfg.ring ? " inline" : "", plan->icfg.lds_bytes);
+        const IgemmCfg& c = plan->icfg;
+        // Filters come through a ring of registers, or from the workgroup's own pack.
+        snprintf(buf, len, "%s %s out=%dx%dx%d tile=%dx32 rows=%d%s threads=%d%s%s lds=%zu",
+                 g.upAr == 2 ? "igemm_f32_up2x3" : names[plan->desc.precision], mode_name(plan->desc.mode), plan->m.nOut,
+                 g.OH, g.OW, 4 * c.MB / g.upAr, c.MB, c.ring ? "" : " ring", 256 * c.splits, c.vec4 ? " ld16" : "",
+                 c.ring ? " inline" : "", c.lds_bytes);
         break;
     }
     case KK_IGEMM_UP: {

@@ -93,7 +93,12 @@ enum {
     COGCONV_SPLIT_BF16 = 3 /* three-term x_hi*w_hi + x_hi*w_lo + x_lo*w_hi */
 };
 
-/* Kernel-family hint; COGCONV_ALGO_AUTO lets the plan (and its autotuner) pick. */
+/* Kernel-family hint; COGCONV_ALGO_AUTO lets the plan (and its autotuner) pick.
+ * FP32 under AUTO may take a form that computes each product as six products of
+ * BF16 terms (see cogconv_plan_describe: "x3"): on sums its error is below
+ * the FP32 kernels', but a single product may be off by two half-ulps where FP32
+ * multiplies round to one.  IMPLICIT_GEMM keeps to FP32 products for FP32 (and to
+ * the tiled kernel for BF16 / FP16 / split-BF16). */
 enum {
     COGCONV_ALGO_AUTO = 0,
     COGCONV_ALGO_DIRECT = 1,        /* LDS-tiled direct kernel, any op         */

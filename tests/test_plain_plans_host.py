@@ -1,5 +1,6 @@
-"""The plans the serving loop makes (no GPU): FP32 requests are planned as if the
-split-BF16 forms were not offered, which pack operand 2 into a workspace."""
+"""The plans that leave the split-BF16 forms of FP32 out (no GPU): the serving loop's,
+which has no workspace for a packed operand 2, and those under the implicit-GEMM
+hint, which asks for FP32 products."""
 import ctypes
 
 import pytest
@@ -51,3 +52,35 @@ def test_low_precision_requests_run_the_default_plan():
     plan = L.Plan(cd)
     assert serving_plan(cd) == (plan.description, plan.workspace_bytes)
     plan.close()
+
+
+@pytest.mark.parametrize("mode,border,sampling,step,N,K,side,F,prefix", [
+    (O.PF_BRS, O.ZERO, O.UP, 2, 32, 32, 256, 7, "igemm_f32_up2 "),
+    (O.PF_BRS, O.ZERO, O.NONE, 1, 64, 64, 96, 3, "igemm_f32 "),
+    (O.PF_BRS, O.CLAMP, O.DOWN, 2, 24, 40, 150, 5, "igemm_f32 "),
+    (O.FA_BRS, O.VALID, O.NONE, 1, 22, 2, 250, 3, "fa_igemm_f32 "),
+])
+def test_implicit_gemm_hint_keeps_fp32_products(mode, border, sampling, step, N, K, side, F, prefix):
+    ws = (K, side - F + 1, side - F + 1) if mode == O.FA_BRS else (K * N, F, F)
+    _, cd = desc_pair(mode, border, O.XCORR, sampling, step, 1, (N, side, side), ws, algo=L.ALGO_IMPLICIT_GEMM)
+    plan = L.Plan(cd)
+    assert plan.description.startswith(prefix), plan.description
+    plan.close()
+
+
+def test_implicit_gemm_hint_refuses_what_it_has_no_kernel_for():
+    _, cd = desc_pair(O.PF_BRS, O.CLAMP, O.XCORR, O.DOWN, 2, 1, (22, 128, 128), (16 * 22, 9, 9),
+                      algo=L.ALGO_IMPLICIT_GEMM)
+    with pytest.raises(L.CogconvError) as e:
+        L.Plan(cd)
+    assert e.value.status == L.ERR_UNSUPPORTED
+
+
+def test_register_ring_is_named_where_there_is_one():
+    _, cd = desc_pair(O.PF_BRS, O.ZERO, O.XCORR, O.NONE, 1, 1, (16, 64, 64), (32 * 16, 3, 3), precision=L.BF16)
+    names = []
+    for v in range(L.variant_count(cd)):
+        plan = L.Plan(cd, v)
+        names.append(plan.description)
+        plan.close()
+    assert all((" ring" in n) != (" inline" in n) for n in names) and any(" inline" in n for n in names)
