@@ -357,7 +357,8 @@ int plan_variant_count(const cogconv_desc* desc, int* count);
 // forms were not there, whose packed banks its admission budget has no room set
 // aside for, and which are chosen by how many requests are stacked.
 int plan_create_serving(const cogconv_desc* desc, cogconv_plan* plan);
-bool tune_cache_lookup(const cogconv_desc* desc, int* variant, std::string* name);
+// `plain`: the best of the candidates that plan_create_serving offers.
+bool tune_cache_lookup(const cogconv_desc* desc, bool plain, int* variant, std::string* name);
 
 }  // namespace cogconv
 

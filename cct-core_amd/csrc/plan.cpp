@@ -1248,23 +1248,37 @@ int make_plan(const cogconv_desc* desc, int vi, cogconv_plan* plan, bool serving
         pick = 0;
         int tuned;
         std::string tunedName;
-        if (tune_cache_lookup(desc, &tuned, &tunedName) && tuned < (int)vars.size()) {
-            // Accept the cached index only if it still names the same configuration.
-            cogconv_plan_s tmp;
-            std::memset(&tmp, 0, sizeof tmp);
-            tmp.desc = *desc;
-            tmp.g = g;
-            tmp.m = m;
-            tmp.kind = vars[tuned].kind;
-            tmp.dcfg = vars[tuned].d;
-            tmp.scfg = vars[tuned].s;
-            tmp.icfg = vars[tuned].i;
-            tmp.fcfg = vars[tuned].f;
-            tmp.ps = vars[tuned].ps;
-            tmp.fft = vars[tuned].fft;
-            char name[192];
-            describe_into(&tmp, name, sizeof name);
-            if (tunedName == name) pick = tuned;
+        if (tune_cache_lookup(desc, plain_only(desc, serving), &tuned, &tunedName)) {
+            // The candidate that the sample names, if there is one: by the sample's index
+            // where that holds (samples of another list, or of a library with other
+            // candidates, keep their meaning).
+            const auto named = [&](int i) {
+                cogconv_plan_s tmp;
+                std::memset(&tmp, 0, sizeof tmp);
+                tmp.desc = *desc;
+                tmp.g = g;
+                tmp.m = m;
+                tmp.kind = vars[i].kind;
+                tmp.dcfg = vars[i].d;
+                tmp.scfg = vars[i].s;
+                tmp.icfg = vars[i].i;
+                tmp.fcfg = vars[i].f;
+                tmp.ps = vars[i].ps;
+                tmp.fft = vars[i].fft;
+                char name[192];
+                describe_into(&tmp, name, sizeof name);
+                return tunedName == name;
+            };
+            const int n = (int)vars.size();
+            if (tuned < n && named(tuned)) {
+                pick = tuned;
+            } else {
+                for (int i = 0; i < n; i++)
+                    if (named(i)) {
+                        pick = i;
+                        break;
+                    }
+            }
         }
     }
     cogconv_plan p = new (std::nothrow) cogconv_plan_s;

@@ -11,6 +11,8 @@
 // or the sample used fewer steps than asked for (Profiler.scala:100-112).  The
 // cache is a text file, one sample per line:
 //   device <TAB> descriptor key <TAB> variant <TAB> avg_us <TAB> warmup <TAB> run <TAB> unix_ms <TAB> description
+// Where the fastest candidate is a form that the serving loop does not offer, the
+// fastest of those it does has a sample of its own, its key ending in " plain".
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -32,6 +34,13 @@ struct Sample {
     long long created_ms;
     std::string name;
 };
+
+const char* const PLAIN = " plain";
+
+// Forms that the serving loop does not offer (enumerate_variants).
+bool not_plain(const cogconv_plan_s* p) {
+    return p->desc.precision == COGCONV_FP32 && (p->kind == KK_FRAME_ROWS || p->kind == KK_FA_IGEMM_LP);
+}
 
 std::mutex g_mu;
 std::map<std::string, Sample> g_cache;  // key: device + '\t' + descriptor key
@@ -81,14 +90,15 @@ struct Ev {
 
 }  // namespace
 
-bool cogconv::tune_cache_lookup(const cogconv_desc* desc, int* variant, std::string* name) {
+bool cogconv::tune_cache_lookup(const cogconv_desc* desc, bool plain, int* variant, std::string* name) {
     {
         std::lock_guard<std::mutex> lk(g_mu);
         if (g_cache.empty()) return false;  // no device query while nothing was tuned
     }
     const std::string key = current_device_name() + "\t" + desc_key(desc);
     std::lock_guard<std::mutex> lk(g_mu);
-    auto it = g_cache.find(key);
+    auto it = plain ? g_cache.find(key + PLAIN) : g_cache.end();
+    if (it == g_cache.end()) it = g_cache.find(key);
     if (it == g_cache.end()) return false;
     *variant = it->second.variant;
     *name = it->second.name;
@@ -127,8 +137,11 @@ extern "C" int cogconv_autotune(const cogconv_desc* desc, const cogconv_tune_opt
         auto it = g_cache.find(key);
         if (it != g_cache.end()) {
             const Sample& s = it->second;
-            if (s.variant < count &&
-                (s.run > o.run_steps || (s.run == o.run_steps && s.warmup >= o.warmup_steps))) {
+            // (A sample without its plain one is of a library that did not keep it.)
+            const std::string kernel = s.name.substr(0, s.name.find(' '));
+            const bool split = kernel.size() > 2 && kernel.compare(kernel.size() - 2, 2, "x3") == 0;
+            const bool whole = s.variant < count && (!split || g_cache.count(key + PLAIN));
+            if (whole && (s.run > o.run_steps || (s.run == o.run_steps && s.warmup >= o.warmup_steps))) {
                 result->variant = s.variant;
                 result->avg_us = s.avg_us;
                 result->from_cache = 1;
@@ -171,8 +184,8 @@ extern "C" int cogconv_autotune(const cogconv_desc* desc, const cogconv_tune_opt
     if ((e = check_hip(hipEventCreate(&e0.e), "hipEventCreate")) ||
         (e = check_hip(hipEventCreate(&e1.e), "hipEventCreate")))
         return e;
-    int best = -1;
-    double bestUs = 0;
+    int best = -1, bestPlain = -1;
+    double bestUs = 0, bestPlainUs = 0;
     for (int i = 0; i < count; i++) {
         for (int w = 0; w < o.warmup_steps; w++) {
             e = cogconv_launch(plans[i], b0.f(), b1.f(), bo.f(), bw.p, stream);
@@ -197,12 +210,21 @@ extern "C" int cogconv_autotune(const cogconv_desc* desc, const cogconv_tune_opt
             best = i;
             bestUs = us;
         }
+        if (!not_plain(plans[i]) && (bestPlain < 0 || us < bestPlainUs)) {
+            bestPlain = i;
+            bestPlainUs = us;
+        }
     }
-    char name[192];
+    char name[192], plainName[192] = "";
     cogconv_plan_describe(plans[best], name, sizeof name);
+    if (bestPlain >= 0) cogconv_plan_describe(plans[bestPlain], plainName, sizeof plainName);
     {
         std::lock_guard<std::mutex> lk(g_mu);
         g_cache[key] = Sample{best, bestUs, o.warmup_steps, o.run_steps, now_ms(), name};
+        if (best == bestPlain || bestPlain < 0)
+            g_cache.erase(key + PLAIN);
+        else
+            g_cache[key + PLAIN] = Sample{bestPlain, bestPlainUs, o.warmup_steps, o.run_steps, now_ms(), plainName};
     }
     result->variant = best;
     result->avg_us = bestUs;
