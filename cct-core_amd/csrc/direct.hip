@@ -556,15 +556,21 @@ hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s) {
 }
 
 // Constant fill of n floats (the autotuner's synthetic inputs).
-__global__ void k_fill_value(float* __restrict__ p, size_t n, float v) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = v;
+// Uniform in [-1, 1), every bit of the fraction in use, from the element's index and the seed.
+__global__ void k_fill_varied(float* __restrict__ p, size_t n, unsigned seed) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        unsigned h = ((unsigned)i + seed) * 0x9e3779b9u;
+        h = (h ^ (h >> 15)) * 0x85ebca6bu;
+        h = (h ^ (h >> 13)) * 0xc2b2ae35u;
+        h ^= h >> 16;
+        p[i] = (float)(int)h * 0x1p-31f;
+    }
 }
 
-hipError_t launch_fill_value(float* p, size_t n, float v, hipStream_t s) {
+hipError_t launch_fill_varied(float* p, size_t n, unsigned seed, hipStream_t s) {
     if (n == 0) return hipSuccess;
     const size_t blocks = std::min<size_t>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_fill_value, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
+    hipLaunchKernelGGL(k_fill_varied, dim3((unsigned)blocks), dim3(256), 0, s, p, n, seed);
     return hipGetLastError();
 }
 

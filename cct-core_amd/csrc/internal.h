@@ -337,7 +337,7 @@ void* fft_state_new();
 void fft_release(void* state);
 int launch_fft(const Geom& g, const FftCfg& c, void** state, const float* x, const float* f, float* out, void* ws,
                hipStream_t s, const Epi& e);
-hipError_t launch_fill_value(float* p, size_t n, float v, hipStream_t s);
+hipError_t launch_fill_varied(float* p, size_t n, unsigned seed, hipStream_t s);
 
 // Request-table launches (plan.cpp): plans that take one, and the launch on a
 // table already in device memory (x16: every entry's operand 1 is 16-byte aligned).

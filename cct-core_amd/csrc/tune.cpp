@@ -3,8 +3,11 @@
 //
 // Counterpart of Profiler.bestVariant and ProfilerCache
 // (src/main/scala/cogx/runtime/execution/Profiler.scala:131-190, 49-130;
-// ProfilerCache.scala:39-122): candidates are timed on synthetic inputs (input
-// i of n filled with (i+1)/n, Profiler.scala:84-92), a flush buffer is written
+// ProfilerCache.scala:39-122): candidates are timed on synthetic inputs (uniform
+// in [-1, 1); the reference fills input i of n with (i+1)/n, Profiler.scala:84-92,
+// but the BF16 terms of such operands are zero but one, on which the matrix cores
+// draw less power: 9x9 FP32, 8 images 256x256x32, took 288 us on them in the forms of
+// 2 and of 8 rows a wave, where varied operands take 364 and 350), a flush buffer is written
 // before every timed step so that each step starts with cold caches
 // (Profiler.scala:80-83), the lowest average step time wins (ties keep the
 // earlier candidate), and a cached sample is reused unless profiling is forced
@@ -177,8 +180,8 @@ extern "C" int cogconv_autotune(const cogconv_desc* desc, const cogconv_tune_opt
         (e = check_hip(bw.alloc(ws), "hipMalloc (tuning workspace)")) ||
         (e = check_hip(bf.alloc((size_t)o.flush_bytes), "hipMalloc (cache flush buffer)")))
         return e;
-    if ((e = check_hip(launch_fill_value(b0.f(), n0, 0.5f, s), "tuning input fill")) ||
-        (e = check_hip(launch_fill_value(b1.f(), n1, 1.0f, s), "tuning input fill")))
+    if ((e = check_hip(launch_fill_varied(b0.f(), n0, 1u, s), "tuning input fill")) ||
+        (e = check_hip(launch_fill_varied(b1.f(), n1, 2u, s), "tuning input fill")))
         return e;
     Ev e0, e1;
     if ((e = check_hip(hipEventCreate(&e0.e), "hipEventCreate")) ||
