@@ -7,6 +7,7 @@
 //   Up/Down(1) -> NoSampling      src/main/scala/cogx/api/CogFunctionAPI.scala:1140-1144
 //   kernel routing                ConvolveHyperKernel.scala:1003-1148 (re-decided for gfx950, see choose_kernel)
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -615,30 +616,39 @@ bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, 
     return true;
 }
 
-// Estimated time (us) of one call: a launch floor, plus the longer of one block's
-// serial time and the whole grid's time at full load.  A chunk of planes costs its
-// staging and its MFMA time `mfma` (one wave's at 2.4 GHz); `px` staged pixels.
+// `last`: what the empty part of a partly filled last round of blocks counts for.
+double block_rounds(double blocks, double last) { return blocks + last * (std::ceil(blocks) - blocks); }
+
+// Estimated time (us) of one call: a launch floor, plus a soft maximum (a norm of
+// exponent `soft`) of one block's serial time and the whole grid's time at full load,
+// whose last, partly filled round counts for `last` of a full one.  A chunk of planes
+// costs its staging and its MFMA time `mfma` (one wave's at 2.4 GHz); `px` staged pixels;
+// `rough` blocks of 16 output planes stored element by element.
 struct CallTime {
-    double launch, chunk, mfma, block, mfmaLoad, pxLoad;
-    double us(double blocks, double chunks, double m, double px) const {
-        return launch + std::max(chunks * (chunk + mfma * m), blocks / 256 * (block + chunks * (mfmaLoad * m + pxLoad * px)));
+    double launch, chunk, mfma, block, mfmaLoad, pxLoad, last, soft, roughLoad;
+    double us(double blocks, double chunks, double m, double px, double rough = 0) const {
+        const double rounds = block_rounds(blocks / 256, last);
+        return launch + std::pow(std::pow(chunks * (chunk + mfma * m), soft) +
+                                     std::pow(rounds * (block + roughLoad * rough + chunks * (mfmaLoad * m + pxLoad * px)), soft),
+                                 1 / soft);
     }
 };
 
 // The constants fit calls measured on this card with operands from memory (sides 24
-// to 256, 3 to 64 planes, 1 to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log
-// error 0.1 to 0.14 rms).  FP32 against the MFMA kernel: the faster estimate is 2%
-// from always knowing the faster kernel, 1.14x the MFMA kernel on 250 calls (1.15x
-// with an output step of 2, 157 calls; 1.21x up-sampled, 300 calls).  BF16 / FP16 (500
-// calls): 2% from the best configuration; split-BF16 (260): 3%; packing in the kernel
-// where it is estimated faster gains another 1.07x and 1.10x.
+// to 256, 3 to 64 planes, 8 to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log
+// error 0.06 to 0.11 rms).  Each fit on half of the calls was judged on the others.
+// FP32 against the MFMA kernel, taken below 0.9 of its estimate: 357 of 650 calls,
+// 1.55x on them, none slower; with an output step of 2, 164 of 317, 1.45x, none slower;
+// up-sampled, below 0.85, 289 of 550, 1.58x, 6 of them slower, at worst 0.86x.  (The lines
+// lie where the losses end: at 1.0 of the estimates the first two have 13 more.)
+// BF16 / FP16 (1350 calls): 1.5% from the best configuration on average; split-BF16 (470): 1.4%.
 double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit[] = {{8.9, 1.24, 1.34, 0.02, 1.56, 0.0028},   // FP32
-                                   {6.6, 1.23, 2.10, 0.45, 1.18, 0.0034},   // BF16
-                                   {6.6, 1.23, 2.10, 0.45, 1.18, 0.0034},   // FP16
-                                   {6.6, 1.03, 1.61, 0.43, 1.35, 0.0027}};  // split-BF16
-    static const CallTime down = {6.9, 1.82, 2.82, 1.66, 3.48, 0.0005};
-    static const CallTime up = {8.6, 0.90, 1.69, 1.00, 1.41, 0.0045};
+    static const CallTime fit[] = {{7.46, 1.79, 1.15, 0.445, 1.46, 0.00273, 0.656, 3.07, 0},   // FP32
+                                   {6.17, 1.03, 1.91, 0.589, 1.10, 0.00313, 0.517, 1.63, 0},   // BF16
+                                   {6.17, 1.03, 1.91, 0.589, 1.10, 0.00313, 0.517, 1.63, 0},   // FP16
+                                   {6.20, 1.25, 1.28, 0.396, 1.08, 0.00325, 0.682, 2.64, 0}};  // split-BF16
+    static const CallTime down = {6.83, 2.33, 2.36, 0.668, 2.86, 0.00184, 0.520, 5.55, 0};
+    static const CallTime up = {7.49, 1.42, 1.63, 1.26, 1.33, 0.00633, 0.609, 4.56, 0};
     const double products = d->precision == COGCONV_FP32 ? 6 : (d->precision == COGCONV_SPLIT_BF16 ? 3 : 1);
     const double mfma = g.FH * g.FW * c.MB * products * 32 / 2400.0;  // 32 cycles each
     if (g.upAr == 2)  // half the taps a wave, half the waves' rows a block
@@ -648,8 +658,8 @@ double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, co
         return down.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
                        (8.0 * c.MB - 2 + g.FH) * (62 + g.FW));
     // A workgroup that packs its own filters: one launch, its staging in the chunk.
-    static const CallTime lpInline = {3.7, 0.16, 8.93, 0.36, 4.55, 0.0007},
-                          splitInline = {3.7, 0.78, 3.01, 0.10, 1.88, 0.0018};
+    static const CallTime lpInline = {2.96, 0.187, 7.95, 0.540, 2.14, 0.00111, 0.813, 1.62, 0},
+                          splitInline = {2.91, 1.52, 2.27, 0.445, 1.85, 0.00115, 0.654, 1.96, 0};
     if (c.ring)
         return (products == 3 ? splitInline : lpInline)
             .us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
@@ -661,7 +671,8 @@ double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, co
 }
 
 double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime unit = {4.3, 1.32, 2.40, 1.13, 2.52, 0.0052}, down = {3.7, 1.93, 3.11, 2.19, 2.84, 0.0038};
+    static const CallTime unit = {2.26, 1.05, 0.233, 1.90, 2.28, 0.00255, 0.896, 0.974, 0},
+                          down = {3.69, 2.07, 2.63, 1.23, 2.67, 0.00322, 0.729, 5.14, 0};
     const CallTime& fit = g.dnR == 2 ? down : unit;
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
     return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
@@ -671,16 +682,16 @@ double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
 // FP32 FilterAdjoint as split-BF16 products (k_fa_rows_lp): a launch floor, the
 // longer of one block's walk and the grid's at full load (in blocks of four waves
 // over 256 CUs), and the partials' writing and summing; and the FP32 MFMA kernel.
-// 139 measured calls (1x1 and 3x3, sides 24 to 256, log error 0.17 and 0.15 rms); at 0.8
-// of the other's estimate it takes 53 of 252 further calls, 1.42x faster on them (4
-// slower, at worst 0.69x), with 0.7 times the MFMA kernel's relative error.
+// 520 measured calls (1x1 and 3x3, sides 24 to 256, log error 0.05 and 0.11 rms, each half
+// judged by the other's fit); at 0.8 of the other's estimate it takes 172 of them, 1.46x
+// faster on them and none slower by 3% (first at 0.9: 0.94x), with 0.7 times the MFMA
+// kernel's relative error.
 double fa_rows_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
     const double points = (double)g.OH * g.OW, waves = c.nb * c.kh;
-    const double blocks = (double)c.nTiles * c.kTiles * c.splits * waves / 1024;
+    const double rounds = block_rounds((double)c.nTiles * c.kTiles * c.splits * waves / 1024, 0.88);
     const double mfma = points * c.kbw * 6 * 16 / 2400.0;  // one wave's a row
-    const double staged = (c.kh * c.kbw * 16 * 32.0 + c.nb * 16 * 40.0) / waves / 64;
-    return 8.5 + std::max(c.rowsPer * (0.61 + 1.79 * mfma), blocks * (1.04 + c.rowsPer * (2.27 * mfma + 0.021 * staged + 0.11))) +
-           0.55e-6 * 4 * c.splits * c.K * m.N * points;
+    return 7.88 + std::max(c.rowsPer * (0.488 + 1.96 * mfma), rounds * (0.49 + c.rowsPer * (1.45 * mfma + 0.354))) +
+           0.832e-6 * 4 * c.splits * c.K * m.N * points;
 }
 
 double fa_igemm_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
@@ -690,15 +701,16 @@ double fa_igemm_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
     const double items = (double)((chunks + c.splits - 1) / c.splits);
     const double mfma = (double)c.MB * c.CBW * c.RR * (cw / 4) * 32 / 4 / 2400.0;
     const double staged = (c.RR * (double)c.K + (c.RR + g.OH - 1) * (double)planes) * cw * 4e-3;  // KB
-    return 5.3 + std::max(1.0, (double)c.colGroups * c.splits / 256) * items * (4.34 + 1.44 * mfma + 0.025 * staged) +
-           0.45e-6 * 4 * c.splits * c.K * m.N * points;
+    const double rounds = block_rounds((double)c.colGroups * c.splits / 256, 0.59);
+    return 7.23 + items * std::max(2.92 + 1.26 * mfma + 0.0259 * staged, rounds * (3.67 + 0.93 * mfma + 0.0457 * staged)) +
+           0.886e-6 * 4 * c.splits * c.K * m.N * points;
 }
 
 double up2q_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit = {4.8, 1.25, 2.75, 2.78, 3.04, 0.0022};
+    static const CallTime fit = {1.31, 0.683, 0.142, 2.75, 2.05, 0.0029, 0.737, 0.62, 4.61};
     const double mfma = c.MB * g.FH * g.FW / 2.0 * (c.RC / 4) * 4 * 32 / 2400.0;
     return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
-                  c.RC / 16.0 * c.tileRows * c.tileCols);
+                  c.RC / 16.0 * c.tileRows * c.tileCols, g.OW % 4 ? c.MB : 0);  // 16-byte stores need aligned rows
 }
 
 SmallCfg choose_small(const Geom& g, const PlaneMap& m, long blocks = 4096) {
@@ -1024,9 +1036,11 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         IgemmCfg lp;
         if (!choose_igemm_lp(desc, g, m, &lp)) return;
         // k_frame_rows wherever it is built (3x3 to 9x9, unit steps, its offsets in 31
-        // bits): faster than k_igemm_lp in 97% of 650 measured calls, 1.5x on average
-        // and at most 1.25x slower.  One kernel's configurations only, so that
-        // candidates agree bit for bit.
+        // bits): on 1350 calls, many of them small, 1.55x k_igemm_lp on average; 57
+        // slower by more than 3%, at worst 0.76x (5x5 and 9x9 with at most 16 outputs and 17 to 32
+        // planes, 10 to 20 us, where half of a 32-output block idles).  One kernel's
+        // configurations only, so that candidates, batches and stacked requests
+        // agree bit for bit; the implicit-GEMM hint takes k_igemm_lp.
         // Rows a wave, output blocks a workgroup, filters packed in the kernel (two blocks for 3x3 BF16 / FP16: each
         // pixel staged once for 64 outputs, 64 -> 64 planes, 32 images 128x128
         // 101 -> 85 us; 5x5 122 -> 117, split-BF16 level, not built).
@@ -1097,7 +1111,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         while (rt_first < 2 && (long)drt[rt_first].tilesR * drt[rt_first].tilesC * m.nOut < 512) rt_first++;
     }
     // The split-BF16 frame kernel where it is estimated faster than the FP32 MFMA
-    // one by more than the estimates' own error at the crossing (5%).
+    // one by more than the estimates' own error at the crossing (frame_rows_us).
     IgemmCfg rows[3];
     bool rows_ok[3];
     int rows_first = -1;
@@ -1108,7 +1122,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
             rows_first = i;
     }
     if (rows_first >= 0 && igemm_ok &&
-        frame_rows_us(desc, g, m, rows[rows_first]) > 0.95 * igemm_frame_us(g, m, ig))
+        frame_rows_us(desc, g, m, rows[rows_first]) > 0.9 * igemm_frame_us(g, m, ig))
         rows_first = -1;
     PhaseSet up;
     const bool up_ok = choose_igemm_up(desc, g, m, &up);
@@ -1127,7 +1141,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     PhaseSet upq = up;
     const bool upq_ok = up_ok && (choose_igemm_up2q(g, m, up, &upq.f, 1, 0, 80 * 1024, true) ||
                                   choose_igemm_up2q(g, m, up, &upq.f));
-    if (rows_first >= 0 && upq_ok && frame_rows_us(desc, g, m, rows[rows_first]) > 0.9 * up2q_us(g, m, upq.f.c))
+    if (rows_first >= 0 && upq_ok && frame_rows_us(desc, g, m, rows[rows_first]) > 0.85 * up2q_us(g, m, upq.f.c))
         rows_first = -1;
     if (fft_first) add_fft(fc);
     else if (rows_first >= 0) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[rows_first], nullptr);
