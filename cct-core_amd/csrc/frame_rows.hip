@@ -159,6 +159,7 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     typedef typename LpType<PREC>::V V;
     constexpr int TC = Z::TC, NPIX = Z::NPIX, NP = Z::NP, NA = NP * RW, NT = Z::taps(0);
     constexpr bool EXACT = T == 3;  // FP32 results
+    static_assert(!EXACT || (!INLINE && MW == 1), "the redo's bounds are those of one packed output block");
     extern __shared__ __attribute__((aligned(16))) unsigned char fr_smem[];
     unsigned* sRange = reinterpret_cast<unsigned*>(fr_smem + 2 * T * NPIX * 16);
 
@@ -281,9 +282,8 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
                          (size_t)mt * chunks * F * F;
     bool smallW = false;
     if (EXACT) {
-        if (!INLINE)
-            for (int i = lane; i < chunks * F * F; i += 64) smallW |= range[i].y != 0;
-        if (tid < 4) sRange[tid] = 0u;
+        for (int i = lane; i < chunks * F * F; i += 64) smallW |= range[i].y != 0;
+        if (tid < 2) sRange[tid] = 0u;
         __syncthreads();  // before the first chunk's stores
     }
 
@@ -420,7 +420,6 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     // order of the filters in memory); FB units of a thread at a time.
     constexpr int FN = F * F * 64, FU = (FN + NTH - 1) / NTH, FB = FU <= 3 ? FU : 4;
     float fv[INLINE ? FB : 1][8];
-    unsigned mostW = 0u;
     const bool bpf = m.mode == COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM;
     const int planeW = (bpf ? m.T / m.N : 1) * F * F * 4;  // bytes between an output's planes
     const __amdgpu_buffer_rsrc_t fr = buffer_rsrc(Wt, (uint32_t)m.T * F * F * 4u);
@@ -438,7 +437,6 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
         }
     };
     auto store_filters = [&](int k0) __attribute__((always_inline)) {
-        unsigned least = ~0u;
 #pragma unroll
         for (int k = 0; k < FB; k++) {
             const int u = tid + NTH * (k0 + k);
@@ -448,10 +446,6 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const float w = fv[INLINE ? k : 0][q];
-                if (EXACT) {
-                    mostW = max(mostW, magnitude(w));
-                    least = min(least, magnitude(w) - 1u);
-                }
                 E t3[T];
                 split_terms<T>(w, t3);
 #pragma unroll
@@ -461,7 +455,6 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
             for (int e = 0; e < T; e++)
                 *reinterpret_cast<V*>(sFilt + ((pos % F * F + pos / F) * T + e) * FRAG + u / (F * F) * 16) = s[e];
         }
-        if (EXACT && any_small(least) && lane == 0) sRange[2] = 1u;
     };
     if (AHEAD) load(0, 0, 0);
     if (INLINE && FB == FU) load_filters(0, 0);
@@ -521,20 +514,14 @@ __global__ __launch_bounds__(256 * MW, OCC) void k_frame_rows(Geom g, PlaneMap m
     if (EXACT) {
         constexpr unsigned FINITE = 0x7f7fffffu;
         float bound = 1.f;
-        zeros = sRange[0] != 0 || (INLINE ? sRange[2] != 0 : __any(smallW));
+        smallW = __any(smallW);  // the same in every wave
+        zeros = sRange[0] != 0 || smallW;
         if (sRange[0]) {
             unsigned wMost = 0u;
-            if (INLINE) {
-                mostW = wave_max(mostW);
-                if (lane == 0) atomicMax(&sRange[3], mostW);
-                __syncthreads();
-                wMost = sRange[3];
-            } else {
-                for (int i = lane; i < chunks * F * F; i += 64) wMost = max(wMost, range[i].x);
-            }
+            for (int i = lane; i < chunks * F * F; i += 64) wMost = max(wMost, range[i].x);
             bound += __uint_as_float(min(wave_max(wMost), FINITE));
         }
-        if (INLINE ? sRange[2] != 0 : __any(smallW)) {  // the same in every wave
+        if (smallW) {
             most = wave_max(most);
             if (lane == 0) atomicMax(&sRange[1], most);
             __syncthreads();
