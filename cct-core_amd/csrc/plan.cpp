@@ -623,68 +623,88 @@ double block_rounds(double blocks, double last) { return blocks + last * (std::c
 // exponent `soft`) of one block's serial time and the whole grid's time at full load,
 // whose last, partly filled round counts for `last` of a full one.  A chunk of planes
 // costs its staging and its MFMA time `mfma` (one wave's at 2.4 GHz); `px` staged pixels;
-// `rough` blocks of 16 output planes stored element by element.
+// `rough` output blocks stored in rows that are not 16-byte aligned.
 struct CallTime {
-    double launch, chunk, mfma, block, mfmaLoad, pxLoad, last, soft, roughLoad;
-    double us(double blocks, double chunks, double m, double px, double rough = 0) const {
-        const double rounds = block_rounds(blocks / 256, last);
-        return launch + std::pow(std::pow(chunks * (chunk + mfma * m), soft) +
-                                     std::pow(rounds * (block + roughLoad * rough + chunks * (mfmaLoad * m + pxLoad * px)), soft),
-                                 1 / soft);
+    double launch, chunk, mfma, block, mfmaLoad, pxLoad, last, soft, roughLoad, rough;
+    double us(double blocks, double chunks, double m, double px, double ua = 0) const {
+        const double serial = chunks * (chunk + mfma * m) + rough * ua;
+        const double loaded =
+            block_rounds(blocks / 256, last) * (block + roughLoad * ua + chunks * (mfmaLoad * m + pxLoad * px));
+        return launch + std::pow(std::pow(serial, soft) + std::pow(loaded, soft), 1 / soft);
     }
 };
 
+// Row of a table by filter size, 3x3 to 9x9.
+const CallTime& by_filter(const CallTime (&fit)[4], const Geom& g) { return fit[std::min(std::max((g.FH - 3) / 2, 0), 3)]; }
+
 // The constants fit calls measured on this card with operands from memory (sides 24
 // to 256, 3 to 64 planes, 8 to 64 outputs, batches 1 to 32, filters 3x3 to 9x9; log
-// error 0.06 to 0.11 rms).  Each fit on half of the calls was judged on the others.
-// FP32 against the MFMA kernel, taken below 0.9 of its estimate: 357 of 650 calls,
-// 1.55x on them, none slower; with an output step of 2, 164 of 317, 1.45x, none slower;
-// up-sampled, below 0.85, 289 of 550, 1.58x, 6 of them slower, at worst 0.86x.  (The lines
-// lie where the losses end: at 1.0 of the estimates the first two have 13 more.)
-// BF16 / FP16 (1350 calls): 1.5% from the best configuration on average; split-BF16 (470): 1.4%.
+// error 0.02 to 0.09 rms by filter size in FP32, 0.07 to 0.11 below).  Each fit on half of
+// the calls was judged on the others.  FP32 against the MFMA kernel, taken below 0.97 of
+// its estimate: 421 of 650 calls, none slower by 3%; with an output step of 2, 184 of 317,
+// none; up-sampled, below 0.92, 327 of 550, 11 slower, at worst 0.86x.  (At 1.0, 4, 1 and
+// 22 are slower; at 0.85 the calls left to the MFMA kernels lose 2%.)
+// BF16 / FP16 (1350 calls): 1.0% from the best form on average; split-BF16 (470): 1.4%.
 double frame_rows_us(const cogconv_desc* d, const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit[] = {{7.46, 1.79, 1.15, 0.445, 1.46, 0.00273, 0.656, 3.07, 0},   // FP32
-                                   {6.17, 1.03, 1.91, 0.589, 1.10, 0.00313, 0.517, 1.63, 0},   // BF16
-                                   {6.17, 1.03, 1.91, 0.589, 1.10, 0.00313, 0.517, 1.63, 0},   // FP16
-                                   {6.20, 1.25, 1.28, 0.396, 1.08, 0.00325, 0.682, 2.64, 0}};  // split-BF16
-    static const CallTime down = {6.83, 2.33, 2.36, 0.668, 2.86, 0.00184, 0.520, 5.55, 0};
-    static const CallTime up = {7.49, 1.42, 1.63, 1.26, 1.33, 0.00633, 0.609, 4.56, 0};
+    static const CallTime unit[4] = {{6.85, 1.12, 1.88, 0.636, 1.93, 0.000535, 0.493, 2.63, 0, 0},
+                                     {7.28, 3.21, 0.775, 0.384, 1.03, 0.00627, 0.698, 3.09, 0.044, 0},
+                                     {6.83, 1.94, 0.382, 0.701, 0.701, 0.0107, 0.801, 1.10, 0, 0},
+                                     {8.09, 7.23, 0.306, 0.048, 1.04, 0.0094, 0.866, 2.08, 0.263, 0.0553}};
+    // (9x9 with an output step, which the MFMA kernel does not take, as 7x7.)
+    static const CallTime down[4] = {{6.67, 1.97, 3.19, 0.655, 2.03, 0.00307, 0.616, 7.84, 0, 0.0171},
+                                     {7.00, 1.09, 2.62, 0.115, 2.11, 0.00259, 0.562, 4.06, 0, 0},
+                                     {6.06, 0.154, 0.0845, 1.49, 2.59, 0.00359, 0.935, 1.0, 0.122, 0},
+                                     {6.06, 0.154, 0.0845, 1.49, 2.59, 0.00359, 0.935, 1.0, 0.122, 0}};
+    static const CallTime up[4] = {{7.55, 0.941, 2.43, 1.31, 2.98, 0, 0.495, 5.51, 0.0443, 0.0411},
+                                   {7.31, 1.86, 1.51, 1.07, 2.06, 0, 0.595, 4.57, 0.123, 0.239},
+                                   {7.36, 3.17, 1.04, 1.24, 1.65, 0.00121, 0.611, 4.22, 0, 0.0354},
+                                   {7.62, 2.97, 1.32, 1.31, 1.22, 0.00908, 0.662, 5.18, 0, 0.0315}};
+    static const CallTime lp = {6.17, 1.03, 1.91, 0.589, 1.10, 0.00313, 0.517, 1.63, 0, 0},
+                          split = {6.20, 1.25, 1.28, 0.396, 1.08, 0.00325, 0.682, 2.64, 0, 0};
+    // A workgroup that packs its own filters: one launch, its staging in the chunk.
+    static const CallTime lpInline = {2.96, 0.187, 7.95, 0.540, 2.14, 0.00111, 0.813, 1.62, 0, 0},
+                          splitInline = {2.91, 1.52, 2.27, 0.445, 1.85, 0.00115, 0.654, 1.96, 0, 0};
     const double products = d->precision == COGCONV_FP32 ? 6 : (d->precision == COGCONV_SPLIT_BF16 ? 3 : 1);
     const double mfma = g.FH * g.FW * c.MB * products * 32 / 2400.0;  // 32 cycles each
+    const double ua = g.OW % 4 ? 1 : 0;
     if (g.upAr == 2)  // half the taps a wave, half the waves' rows a block
-        return up.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma / 2,
-                     (2.0 * c.MB + (g.FH - 1) / 2) * (32 + (g.FW - 1) / 2));
+        return by_filter(up, g).us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma / 2,
+                                   (2.0 * c.MB + (g.FH - 1) / 2) * (32 + (g.FW - 1) / 2), ua);
     if (g.dnR == 2)
-        return down.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
-                       (8.0 * c.MB - 2 + g.FH) * (62 + g.FW));
-    // A workgroup that packs its own filters: one launch, its staging in the chunk.
-    static const CallTime lpInline = {2.96, 0.187, 7.95, 0.540, 2.14, 0.00111, 0.813, 1.62, 0},
-                          splitInline = {2.91, 1.52, 2.27, 0.445, 1.85, 0.00115, 0.654, 1.96, 0};
+        return by_filter(down, g).us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
+                                     (8.0 * c.MB - 2 + g.FH) * (62 + g.FW), ua);
     if (c.ring)
         return (products == 3 ? splitInline : lpInline)
             .us((double)c.tilesR * c.tilesC * c.mTiles * m.B, c.RC / 16, mfma,
                 (4.0 * c.MB + g.FH - 1) * (31 + g.FW) + 32.0 * g.FH * g.FW);
     // In 256-thread units: a workgroup of two output blocks stages its pixels once.
     const int groups = (c.mTiles + c.splits - 1) / c.splits;
-    return fit[d->precision].us((double)c.tilesR * c.tilesC * groups * c.splits * m.B, c.RC / 16, mfma,
-                                (4.0 * c.MB + g.FH - 1) * (31 + g.FW) / c.splits);
+    return (products == 6 ? by_filter(unit, g) : products == 3 ? split : lp)
+        .us((double)c.tilesR * c.tilesC * groups * c.splits * m.B, c.RC / 16, mfma,
+            (4.0 * c.MB + g.FH - 1) * (31 + g.FW) / c.splits, ua);
 }
 
 double igemm_frame_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime unit = {2.26, 1.05, 0.233, 1.90, 2.28, 0.00255, 0.896, 0.974, 0},
-                          down = {3.69, 2.07, 2.63, 1.23, 2.67, 0.00322, 0.729, 5.14, 0};
-    const CallTime& fit = g.dnR == 2 ? down : unit;
+    static const CallTime unit[4] = {{2.49, 1.37, 0.129, 1.19, 2.65, 0.0025, 0.892, 1.19, 0.363, 0.072},
+                                     {2.71, 1.80, 1.54, 1.26, 2.25, 0.00447, 0.923, 3.16, 0.394, 0.132},
+                                     {1.86, 2.15, 0.634, 1.67, 2.32, 0.00181, 0.938, 1.64, 0.124, 0.749},
+                                     {1.84, 0.871, 1.10, 1.43, 2.24, 0.00319, 0.968, 1.78, 0, 0.585}};
+    static const CallTime down[4] = {{3.08, 1.87, 2.39, 1.16, 2.83, 0.00302, 0.770, 3.18, 0.235, 0.408},
+                                     {2.97, 2.89, 2.07, 1.82, 2.48, 0.0027, 0.831, 8.0, 0, 0.528},
+                                     {2.24, 0.684, 0.925, 1.22, 2.62, 0.00249, 0.931, 1.05, 0.0548, 0.396},
+                                     {2.24, 0.684, 0.925, 1.22, 2.62, 0.00249, 0.931, 1.05, 0.0548, 0.396}};
     const double mfma = c.MB * g.FH * g.FW * (c.RC / 8) * 4 * 32 / 2400.0;
-    return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
-                  c.RC / 16.0 * (7 * g.dnR + g.FH) * (31 * g.dnC + g.FW));
+    return by_filter(g.dnR == 2 ? down : unit, g)
+        .us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
+            c.RC / 16.0 * (7 * g.dnR + g.FH) * (31 * g.dnC + g.FW), g.OW % 4 ? c.MB : 0);
 }
 
 // FP32 FilterAdjoint as split-BF16 products (k_fa_rows_lp): a launch floor, the
 // longer of one block's walk and the grid's at full load (in blocks of four waves
 // over 256 CUs), and the partials' writing and summing; and the FP32 MFMA kernel.
 // 520 measured calls (1x1 and 3x3, sides 24 to 256, log error 0.05 and 0.11 rms, each half
-// judged by the other's fit); at 0.8 of the other's estimate it takes 172 of them, 1.46x
-// faster on them and none slower by 3% (first at 0.9: 0.94x), with 0.7 times the MFMA
+// judged by the other's fit); at 0.88 of the other's estimate it takes 258 of them, 1.37x
+// faster on them and one slower by 3% (0.95x; 13 at 0.95), with 0.7 times the MFMA
 // kernel's relative error.
 double fa_rows_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
     const double points = (double)g.OH * g.OW, waves = c.nb * c.kh;
@@ -707,10 +727,13 @@ double fa_igemm_us(const Geom& g, const PlaneMap& m, const FaCfg& c) {
 }
 
 double up2q_us(const Geom& g, const PlaneMap& m, const IgemmCfg& c) {
-    static const CallTime fit = {1.31, 0.683, 0.142, 2.75, 2.05, 0.0029, 0.737, 0.62, 4.61};
+    static const CallTime fit[4] = {{1.80, 1.40, 1.28, 3.10, 1.36, 0.00521, 0.599, 1.0, 5.41, 0},
+                                    {2.01, 1.18, 0.703, 2.84, 2.22, 0.00383, 0.732, 1.0, 4.54, 1.04},
+                                    {1.43, 1.95, 0.804, 3.28, 2.02, 0.00631, 0.765, 1.25, 4.85, 0},
+                                    {1.88, 2.04, 0.0264, 2.67, 2.27, 0.00402, 0.857, 1.0, 5.22, 0}};
     const double mfma = c.MB * g.FH * g.FW / 2.0 * (c.RC / 4) * 4 * 32 / 2400.0;
-    return fit.us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
-                  c.RC / 16.0 * c.tileRows * c.tileCols, g.OW % 4 ? c.MB : 0);  // 16-byte stores need aligned rows
+    return by_filter(fit, g).us((double)c.tilesR * c.tilesC * c.mTiles * m.B, (m.R + c.RC - 1) / c.RC, mfma,
+                                c.RC / 16.0 * c.tileRows * c.tileCols, g.OW % 4 ? c.MB : 0);
 }
 
 SmallCfg choose_small(const Geom& g, const PlaneMap& m, long blocks = 4096) {
@@ -1099,7 +1122,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
         if (fx_first < 0 || fa_rows_us(g, m, best) < fa_rows_us(g, m, fx[fx_first])) fx_first = (int)fx.size();
         fx.push_back(best);
     }
-    if (fx_first >= 0 && fa_ok && fa_rows_us(g, m, fx[fx_first]) > 0.8 * fa_igemm_us(g, m, fa)) fx_first = -1;
+    if (fx_first >= 0 && fa_ok && fa_rows_us(g, m, fx[fx_first]) > 0.88 * fa_igemm_us(g, m, fa)) fx_first = -1;
     const SmallCfg sm = choose_small(g, m);
     const DirectCfg dr = choose_direct(g, 4);
     DirectCfg drt[3];
@@ -1122,7 +1145,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
             rows_first = i;
     }
     if (rows_first >= 0 && igemm_ok &&
-        frame_rows_us(desc, g, m, rows[rows_first]) > 0.9 * igemm_frame_us(g, m, ig))
+        frame_rows_us(desc, g, m, rows[rows_first]) > 0.97 * igemm_frame_us(g, m, ig))
         rows_first = -1;
     PhaseSet up;
     const bool up_ok = choose_igemm_up(desc, g, m, &up);
@@ -1141,7 +1164,7 @@ void enumerate_variants(const cogconv_desc* desc, const Geom& g, const PlaneMap&
     PhaseSet upq = up;
     const bool upq_ok = up_ok && (choose_igemm_up2q(g, m, up, &upq.f, 1, 0, 80 * 1024, true) ||
                                   choose_igemm_up2q(g, m, up, &upq.f));
-    if (rows_first >= 0 && upq_ok && frame_rows_us(desc, g, m, rows[rows_first]) > 0.85 * up2q_us(g, m, upq.f.c))
+    if (rows_first >= 0 && upq_ok && frame_rows_us(desc, g, m, rows[rows_first]) > 0.92 * up2q_us(g, m, upq.f.c))
         rows_first = -1;
     if (fft_first) add_fft(fc);
     else if (rows_first >= 0) add(KK_FRAME_ROWS, nullptr, nullptr, &rows[rows_first], nullptr);

@@ -13,7 +13,6 @@ NONE, UP, DOWN = L.NO_SAMPLING, L.UPSAMPLE_INPUT, L.DOWNSAMPLE_OUTPUT
 @pytest.mark.parametrize("mode,border,sampling,precision,B,N,K,H,W,F,kernel", [
     # FP32 MFMA kernels against the split-BF16 forms
     (BPF, CLAMP, NONE, L.FP32, 2, 16, 24, 146, 116, 9, "igemm_f32 "),       # 41.0, 53.7 split
-    (BPF, FULL, NONE, L.FP32, 19, 7, 10, 68, 108, 7, "igemm_f32 "),         # 47.9, 56.9
     (PF, CYCLIC, DOWN, L.FP32, 16, 23, 25, 134, 162, 3, "igemm_f32 "),      # 32.3, 36.0
     (PF, CYCLIC, UP, L.FP32, 2, 32, 39, 141, 126, 3, "igemm_f32_up2 "),     # 20.6, 25.2
     (PF, ZERO, UP, L.FP32, 3, 7, 33, 48, 64, 9, "igemm_f32_up2 "),          # 16.9, 20.4
@@ -22,6 +21,9 @@ NONE, UP, DOWN = L.NO_SAMPLING, L.UPSAMPLE_INPUT, L.DOWNSAMPLE_OUTPUT
     # the split-BF16 forms where they are faster
     (PF, CLAMP, NONE, L.FP32, 8, 32, 32, 256, 256, 9, "igemm_f32x3 "),      # 341, 726 FP32 MFMA
     (PF, ZERO, UP, L.FP32, 8, 32, 32, 256, 256, 7, "igemm_f32_up2x3 "),     # 265, 484
+    (BPF, FULL, NONE, L.FP32, 19, 7, 10, 68, 108, 7, "rows=2 "),            # 46.2, 47.9 FP32 MFMA, 56.9 one row a wave
+    (PF, ZERO, NONE, L.FP32, 11, 34, 10, 28, 39, 3, "igemm_f32x3 "),        # 13.9, 17.5
+    (PF, ZERO, UP, L.FP32, 5, 12, 49, 49, 51, 3, "igemm_f32_up2x3 "),       # 11.8, 24.8
     # rows a wave of the low-precision forms
     (PF, ZERO, NONE, L.BF16, 3, 25, 9, 180, 222, 5, "rows=2 "),             # 15.4, 18.1 with four (15.9 tiled)
     (BPF, FULL, NONE, L.SPLIT_BF16, 13, 12, 31, 94, 61, 5, "rows=2 "),      # 21.1, 31.5 with four (27.9 tiled)
