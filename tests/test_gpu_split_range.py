@@ -1,7 +1,7 @@
 """The FP32 plans that run as split-BF16 products (igemm_f32x3, igemm_f32_up2x3 and
 fa_igemm_f32x3) on operands outside the split's range: subnormal ones, whose BF16
 terms all vanish, in every sampling the split forms take, and the time a field
-full of non-finite samples takes."""
+full of non-finite samples takes, and their epilogues."""
 import time
 
 import numpy as np
@@ -113,3 +113,46 @@ def test_masked_fields_keep_their_speed(mode, B, N, K, H, W, F, value):
         b.close()
     plan.close()
     assert best[1] <= 8 * best[0]
+
+
+@pytest.mark.parametrize("form,F", [("unit", 5), ("unit", 9), ("up", 7), ("down", 3), ("weight_grad", 3)])
+@pytest.mark.parametrize("inf", (False, True))
+def test_epilogue_equals_its_own_pass(form, F, inf):
+    """Constants and every kind of field operand, on plain outputs and on ones that
+    are computed a second time."""
+    rng = np.random.default_rng(14)
+    mode, border, sampling, step, _ = FORMS[form]
+    xs = (N, H, W)
+    ws = (K, H - F + 1, W - F + 1) if mode == O.FA_BRS else (K * N, F, F)
+    _, cd = desc_pair(mode, border, O.XCORR, sampling, step, 1, xs, ws)
+    x = rng.uniform(-1, 1, xs).astype(np.float32)
+    if inf:
+        x[3, 7, 11] = np.inf
+    bx = L.DeviceBuffer.from_array(x)
+    bw = L.DeviceBuffer.from_array(rng.uniform(-1, 1, ws).astype(np.float32))
+    plans = [L.Plan(cd, v) for v in range(L.variant_count(cd))]
+    split = [p for p in plans if p.description.split()[0].endswith("x3")]
+    assert split
+    planes, rows, cols = split[0].out_shape
+    n = planes * rows * cols
+    fields = [(2, rows, cols, planes, 1), (2, rows, cols, 1, 0), (0, 1, 1, planes, 1), (0, 1, 1, 1, 0)]
+    operands = [L.DeviceBuffer.from_array(rng.uniform(0.5, 2, (t[3], t[1], t[2])).astype(np.float32)) for t in fields]
+    epi = L.make_epilogue([(L.EPI_MUL_FIELD, 0, 0), (L.EPI_SUB_FIELD, 0, 1), (L.EPI_ADD_FIELD, 0, 2),
+                           (L.EPI_DIV_FIELD, 0, 3), (L.EPI_TANH, 0, 0), (L.EPI_MAX_CONST, -0.25, 0)],
+                          [L.field_type(*t) for t in fields])
+    out, want, got = (L.DeviceBuffer(4 * n) for _ in range(3))
+    for plan in split:
+        print("CASE split epilogue", form, inf, plan.description, flush=True)
+        wk = L.DeviceBuffer(plan.workspace_bytes)
+        plan.launch(bx, bw, out, wk)
+        L.elementwise(out, want, (2, rows, cols, planes, 1), epi, operands)
+        plan.set_epilogue(epi)
+        plan.launch_epilogue(bx, bw, got, wk, operands)
+        L.synchronize()
+        a, b = got.download(plan.out_shape), want.download(plan.out_shape)
+        assert np.array_equal(a, b, equal_nan=True), plan.description
+        wk.close()
+    for p in plans:
+        p.close()
+    for b in operands + [bx, bw, out, want, got]:
+        b.close()
