@@ -387,4 +387,5 @@ struct cogconv_plan_s {
     int variant;  // index into the plan's candidate list (autotuning)
     cogconv::Epi epi;       // elementwise epilogue (epi.n == 0: none); src[] set per launch
     int epi_operands;       // field operands the epilogue reads
+    cogconv_plan_s* plain;  // what launches without a workspace run (plan_for), made at the first
 };

@@ -1405,7 +1405,10 @@ extern "C" int cogconv_plan_variant(cogconv_plan plan, int32_t* variant) {
 
 extern "C" int cogconv_plan_destroy(cogconv_plan plan) {
     clear_error();
-    if (plan) fft_release(plan->fft_state);
+    if (plan) {
+        fft_release(plan->fft_state);
+        if (plan->plain) cogconv_plan_destroy(plan->plain);
+    }
     delete plan;
     return COGCONV_OK;
 }
@@ -1640,6 +1643,25 @@ int launch_all(cogconv_plan plan, const float* in0, const float* in1, float* out
     return check_hip(e, "convolution launch");
 }
 
+// The plan that a launch with `workspace` runs; null where it needs one.  FP32 frame
+// modes had kernels without a workspace before the split-BF16 form took most of them:
+// without one (a program that never asked, or one plan on several streams) they run the
+// plan that leaves the split form out, made at the first such launch.
+cogconv_plan plan_for(cogconv_plan plan, const void* workspace) {
+    if (workspace || !plan->workspace) return plan;
+    if (plan->kind != KK_FRAME_ROWS || plan->desc.precision != COGCONV_FP32) return nullptr;
+    cogconv_plan p = __atomic_load_n(&plan->plain, __ATOMIC_ACQUIRE);
+    if (!p) {
+        cogconv_plan made = nullptr;
+        if (make_plan(&plan->desc, -1, &made, true)) return nullptr;
+        if (__atomic_compare_exchange_n(&plan->plain, &p, made, false, __ATOMIC_ACQ_REL, __ATOMIC_ACQUIRE))
+            p = made;
+        else
+            cogconv_plan_destroy(made);
+    }
+    return p->workspace ? nullptr : p;
+}
+
 // The plan's epilogue with its field operands bound to `operands`.
 int bind_epilogue(const cogconv_plan_s* plan, const float* const* operands, Epi* ep) {
     *ep = plan->epi;
@@ -1652,11 +1674,11 @@ extern "C" int cogconv_launch(cogconv_plan plan, const float* in0, const float* 
                               cogconv_stream stream) {
     clear_error();
     if (!plan || !in0 || !in1 || !out) return fail(COGCONV_ERR_INVALID_ARG, "null plan or buffer");
-    if (plan->workspace && !workspace)
-        return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);
+    const cogconv_plan run = plan_for(plan, workspace);
+    if (!run) return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);
     if (plan->epi_operands)
         return fail(COGCONV_ERR_INVALID_ARG, "the plan's epilogue reads field operands: use cogconv_launch_epilogue");
-    return launch_all(plan, in0, in1, out, workspace, reinterpret_cast<hipStream_t>(stream), plan->epi);
+    return launch_all(run, in0, in1, out, workspace, reinterpret_cast<hipStream_t>(stream), plan->epi);
 }
 
 bool cogconv::plan_table_capable(const cogconv_plan_s* plan) {
@@ -1695,7 +1717,8 @@ extern "C" int cogconv_launch_table(cogconv_plan plan, const cogconv_image_io* h
         return fail(COGCONV_ERR_UNSUPPORTED, "table launches are offered for the MFMA frame plans (no up-sampling)");
     if (packed && !packs_operand(plan)) return fail(COGCONV_ERR_INVALID_ARG, "plan does not pack operand 2");
     if (!packed && !in1) return fail(COGCONV_ERR_INVALID_ARG, "null operand 2");
-    if ((plan->workspace || packed) && !workspace)
+    const cogconv_plan run = packed && !workspace ? nullptr : plan_for(plan, workspace);
+    if (!run || !plan_table_capable(run))
         return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);
     if (plan->epi_operands)
         return fail(COGCONV_ERR_INVALID_ARG, "table launches take no epilogue field operands");
@@ -1710,6 +1733,9 @@ extern "C" int cogconv_launch_table(cogconv_plan plan, const cogconv_image_io* h
                                           hipMemcpyHostToDevice, s),
                            "table copy"))
         return st;
+    if (run != plan)
+        return check_hip(launch_igemm_f32(run->g, run->m, run->icfg, nullptr, in1, nullptr, s, plan->epi, device_table),
+                         "table launch");
     return launch_table(plan, device_table, x16, in1, workspace, packed != 0, s);
 }
 
@@ -1717,11 +1743,11 @@ extern "C" int cogconv_launch_epilogue(cogconv_plan plan, const float* in0, cons
                                        void* workspace, const float* const* operands, cogconv_stream stream) {
     clear_error();
     if (!plan || !in0 || !in1 || !out) return fail(COGCONV_ERR_INVALID_ARG, "null plan or buffer");
-    if (plan->workspace && !workspace)
-        return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);
+    const cogconv_plan run = plan_for(plan, workspace);
+    if (!run) return fail(COGCONV_ERR_INVALID_ARG, "plan needs %zu bytes of workspace", plan->workspace);
     Epi ep;
     if (int st = bind_epilogue(plan, operands, &ep)) return st;
-    return launch_all(plan, in0, in1, out, workspace, reinterpret_cast<hipStream_t>(stream), ep);
+    return launch_all(run, in0, in1, out, workspace, reinterpret_cast<hipStream_t>(stream), ep);
 }
 
 namespace {

@@ -82,9 +82,9 @@ enum {
     COGCONV_CONVOLUTION = 1
 };
 
-/* Arithmetic of the plan.  FP32 is the plain form (FP32 products, FP32
- * accumulation).  The others are the precision variants of the
- * contraction modes (ProjectFrame / BackProjectFrame / FilterAdjoint with
+/* Arithmetic of the plan.  FP32 is the plain form: operands and sums in FP32
+ * (products too under COGCONV_ALGO_IMPLICIT_GEMM, see there).  The others are the
+ * precision variants of the contraction modes (ProjectFrame / BackProjectFrame / FilterAdjoint with
  * block reduction): MFMA implicit GEMM with FP32 accumulation. */
 enum {
     COGCONV_FP32 = 0,
@@ -215,7 +215,11 @@ int cogconv_output_type(const cogconv_desc* desc, cogconv_field_type* out);
 int cogconv_plan_create(const cogconv_desc* desc, cogconv_plan* plan);
 int cogconv_plan_destroy(cogconv_plan plan);
 int cogconv_plan_output_type(cogconv_plan plan, cogconv_field_type* out);
-/* Device scratch a launch needs (0 for most plans); the caller allocates it. */
+/* Device scratch a launch needs; the caller allocates it.  Every launch writes it: the
+ * BF16 / FP16 / split-BF16 frame plans and the FP32 ones that run as split-BF16
+ * products ("x3" in the description) pack operand 2 into it, plans with a split
+ * reduction keep partial sums there.  So launches that overlap (one plan on several
+ * streams) need a workspace each.  0 for the other plans. */
 int cogconv_plan_workspace_bytes(cogconv_plan plan, size_t* bytes);
 /* Algorithmic FLOPs of one launch: 2 * (multiply-adds with a non-zero tap). */
 int cogconv_plan_flops(cogconv_plan plan, double* flops);
@@ -225,7 +229,8 @@ int cogconv_plan_bytes(cogconv_plan plan, double* bytes);
 int cogconv_plan_describe(cogconv_plan plan, char* buf, size_t len);
 /* Enqueue one ConvolveOp: out = op(in0, in1).  in0/in1/out are planar float32
  * device buffers of the plan's FieldTypes; `workspace` holds
- * cogconv_plan_workspace_bytes bytes (may be NULL when that is 0). */
+ * cogconv_plan_workspace_bytes bytes (may be NULL when that is 0, and for FP32 frame
+ * plans, which then run a kernel with FP32 products and no workspace). */
 int cogconv_launch(cogconv_plan plan, const float* in0, const float* in1, float* out, void* workspace,
                    cogconv_stream stream);
 
@@ -313,9 +318,9 @@ int cogconv_separable(const float* in, const cogconv_field_type* type, const flo
  * split-BF16 frame plans convert operand 2 into a packed low-precision form in
  * the workspace on every cogconv_launch.  cogconv_plan_pack_operand does that
  * conversion once (*packed = 1; 0 for plans that do not pack, which leave the
- * workspace alone), and cogconv_launch_packed then runs the convolution on the
- * packed form kept in `workspace` (COGCONV_ERR_INVALID_ARG for plans that do
- * not pack).  The workspace must not be written between the two. */
+ * workspace alone, and for the FP32 ones, which read operand 2 itself as well), and
+ * cogconv_launch_packed then runs the convolution on the packed form kept in
+ * `workspace` (COGCONV_ERR_INVALID_ARG for plans that do not pack).  The workspace must not be written between the two. */
 int cogconv_plan_pack_operand(cogconv_plan plan, const float* in1, void* workspace, cogconv_stream stream,
                               int32_t* packed);
 int cogconv_launch_packed(cogconv_plan plan, const float* in0, float* out, void* workspace, cogconv_stream stream);
