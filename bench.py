@@ -225,7 +225,7 @@ def timed_steps(L, ops, stream, steps, warmup):
 def roofline(plan, ms, peak_tflops, name, reps, traffic_file):
     """Roofline object for one launch of `plan` taking `ms`: compute-bound when
     its algorithmic FLOP/byte is above the ridge of `peak_tflops` and HBM."""
-    if "x3 " in plan.description:
+    if plan.description.split()[0].endswith("x3"):
         peak_tflops = round(PEAK_BF16_TFLOPS / 6, 1)  # FP32 as six BF16 products
     ai = plan.flops / plan.bytes
     ridge = peak_tflops * 1e12 / (PEAK_HBM_GBS * 1e9)
@@ -242,7 +242,7 @@ def roofline(plan, ms, peak_tflops, name, reps, traffic_file):
     if os.path.exists(path):
         with open(path) as fh:
             t = json.load(fh).get(name)
-        if t:
+        if t and t.get("plan", plan.description) == plan.description:  # counted for this kernel
             roof["traffic"] = t["hbm_bytes_per_launch"]
             roof["traffic_source"] = ("profiles/%s (rocprofv3 FETCH_SIZE + WRITE_SIZE per dispatch, "
                                       "copy-calibrated)" % traffic_file)
