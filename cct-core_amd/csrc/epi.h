@@ -76,8 +76,8 @@ __device__ __forceinline__ float epi(const Epi& e, float v, int plane, int point
 // once per op and element, and the N operand loads of a field op are in flight
 // together.  Element by element these dependent loads were most of a small
 // launch: bias and rectifier on 16 images 64x64x16 -> 32 planes, 3x3, took
-// 22.7 us, and 13.8 us this way (12.4 us without an epilogue).  Every (plane, point) must be a valid output element, also where
-// the caller does not store the result.
+// 22.7 us, and 13.8 us this way (12.4 us without an epilogue).  Every (plane, point)
+// must be a valid output element, also where the caller does not store the result.
 template <int N>
 __device__ __forceinline__ void epi_eval_n(const Epi& e, float (&v)[N], const int (&plane)[N], const int (&point)[N]) {
 #pragma clang fp contract(off)

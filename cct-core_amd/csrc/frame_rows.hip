@@ -7,12 +7,15 @@
 //
 //   BF16, FP16    T = 1: operands rounded once, one product.
 //   split-BF16    T = 2: x = x0 + x1, the products x0 w0 + x0 w1 + x1 w0.
-//   FP32          T = 3, exact: x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),
+//   FP32          T = 3: x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),
 //     x2 = x - x0 - x1.  Round to nearest leaves remainders of 16 and 8 bits, so the
 //     terms hold all 24 bits of x.  Of the nine products of two operands the six
 //     with term indexes summing to at most 2 are computed, each exact on the
-//     MFMA with FP32 accumulation; the other three are below 2^-25 of the product,
-//     under the rounding of one FP32 multiply.  Six BF16 MFMAs do the work of one
+//     MFMA with FP32 accumulation; the other three come to 2^-24 of the product
+//     at most.  So a sum of one product may be off by two half-ulps where an FP32 multiply
+//     is off by one (1.82 measured; 3.8% of such products are not correctly rounded),
+//     while in longer sums fewer roundings halve the error (9x9 below); the
+//     implicit-GEMM hint keeps to FP32 products.  Six BF16 MFMAs do the work of one
 //     FP32 MFMA in 6/16 of its cycles.
 //
 // gfx950 mapping: v_mfma_f32_32x32x16, A = filters (32 output planes x 16 input
@@ -26,7 +29,8 @@
 // registers and walks down the tile: the pixels of tile row y, read from LDS once
 // per tap column, meet tap row i for every output row y - i the wave owns.  So an
 // LDS read of a pixel fragment feeds up to F tap rows and a filter fragment RW
-// rows: RW = 4, 9x9: 63 16-byte reads for 216 MFMAs of 32 cycles a tap column.
+// rows: FP32 9x9, RW = 8: 48 16-byte reads of pixels and 27 filter fragments for 432
+// MFMAs of 32 cycles a tap column.
 // Filter fragments come straight from the packed bank in L2 (1 KiB contiguous
 // each) and pass through a ring of registers: each is loaded into the registers of
 // the fragment it replaces right after that one's last use, a tap column ahead.
@@ -35,11 +39,13 @@
 // instruction writes whole 32-pixel rows of two planes at any alignment.
 //
 // Measured against the kernels it replaced (us a call): FP32 9x9, 32 -> 32 planes,
-// 8 images 256x256: 730 -> 331; split-BF16 3x3, 64 -> 64 planes, 32 images 128x128:
-// 170 -> 122; FP32 2x up-sampled 7x7, 32 -> 32 planes, 8 images 256x256: 485 -> 262 (its
-// bound now: 126 of matrix cores at their peak, 55 of output stores); BF16 and FP16 3x3 to 9x9 over 400 random calls (3 to 64 planes, 24 to
-// 256 a side): 1.5x.  What bounds it: the matrix cores at FP32 (70% of their peak
-// at 9x9); for one term the latency of staging and of the filter stream.
+// 8 images 256x256: 730 -> 327; split-BF16 3x3, 64 -> 64 planes, 32 images 128x128:
+// 170 -> 122; FP32 2x up-sampled 7x7, 32 -> 32 planes, 8 images 256x256: 485 -> 257 (126 of
+// matrix cores at their peak, 55 of output stores); BF16 and FP16 3x3 to 9x9 over 1350
+// random calls (3 to 64 planes, 24 to 256 a side): 1.5x.  What bounds it: the matrix cores
+// in FP32 (busy 75% of the cycles at 9x9, 69% at 7x7, 62% up-sampled, at the clock that
+// the power limit leaves: 327 us are 64% of the nominal rate); for one term the
+// latency of staging and of the filter stream (35% busy at 7x7, 49% at 9x9).
 #include <algorithm>
 #include <type_traits>
 

@@ -313,11 +313,11 @@ hipError_t launch_up2q_lp(int precision, const Geom& g, const PlaneMap& m, const
 hipError_t launch_igemm_lp(int precision, const Geom& g, const PlaneMap& m, const IgemmCfg& c, const float* x,
                            const float* w, float* out, void* ws, hipStream_t s, int stage = LP_PACK_AND_RUN,
                            const Epi& e = kNoEpi, const cogconv_image_io* tab = nullptr, bool x16 = false);
-// FP32 frame modes as split-BF16 products, and the split-BF16 ones (frame_rows.hip):
-// c.variant is the sampling, c.MB holds the output rows of a wave, c.splits the
-// 32-plane output blocks of a workgroup, c.RC the planes padded to whole 16-plane
-// chunks.  `stage` as in launch_igemm_lp
-// (the FP32 form packs on every launch).
+// The row-walking frame kernel (frame_rows.hip): FP32 frame modes as split-BF16 products,
+// and the BF16, FP16 and split-BF16 ones at unit steps.  c.variant is the sampling, c.MB
+// the output rows of a wave, c.splits the 32-plane output blocks of a workgroup, c.RC
+// the planes padded to whole 16-plane chunks, c.ring whether plain launches pack in the
+// kernel.  `stage` as in launch_igemm_lp (the FP32 form packs on every launch).
 enum FrameRowsSampling { FR_UNIT = 0, FR_UP0 = 1, FR_UP1 = 2, FR_DOWN = 3 };
 size_t frame_rows_lds_bytes(int F, int RW, int MW, int sampling, int precision);  // 0: not built
 bool frame_rows_inline(int F, int RW, int MW, int sampling, int precision);  // plain launches may pack in the kernel (c.ring)

@@ -569,9 +569,10 @@ bool choose_igemm_lp(const cogconv_desc* d, const Geom& g, const PlaneMap& m, Ig
     return false;
 }
 
-// FP32 and split-BF16 frame block-reduce modes as split-BF16 products
-// (k_frame_rows): square filters, unit steps, 2x up-sampled input or every
-// second output; `rw` output rows a wave.
+// Frame block-reduce modes on the row-walking kernel (k_frame_rows): square filters,
+// unit steps and, in FP32 (as split-BF16 products), 2x up-sampled input or every second
+// output; `rw` output rows a wave, `mw` output blocks a workgroup, `own`: filters packed
+// in the kernel.
 bool choose_frame_rows(const cogconv_desc* d, const Geom& g, const PlaneMap& m, IgemmCfg* out, int rw, int mw = 1,
                        bool own = false) {
     if (d->mode != COGCONV_PROJECT_FRAME_BLOCK_REDUCE_SUM && d->mode != COGCONV_BACK_PROJECT_FRAME_BLOCK_REDUCE_SUM)
