@@ -97,8 +97,10 @@ enum {
  * FP32 under AUTO may take a form that computes each product as six products of
  * BF16 terms (see cogconv_plan_describe: "x3"): on sums its error is below
  * the FP32 kernels', but a single product may be off by two half-ulps where FP32
- * multiplies round to one.  IMPLICIT_GEMM keeps to FP32 products for FP32 (and to
- * the tiled kernel for BF16 / FP16 / split-BF16). */
+ * multiplies round to one, and as the choice depends on the batch an image's result
+ * may differ in its last bits between batch sizes.  IMPLICIT_GEMM keeps to FP32
+ * products for FP32 (the same bits at every batch size) and to the tiled kernel for
+ * BF16 / FP16 / split-BF16. */
 enum {
     COGCONV_ALGO_AUTO = 0,
     COGCONV_ALGO_DIRECT = 1,        /* LDS-tiled direct kernel, any op         */

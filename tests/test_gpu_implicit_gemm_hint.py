@@ -108,3 +108,21 @@ def test_fp32_products_round_once(sampling, step, border):
             print("CASE hinted FP32", name, flush=True)
             assert not name.split()[0].endswith("x3")
             assert np.array_equal(run_gpu(cd, x, w, variant=v), want), name
+
+
+@pytest.mark.parametrize("sampling,step,border,F", [(O.NONE, 1, O.CLAMP, 9), (O.NONE, 1, O.ZERO, 3), (O.UP, 2, O.ZERO, 5),
+                                                    (O.DOWN, 2, O.CYCLIC, 5)])
+def test_fp32_bits_do_not_depend_on_the_batch(sampling, step, border, F):
+    """One image's result under the hint is the same at every batch size."""
+    rng = np.random.default_rng(22)
+    N, K, H, W = 20, 36, 50, 64
+    x = rng.uniform(-1, 1, (16 * N, H, W)).astype(np.float32)
+    w = rng.uniform(-1, 1, (K * N, F, F)).astype(np.float32)
+    first = None
+    for B in (1, 3, 16):
+        a = np.ascontiguousarray(x[:B * N])
+        _, cd = desc_pair(O.PF_BRS, border, O.XCORR, sampling, step, B, a.shape, w.shape, algo=L.ALGO_IMPLICIT_GEMM)
+        print("CASE batch", B, sampling, F, flush=True)
+        got = run_gpu(cd, a, w)[:K]
+        first = got if first is None else first
+        assert np.array_equal(got, first)
